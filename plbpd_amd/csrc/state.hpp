@@ -90,7 +90,7 @@ struct plb_state {
     // outer layer only; ntmp off that layer is n(c + c_k, k) until restored
     bool lit_ntmp_folded;
     bool moments_valid;
-    void* scratch;  // reductions, face staging
+    void* scratch;  // reductions
     size_t scratch_bytes;
     hipStream_t stream;
     // graph of a fixed number of fused steps
@@ -148,7 +148,7 @@ int lit_collide_push(plb_state* s, double tau, const double F[3]);
 int lit_moments_collide_push(plb_state* s, double tau, const double F[3], const plb_boundary* bc_vel,
                              const plb_boundary* bc_rho);
 int lit_noslip(plb_state* s, const plb_boundary* bc);
-// The same pass staged in the library's static device buffer: no allocation.
+// The same pass for faces within the documented size limit of the entry point.
 int lit_noslip_noalloc(plb_state* s, const plb_boundary* bc);
 int lit_periodic(plb_state* s, const plb_boundary* bc);
 int lit_moments(plb_state* s);
