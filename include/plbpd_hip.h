@@ -202,13 +202,15 @@ int plb_apply_noslip(plb_state* s, const plb_boundary* bc);
  * PLB_ERR_LOGIC.  The pass works in the state's own arrays, so calls on
  * different states do not meet. */
 int plb_apply_noslip_noalloc(plb_state* s, const plb_boundary* bc);
-/* Boundary::apply_periodicity (Boundary.cpp:91-99, 223-281). */
+/* Boundary::apply_periodicity (Boundary.cpp:91-99, 223-281).  Deferred in
+ * literal mode like the moments after it (see plb_calc_moments). */
 int plb_apply_periodicity(plb_state* s, const plb_boundary* bc);
 /* CalcMoments::operator() (CalcMoments.hpp:46-73).  Literal mode with
- * PLB_TUNE_LITERAL_FUSE on: the moments, and the resets that directly follow
- * them, run with the next call on the state -- folded into the collide+push
- * kernel when that sequence is collide then plb_stream(s, "push"), else
- * before the call does anything -- so every observable value is unchanged. */
+ * PLB_TUNE_LITERAL_FUSE on: the periodic copies, the moments directly after
+ * them, and the resets that directly follow the moments, run with the next
+ * call on the state -- folded into the collide+push kernel when the sequence
+ * goes on with collide and plb_stream(s, "push"), else before the call does
+ * anything -- so every observable value is unchanged. */
 int plb_calc_moments(plb_state* s);
 /* Boundary::reset / reset_velocity / reset_density (Boundary.cpp:58-89).
  * Deferred in literal mode directly after plb_calc_moments, as described
@@ -235,10 +237,11 @@ int plb_synchronize(plb_state* s);
  * Streaming.cpp:12, Boundary.cpp:12-16, CalcMoments.cpp:5), measured with HIP
  * events on the state's stream.  ms_out: PLB_NSTAGES accumulated values.  A
  * literal collision run together with its push is counted under
- * PLB_STAGE_COLLIDE; PLB_STAGE_STREAM counts the pushes run alone.  Moments
- * and resets folded into the next step's kernel (inside a literal plb_step,
- * or deferred as plb_calc_moments describes) are counted under
- * PLB_STAGE_COLLIDE too. */
+ * PLB_STAGE_COLLIDE; PLB_STAGE_STREAM counts the pushes run alone.  Periodic
+ * copies, moments and resets folded into the next step's kernel (inside a
+ * literal plb_step, or deferred as plb_calc_moments describes) are counted
+ * under PLB_STAGE_COLLIDE too, resets run with their moments under
+ * PLB_STAGE_MOMENTS. */
 int plb_enable_timers(plb_state* s, int on);
 int plb_stage_times(plb_state* s, double* ms_out);
 
@@ -306,9 +309,9 @@ int plb_bench_pattern(int device, int q, int x, int y, int z, int sbytes, int ve
                               /* themselves for buffers over 4 GiB); default 0         */
 #define PLB_TUNE_LITERAL_FUSE 8 /* literal mode: 1 (default) runs a collision and the */
                                 /* push that follows it as one kernel (same values in */
-                                /* n and ntmp, one pass fewer over n), and computes   */
-                                /* each step's moments and resets in the next step's */
-                                /* kernel (same rho and u), inside plb_step and for   */
+                                /* n and ntmp, one pass fewer over n), and does each  */
+                                /* step's periodic copies, moments and resets in the */
+                                /* next step's kernel (same rho and u), inside plb_step and for   */
                                 /* the staged calls alike; 0 runs one kernel per      */
                                 /* reference call                                      */
 #define PLB_TUNE_TWO_STEP 9     /* fused pull step: 1 advances two steps per launch   */

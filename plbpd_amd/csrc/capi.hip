@@ -2,7 +2,6 @@
 // reference operator call, fused stepping, HIP-graph replay, timers.
 #include <cmath>
 #include <cstring>
-#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -109,35 +108,39 @@ int timed(plb_state* s, int stage, Fn&& fn) {
 
 // Literal calls deferred in s->lit_queue run, in order, before any other call
 // observes or changes the state; plb_stream("push") instead folds them into
-// its kernel.
+// its kernel.  Moments and the resets after them are one kernel (counted
+// under the moments' stage).
 int lit_flush(plb_state* s) {
     std::vector<LitOp> q;
     q.swap(s->lit_queue);
-    for (const LitOp& op : q) {
+    for (size_t i = 0; i < q.size(); ++i) {
         int rc;
-        switch (op.kind) {
-            case kLitMoments: rc = timed(s, PLB_STAGE_MOMENTS, [&] { return lit_moments(s); }); break;
-            case kLitResetVelocity:
-                rc = timed(s, PLB_STAGE_RESET_VELOCITY, [&] { return lit_reset_velocity(s, &op.bc); });
+        switch (q[i].kind) {
+            case kLitPeriodic:
+                rc = timed(s, PLB_STAGE_PERIODIC, [&] { return lit_periodic(s, &q[i].bc); });
                 break;
-            case kLitResetDensity:
-                rc = timed(s, PLB_STAGE_RESET_DENSITY, [&] { return lit_reset_density(s, &op.bc); });
+            case kLitMoments: {
+                const plb_boundary *bv = nullptr, *br = nullptr;
+                if (i + 1 < q.size() && q[i + 1].kind == kLitResetVelocity) bv = &q[++i].bc;
+                if (i + 1 < q.size() && q[i + 1].kind == kLitResetDensity) br = &q[++i].bc;
+                rc = timed(s, PLB_STAGE_MOMENTS, [&] { return lit_moments(s, bv, br); });
                 break;
-            default:
-                rc = timed(s, PLB_STAGE_COLLIDE, [&] { return lit_collide(s, op.tau, op.force); });
+            }
+            case kLitCollide:
+                rc = timed(s, PLB_STAGE_COLLIDE, [&] { return lit_collide(s, q[i].tau, q[i].force); });
                 break;
+            default: rc = fail(PLB_ERR_LOGIC, "reset deferred without its moments"); break;
         }
         if (rc) return rc;
     }
     return PLB_OK;
 }
 
-bool lit_queue_is(const plb_state* s, std::initializer_list<LitOpKind> kinds) {
-    if (s->lit_queue.size() != kinds.size()) return false;
-    size_t i = 0;
-    for (LitOpKind k : kinds)
-        if (s->lit_queue[i++].kind != k) return false;
-    return true;
+// Whether the last deferred literal call is of this kind (each kind is only
+// ever deferred directly after its predecessor, so the last one tells what the
+// queue holds).
+bool lit_last_is(const plb_state* s, LitOpKind kind) {
+    return !s->lit_queue.empty() && s->lit_queue.back().kind == kind;
 }
 
 LitOp lit_op(LitOpKind kind, const plb_boundary* bc = nullptr, double tau = 0.0, const double* force = nullptr) {
@@ -471,8 +474,7 @@ int plb_collide_srt(plb_state* s, double tau, const double force[3]) {
     if (s->mode == PLB_MODE_LITERAL) {
         // a collision waits for the push after nothing or after the moments
         // and resets of the step before
-        if (!s->tune_lit_fuse ||
-            !(s->lit_queue.empty() || lit_queue_is(s, {kLitMoments, kLitResetVelocity, kLitResetDensity})))
+        if (!s->tune_lit_fuse || !(s->lit_queue.empty() || lit_last_is(s, kLitResetDensity)))
             if ((rc = lit_flush(s))) return rc;
         if (!force) return fail(PLB_ERR_INVALID_ARGUMENT, "null force");
         if (!s->tune_lit_fuse)
@@ -498,18 +500,18 @@ int plb_stream(plb_state* s, const char* stream_type) {
     const std::string t = stream_type ? stream_type : "";
     // a queue left from before the fusion knob was turned off runs call by call
     const bool fold = s->tune_lit_fuse && t == "push";
-    if (fold && lit_queue_is(s, {kLitMoments, kLitResetVelocity, kLitResetDensity, kLitCollide})) {
+    if (fold && lit_last_is(s, kLitCollide)) {
         const std::vector<LitOp> q = std::move(s->lit_queue);
         s->lit_queue.clear();
-        return timed(s, PLB_STAGE_COLLIDE,
-                     [&] {
-                         return lit_moments_collide_push(s, q[3].tau, q[3].force, &q[1].bc, &q[2].bc);
-                     });
-    }
-    if (fold && lit_queue_is(s, {kLitCollide})) {
-        const LitOp c = s->lit_queue[0];
-        s->lit_queue.clear();
-        return timed(s, PLB_STAGE_COLLIDE, [&] { return lit_collide_push(s, c.tau, c.force); });
+        const LitOp& c = q.back();
+        if (q.size() == 1)
+            return timed(s, PLB_STAGE_COLLIDE, [&] { return lit_collide_push(s, c.tau, c.force); });
+        // (periodicity,) moments, reset velocity, reset density, collide
+        const plb_boundary* per = q[0].kind == kLitPeriodic ? &q[0].bc : nullptr;
+        const LitOp* r = &c - 2;
+        return timed(s, PLB_STAGE_COLLIDE, [&] {
+            return lit_moments_collide_push(s, c.tau, c.force, per, &r[0].bc, &r[1].bc, nullptr);
+        });
     }
     // every other request finds the deferred calls done, as the reference's does
     rc = lit_flush(s);
@@ -575,16 +577,22 @@ int plb_apply_periodicity(plb_state* s, const plb_boundary* bc) {
     int rc = s && s->mode == PLB_MODE_LITERAL ? enter(s) : enter_keep(s);
     if (rc) return rc;
     if (!bc) return fail(PLB_ERR_INVALID_ARGUMENT, "null boundary");
-    if (s->mode == PLB_MODE_LITERAL) return timed(s, PLB_STAGE_PERIODIC, [&] { return lit_periodic(s, bc); });
+    if (s->mode == PLB_MODE_LITERAL) {
+        if (!s->tune_lit_fuse) return timed(s, PLB_STAGE_PERIODIC, [&] { return lit_periodic(s, bc); });
+        s->lit_queue.push_back(lit_op(kLitPeriodic, bc));  // enter() left the queue empty
+        return PLB_OK;
+    }
     return ensure_fused_bc(s, bc, &s->mask_host);
 }
 
 int plb_calc_moments(plb_state* s) {
-    int rc = s && s->mode == PLB_MODE_LITERAL ? enter(s) : enter_keep(s);
+    int rc = enter_keep(s);
     if (rc) return rc;
     if (s->mode == PLB_MODE_LITERAL) {
-        if (!s->tune_lit_fuse) return timed(s, PLB_STAGE_MOMENTS, [&] { return lit_moments(s); });
-        s->lit_queue.push_back(lit_op(kLitMoments));  // enter() left the queue empty
+        if (!s->tune_lit_fuse || !lit_last_is(s, kLitPeriodic))
+            if ((rc = lit_flush(s))) return rc;
+        if (!s->tune_lit_fuse) return timed(s, PLB_STAGE_MOMENTS, [&] { return lit_moments(s, nullptr, nullptr); });
+        s->lit_queue.push_back(lit_op(kLitMoments));
         return PLB_OK;
     }
     s->moments_valid = false;  // computed on demand from the populations
@@ -594,7 +602,7 @@ int plb_calc_moments(plb_state* s) {
 int plb_reset_velocity(plb_state* s, const plb_boundary* bc) {
     int rc = enter_keep(s);
     if (rc) return rc;
-    if (s->tune_lit_fuse && bc && lit_queue_is(s, {kLitMoments})) {
+    if (s->tune_lit_fuse && bc && lit_last_is(s, kLitMoments)) {
         s->lit_queue.push_back(lit_op(kLitResetVelocity, bc));
         return PLB_OK;
     }
@@ -608,7 +616,7 @@ int plb_reset_velocity(plb_state* s, const plb_boundary* bc) {
 int plb_reset_density(plb_state* s, const plb_boundary* bc) {
     int rc = enter_keep(s);
     if (rc) return rc;
-    if (s->tune_lit_fuse && bc && lit_queue_is(s, {kLitMoments, kLitResetVelocity})) {
+    if (s->tune_lit_fuse && bc && lit_last_is(s, kLitResetVelocity)) {
         s->lit_queue.push_back(lit_op(kLitResetDensity, bc));
         return PLB_OK;
     }
@@ -656,14 +664,15 @@ int plb_step(plb_state* s, int nsteps) {
     for (int i = 0; i < nsteps; ++i) {
         if (s->mode == PLB_MODE_LITERAL) {
             // PLBPD::march_in_time loop body (PLBPD.cpp:24-29).  With the
-            // kernels folded, the moments and resets of every step but the
-            // last are computed by the next step's collision kernel, which
-            // stores rho and u as those stages would before it collides.
+            // kernels folded, the periodic copies, moments and resets of
+            // every step but the last are done by the next step's collision
+            // kernel, which stores of rho only what the next no-slip pass
+            // reads (the last step stores every rho and u).
             const plb_boundary* bc = &s->bc;
             const bool fold = s->tune_lit_fuse != 0;
             if (fold && i > 0) {
                 if ((rc = timed(s, PLB_STAGE_COLLIDE,
-                                [&] { return lit_moments_collide_push(s, s->tau, F, bc, bc); })))
+                                [&] { return lit_moments_collide_push(s, s->tau, F, bc, bc, bc, bc); })))
                     return rc;
             } else if (fold) {
                 if ((rc = timed(s, PLB_STAGE_COLLIDE, [&] { return lit_collide_push(s, s->tau, F); })))
@@ -673,9 +682,13 @@ int plb_step(plb_state* s, int nsteps) {
                 if ((rc = timed(s, PLB_STAGE_STREAM, [&] { return lit_push(s); }))) return rc;
             }
             if ((rc = timed(s, PLB_STAGE_NOSLIP, [&] { return lit_noslip(s, bc); }))) return rc;
-            if ((rc = timed(s, PLB_STAGE_PERIODIC, [&] { return lit_periodic(s, bc); }))) return rc;
             if (fold && i + 1 < nsteps) continue;
-            if ((rc = timed(s, PLB_STAGE_MOMENTS, [&] { return lit_moments(s); }))) return rc;
+            if ((rc = timed(s, PLB_STAGE_PERIODIC, [&] { return lit_periodic(s, bc); }))) return rc;
+            if (fold) {
+                if ((rc = timed(s, PLB_STAGE_MOMENTS, [&] { return lit_moments(s, bc, bc); }))) return rc;
+                continue;
+            }
+            if ((rc = timed(s, PLB_STAGE_MOMENTS, [&] { return lit_moments(s, nullptr, nullptr); }))) return rc;
             if ((rc = timed(s, PLB_STAGE_RESET_VELOCITY, [&] { return lit_reset_velocity(s, bc); }))) return rc;
             if ((rc = timed(s, PLB_STAGE_RESET_DENSITY, [&] { return lit_reset_density(s, bc); }))) return rc;
         } else if (i + 1 < nsteps && s->post_collision && fused_two_eligible(s)) {

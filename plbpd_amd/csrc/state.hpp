@@ -48,12 +48,12 @@ struct TimerPair {
 };
 
 // ------------------------------------------------ deferred literal calls ---
-enum LitOpKind { kLitMoments, kLitResetVelocity, kLitResetDensity, kLitCollide };
+enum LitOpKind { kLitPeriodic, kLitMoments, kLitResetVelocity, kLitResetDensity, kLitCollide };
 struct LitOp {
     LitOpKind kind;
     double tau;        // kLitCollide
     double force[3];   // kLitCollide
-    plb_boundary bc;   // the resets
+    plb_boundary bc;   // the periodic copies, the resets
 };
 
 }  // namespace plb
@@ -83,8 +83,9 @@ struct plb_state {
     // two-step launch, and any call that needs it done runs it first
     bool fused_deferred;
     // literal: calls deferred so that a following push can fold them into
-    // its kernel (at most moments, reset velocity, reset density, collide, in
-    // that order); any other call runs them first, in order
+    // its kernel (a run of periodicity, moments, reset velocity, reset density
+    // and collide, in that order, each of the first four directly after the
+    // one before it); any other call runs them first, in order
     std::vector<plb::LitOp> lit_queue;
     // literal: the last collide+push kernel stored its in-place values on the
     // outer layer only; ntmp off that layer is n(c + c_k, k) until restored
@@ -144,14 +145,18 @@ int lit_initialize(plb_state* s, double rho0, const double u0[3], const plb_init
 int lit_collide(plb_state* s, double tau, const double F[3]);
 int lit_push(plb_state* s);
 int lit_collide_push(plb_state* s, double tau, const double F[3]);
-// bc_vel: the faces whose velocity is reset; bc_rho: those whose density is
-int lit_moments_collide_push(plb_state* s, double tau, const double F[3], const plb_boundary* bc_vel,
-                             const plb_boundary* bc_rho);
+// bc_per: the periodic copies folded in (null: none); bc_vel: the faces whose
+// velocity is reset; bc_rho: those whose density is; bc_noslip: the no-slip
+// faces of this step, when nothing else reads rho or u before the next
+// moments (null: every rho and u is stored)
+int lit_moments_collide_push(plb_state* s, double tau, const double F[3], const plb_boundary* bc_per,
+                             const plb_boundary* bc_vel, const plb_boundary* bc_rho, const plb_boundary* bc_noslip);
 int lit_noslip(plb_state* s, const plb_boundary* bc);
 // The same pass for faces within the documented size limit of the entry point.
 int lit_noslip_noalloc(plb_state* s, const plb_boundary* bc);
 int lit_periodic(plb_state* s, const plb_boundary* bc);
-int lit_moments(plb_state* s);
+// with the resets that follow them in the same kernel (null: none)
+int lit_moments(plb_state* s, const plb_boundary* bc_vel, const plb_boundary* bc_rho);
 int lit_reset_velocity(plb_state* s, const plb_boundary* bc);
 int lit_reset_density(plb_state* s, const plb_boundary* bc);
 int lit_transfer(plb_state* s, int field, int layout, int dtype, void* host, bool upload);
