@@ -317,11 +317,13 @@ int plb_bench_pattern(int device, int q, int x, int y, int z, int sbytes, int ve
 #define PLB_TUNE_TWO_STEP 9     /* fused pull step: 1 advances two steps per launch   */
                                 /* (one read and one write of the populations per two */
                                 /* steps, the same values bit for bit) wherever a     */
-                                /* kernel exists: D3Q19 and D3Q27; x a multiple of 32; */
-                                /* each population's array below 4 GiB; 0 one step per */
-                                /* launch; -1 (default) automatic: on for             */
-                                /* 4- and 8-byte storage on lattices of at least 2^18 */
-                                /* cells (2^19 for D3Q27).  The staged calls pair     */
+                                /* kernel exists: D3Q19 and D3Q27, each population's  */
+                                /* array below 4 GiB, x a multiple of 32 (else        */
+                                /* lattices from 2^18 cells that are not thin); 0 one */
+                                /* step per launch; -1 (default) automatic: on from   */
+                                /* 2^18 cells (2^19 for D3Q27 with x a multiple of    */
+                                /* 32), but for 2-byte storage only where x is no     */
+                                /* multiple of 32.  The staged calls pair             */
                                 /* whole steps (plb_stream records one step and the   */
                                 /* next plb_stream launches both; any call that reads */
                                 /* or changes the state runs a recorded step first)   */
@@ -330,7 +332,7 @@ int plb_bench_pattern(int device, int q, int x, int y, int z, int sbytes, int ve
 #define PLB_TUNE_TWO_TILE_X 11  /* two-step tile width: 64 or 32 cells (one          */
                                 /* workgroup per compute unit either way, 32-cell     */
                                 /* tiles taller); 0 automatic: 32 for 8-byte storage, */
-                                /* else 64                                            */
+                                /* else 64, and for other rows a shape of their own   */
 int plb_set_tuning(plb_state* s, int key, int value);
 /* The streaming scheme the next fused steps will use: PLB_SCHEME_PUSH,
  * PLB_SCHEME_PULL, PLB_SCHEME_PULL_TWO (pull, two steps per launch, for

@@ -310,6 +310,7 @@ int plb_state_create(const plb_state_desc* d, plb_state** out) {
     s->tune_two = -1;
     s->tune_two_zc = 0;
     s->tune_two_bx = 0;
+    s->two_any_bx = s->two_any_by = 0;
     s->num_cu = 256;
     {
         int cu = 0;
@@ -328,6 +329,7 @@ int plb_state_create(const plb_state_desc* d, plb_state** out) {
         mom_bytes = s->ncell * s->sbytes;
     } else {
         s->ncell = X * Y * Z;
+        fused_two_plan(s);
         const size_t pad = d->pop_pad >= 0 ? (size_t)d->pop_pad : (size_t)(2048 + 64);
         s->pstride = ((s->ncell + 63) / 64) * 64 + pad;
         mom_bytes = s->ncell * sizeof(double);

@@ -684,12 +684,19 @@ enum KernelKind { kPush, kPull, kGather, kStreamOnly, kCollideOnly, kAaEven, kAa
 // L2.  The runs hold kx = ceil(pairs / 8) pairs (the last may be shorter),
 // so the rounds are counted per XCD.
 TwoGeom two_geom(const plb_state* s) {
-    const int bx = fused_two_tile_x(s);
-    const int by = two_rows(s->q, (int)s->sbytes, bx);
+    // rows of whole 64- or 32-cell tiles: the compiled shapes; other rows: the
+    // shape that two_shape finds
     TwoGeom g;
+    int bx = fused_two_tile_x(s), by;
+    g.any = bx == 0;
+    if (g.any)
+        bx = s->two_any_bx, by = s->two_any_by;
+    else
+        by = two_rows(s->q, (int)s->sbytes, bx);
     g.bx = (uint32_t)bx;
+    g.by = (uint32_t)by;
     g.wide = (s->tune_index64 || (uint64_t)s->q * s->pstride * s->sbytes > 0xffffffffull) ? 1u : 0u;
-    g.ntx = (uint32_t)s->X / (uint32_t)bx;
+    g.ntx = ((uint32_t)s->X + (uint32_t)bx - 1u) / (uint32_t)bx;
     g.nty = ((uint32_t)s->Y + (uint32_t)by - 1u) / (uint32_t)by;
     const uint64_t ntx = g.ntx, nty = g.nty, Z = (uint64_t)s->Z;
     const uint64_t ncu = (uint64_t)s->num_cu;  // workgroups resident at once (one per compute unit)
@@ -794,7 +801,12 @@ int launch_kind(plb_state* s, KernelKind kind) {
         a.xcd = (uint32_t)xm;
         a.dper = make_fastdiv(xm == 2 ? ntx * (nty / 8) : 1u);
         a.nt_load = s->tune_nt_load;
-        a.nt_store = s->tune_nt_store;
+        // A cell kernel's row that is no whole number of lines ends inside a
+        // line that the next row's wavefronts go on writing; ordinary stores
+        // let the L2 put such lines together (D3Q19 250 x 191 x 133 per step:
+        // FP32-shifted with solids 290 -> 239 us, FP16-shifted 160 -> 137,
+        // FP64 200 x 50 x 50 34 -> 31).
+        a.nt_store = s->tune_nt_store && (kind != kPull || (uint64_t)s->X * sizeof(S) % 128 == 0);
         a.tau = (T)s->tau;
         if (std::is_same<T, float>::value)  // CollisionSRT.cpp:19-20
             a.om = (T)(1. / (double)a.tau);
@@ -932,8 +944,34 @@ int fused_two_tile_x(const plb_state* s) {
     return 0;
 }
 
+void fused_two_plan(plb_state* s) {
+    const TwoShape sh = s->q == 9 ? TwoShape{0, 0} : two_shape(s->q, (int)s->sbytes, s->X, s->Y);
+    s->two_any_bx = sh.bx;
+    s->two_any_by = sh.by;
+}
+
 bool fused_two_eligible(const plb_state* s) {
     if (s->tune_two == 0 || s->aa || !fused_uses_pull(s) || s->mode != PLB_MODE_FUSED) return false;
+    if (s->q != 19 && s->q != 27) return false;
+    // offsets within one population array are 32-bit
+    if ((uint64_t)s->pstride * s->sbytes > 0xffffffffull) return false;
+    const uint64_t cells = (uint64_t)s->X * (uint64_t)s->Y * (uint64_t)s->Z;
+    if (fused_two_tile_x(s) == 0) {
+        // Rows that are no whole number of 32-cell tiles run in tiles of
+        // their own shape (two_shape), with every storage type, from 2^18
+        // cells on.  Their one-step kernel loads and stores rows at any
+        // alignment, and two steps per launch measured faster from there:
+        // D3Q19 250 x 191 x 133 290 -> 155-159 us per step (FP32-shifted,
+        // solids), 475 -> 272 (FP64), 160 -> 120 (FP16-shifted), 200 x 50 x 50
+        // FP64 34 -> 19; D3Q27 75 x 70 x 70 36 -> 23 (FP64), 28 -> 18; below,
+        // 50^3 (2^17 cells) ran 9.7 -> 8.8 (FP64) and 7.2 -> 7.8 (FP32-shifted),
+        // 40^3 5.1 -> 8.2.  Not where the grown borders (one layer each side in
+        // y and z as in x) make up for the saved pass: thin lattices.  A
+        // forced tile width that does not divide the row has no such kernel.
+        if (s->tune_two_bx > 0 || s->X % 32 == 0 || cells < (1ull << 18)) return false;
+        const double grown = (s->two_any_bx + 2.0) * (s->two_any_by + 2.0) * (s->Z + 2.0);
+        return grown <= 1.75 * s->two_any_bx * s->two_any_by * (double)s->Z;
+    }
     // automatic: 4- and 8-byte storage, where two steps per pass measured
     // 1.40x (D3Q19 256^3 FP32-shifted, 10% solids), 1.57x (walls only), 1.26x
     // and 1.41x (FP64), 1.35x (D3Q27 FP32-shifted, walls) and 1.21x (D3Q27
@@ -945,11 +983,7 @@ bool fused_two_eligible(const plb_state* s) {
     // that the launch has too few tiles and chunks of a few planes, and one
     // step per launch measured faster (32^3: 0.66-0.91x; 64 x 64 x 32:
     // 0.67-0.96x; D3Q27 64^3: 0.89-0.94x; D3Q19 64^3 0.94-1.27x)
-    const uint64_t cells = (uint64_t)s->X * (uint64_t)s->Y * (uint64_t)s->Z;
     if (s->tune_two < 0 && cells < (s->q == 27 ? (1ull << 19) : (1ull << 18))) return false;
-    if ((s->q != 19 && s->q != 27) || fused_two_tile_x(s) == 0) return false;
-    // offsets within one population array are 32-bit
-    if ((uint64_t)s->pstride * s->sbytes > 0xffffffffull) return false;
     return true;
 }
 

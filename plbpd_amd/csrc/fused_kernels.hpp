@@ -112,8 +112,8 @@ struct Seams {
     bool wxm, wxp, wym, wyp, wzm, wzp;
 };
 
-template <class I, class T>
-__device__ inline Seams<I> seams(uint32_t x, uint32_t y, uint32_t z, const FusedArgs<T>& a) {
+template <class I, class Args>
+__device__ inline Seams<I> seams(uint32_t x, uint32_t y, uint32_t z, const Args& a) {
     const I X = a.X, XY = (I)a.X * a.Y;
     Seams<I> s;
     s.xm = x == 0 ? (I)(a.X - 1) : (I)0 - (I)1;
@@ -300,9 +300,8 @@ __device__ inline void own_store(const typename Prec<V>::T (&f)[Q], typename Pre
 // taken from the fluid cell's seams with no load (a load of the flag under
 // the branch would make the kernel wait for every load in flight before it,
 // the two-step kernel's next planes among them).
-template <int Q, int K, class P, class I>
-__device__ inline void wall_terms(typename P::T (&f)[Q], typename P::T rho, const Seams<I>& s,
-                                  const FusedArgs<typename P::T>& a) {
+template <int Q, int K, class P, class I, class Args>
+__device__ inline void wall_terms(typename P::T (&f)[Q], typename P::T rho, const Seams<I>& s, const Args& a) {
     using T = typename P::T;
     if constexpr (K < Q) {
         constexpr int R = rev_k<Q>(K);
@@ -322,9 +321,8 @@ __device__ inline void wall_terms(typename P::T (&f)[Q], typename P::T rho, cons
 // wall_terms for a fluid cell, skipped by the wavefronts none of whose cells
 // is next to a wall face (the vote keeps a branch the compiler would
 // otherwise turn into arithmetic for every cell).
-template <int Q, class P, class I>
-__device__ inline void moving_wall_terms(typename P::T (&f)[Q], typename P::T rho, const Seams<I>& s,
-                                         const FusedArgs<typename P::T>& a) {
+template <int Q, class P, class I, class Args>
+__device__ inline void moving_wall_terms(typename P::T (&f)[Q], typename P::T rho, const Seams<I>& s, const Args& a) {
     if (__any(s.wxm || s.wxp || s.wym || s.wyp || s.wzm || s.wzp)) wall_terms<Q, 1, P>(f, rho, s, a);
 }
 
@@ -346,8 +344,8 @@ void fill_wall_cub(const FusedBC<T>& bc, T (&wcub)[27][3]) {
 
 // Moments and, when `collide`, the BGK update with the velocity-shift force
 // in place (bgk.hpp).  Returns rho.
-template <int Q, class P>
-__device__ inline typename P::T bgk(typename P::T (&f)[Q], const FusedArgs<typename P::T>& a, bool collide) {
+template <int Q, class P, class Args>
+__device__ inline typename P::T bgk(typename P::T (&f)[Q], const Args& a, bool collide) {
     return bgk_update<Q, P>(f, a.tau, a.om, a.omm, a.F0, a.F1, a.F2, collide);
 }
 
@@ -384,7 +382,9 @@ struct TwoGeom {
     uint32_t ntx, nty, nzc, zc;
     uint32_t xcd;   // 1: XCD j takes the j-th run of kx (z-chunk, y-tile) pairs; 0: workgroup i takes tile i
     uint32_t kx;
-    uint32_t bx;    // tile width, 64 or 32 cells (one workgroup per compute unit either way)
+    uint32_t bx;    // tile width (one workgroup per compute unit whatever the shape)
+    uint32_t by;    // tile rows
+    uint32_t any;   // 1: a tile shape outside the compiled 64- and 32-cell ones (two_cap)
     uint32_t wide;  // population arrays beyond 4 GiB: per-population base pointers
 };
 // Workgroups of a two-step launch (with the XCD mapping, eight runs of kx
@@ -469,8 +469,42 @@ __host__ __device__ constexpr int two_rows(int q, int sbytes, int bx) {
 // slower at 384^3).
 __host__ __device__ constexpr int two_tile_pref(int q, int sbytes) { return (void)q, sbytes == 8 ? 32 : 64; }
 
-// Two pull steps in one pass (fused_two.hpp), tiles of g.bx x two_rows(Q, S,
-// g.bx) cells.  Returns false where no kernel exists for (Q, V, g.bx, g.wide).
+// Cells of a grown tile, (bx + 2) x (by + 2), that a tile of any shape may
+// have: what fits the LDS, in whole wavefronts where the ring allows it.
+__host__ __device__ constexpr int two_cap(int q, int sbytes) {
+    const int lds = 160 * 1024 / (zring_planes(q) * sbytes + 8);
+    const int maxc = two_split(q, sbytes, true) && sbytes == 4 ? 704 : 1024;
+    return lds < maxc ? (lds > 448 && sbytes == 8 ? 448 : lds) : maxc;
+}
+// The tile shape for rows of X cells and Y rows: nx x ny equal tiles (the last
+// of a row or column may be short).  A launch costs the grown cells of every
+// tile, (bx + 2) x (by + 2) x nx x ny, and the lines its rows touch: a row of
+// (bx + 2) values at any alignment touches one line more than it fills.  (Of
+// the widths of 250, 200, 173, 130, 100, 70 and 36 cells tried on MI355X with
+// 3 to 8 tiles a row, the pick is within 5% of the best for each.)
+struct TwoShape {
+    int bx, by;
+};
+inline TwoShape two_shape(int q, int sbytes, int X, int Y) {
+    const int cap = two_cap(q, sbytes);
+    TwoShape best{0, 0};
+    double cost = 0;
+    const int widest = X < cap / 3 - 2 ? X : cap / 3 - 2;  // at least one row fits
+    for (int w = widest < 8 ? widest : 8; w <= widest; ++w) {
+        const int nx = (X + w - 1) / w, bx = (X + nx - 1) / nx;
+        int by = cap / (bx + 2) - 2;
+        by = by < Y ? by : Y;
+        const int ny = (Y + by - 1) / by;
+        by = (Y + ny - 1) / ny;
+        const double lines = ((bx + 2.0) * sbytes / 128 + 1) / (bx * sbytes / 128.0);
+        const double c = (double)((bx + 2) * (by + 2)) * nx * ny * (1 + 0.25 * lines);
+        if (!best.bx || c < cost) best = TwoShape{bx, by}, cost = c;
+    }
+    return best;
+}
+
+// Two pull steps in one pass (fused_two.hpp), tiles of g.bx x g.by cells.
+// Returns false where no kernel exists for (Q, V, g).
 template <int Q, int V>
 bool launch_pull2(const FusedArgs<typename Prec<V>::T>& a, const TwoGeom& g, bool nb, bool mov,
                   const typename Prec<V>::S* A, typename Prec<V>::S* B, const uint8_t* flags,

@@ -5,9 +5,9 @@
 // Boundary.cpp:189-221), bit for bit, from one read of the populations of
 // step t and one write of those of step t + 2.
 //
-// A workgroup owns a tile of BX x-cells by BY y-rows and sweeps it along z
+// A workgroup owns a tile of bx x-cells by by y-rows and sweeps it along z
 // over a chunk of planes.  At each plane zi it computes step t + 1 on the
-// tile grown by one cell in x and y ((BX + 2) x (BY + 2) cells, one per
+// tile grown by one cell in x and y ((bx + 2) x (by + 2) cells, one per
 // thread), gathering step t from HBM, and keeps the result in an LDS ring
 // (ZRing: the directions with c_z = +1 for three planes, the others for
 // two).  It then computes step t + 2 on the tile at plane zi - 1, gathering
@@ -154,16 +154,17 @@ __device__ inline void ring_store(const typename Prec<V>::T (&f)[Q], typename Pr
 // rev(k) in plane zo where x - c_k is not fluid.  Slots: pa = the c_z = +1
 // group's slot of plane zo - 1, oa = its slot of plane zo, b0 = the other
 // groups' slot of plane zo, c1 = the c_z = -1 group's slot of plane zo + 1.
-template <int Q, int K, int V, int NB, int NI, int RX>
+// RX: cells per grown row.
+template <int Q, int K, int V, int NB, int NI>
 __device__ inline void ring_gather(typename Prec<V>::T (&f)[Q], const typename Prec<V>::S* ring, uint32_t li,
-                                   uint32_t pa, uint32_t oa, uint32_t b0, uint32_t c1, uint32_t m,
+                                   uint32_t RX, uint32_t pa, uint32_t oa, uint32_t b0, uint32_t c1, uint32_t m,
                                    const Seams<uint32_t>& s) {
     if constexpr (K < Q) {
         using Z = ZRing<Q>;
         constexpr int R = rev_k<Q>(K);
         constexpr int cx = Lat<Q>::cx(K), cy = Lat<Q>::cy(K);
         constexpr int g = Z::grp(K), gr = Z::grp(R);
-        const uint32_t moved = ring_at<Q, K, NI>(g == 0 ? pa : (g == 1 ? b0 : c1)) + li - (uint32_t)(cx + cy * RX);
+        const uint32_t moved = ring_at<Q, K, NI>(g == 0 ? pa : (g == 1 ? b0 : c1)) + li - ((uint32_t)cx + (uint32_t)cy * RX);
         const uint32_t own = ring_at<Q, R, NI>(gr == 0 ? oa : b0) + li;
         if constexpr (NB != 0) {
             // own - moved is uniform (li cancels) and, like every ring index,
@@ -174,7 +175,7 @@ __device__ inline void ring_gather(typename Prec<V>::T (&f)[Q], const typename P
         } else {
             f[K] = Prec<V>::load_raw(ring[pull_wall<Q, K>(s) ? own : moved]);
         }
-        ring_gather<Q, K + 1, V, NB, NI, RX>(f, ring, li, pa, oa, b0, c1, m, s);
+        ring_gather<Q, K + 1, V, NB, NI>(f, ring, li, RX, pa, oa, b0, c1, m, s);
     }
 }
 
@@ -189,50 +190,40 @@ __device__ inline void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <int Q, int V, int NB, bool MOV, int BX, int BY, bool W, bool SPLIT>
-__global__ __launch_bounds__(two_threads(BX, BY), 1) void k_pull2(const typename Prec<V>::S* __restrict__ A,
-                                                           typename Prec<V>::S* __restrict__ B,
-                                                           const uint8_t* __restrict__ flags,
-                                                           const uint32_t* __restrict__ nbmask,
-                                                           FusedArgs<typename Prec<V>::T> a, TwoGeom g) {
+// The sweep of one workgroup over the planes [z0, z0 + zc) of the tile of
+// bx x by cells at (x0, y0).  BX, BY: the tile shape where it is compiled in;
+// BX = 0: any shape of at most two_cap() grown cells (bx, by), the ring laid
+// out for that many.  a: FusedArgs, or the like for one domain of a batch.
+template <int Q, int V, int NB, bool MOV, int BX, int BY, bool W, bool SPLIT, class Args>
+__device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict__ A,
+                                           typename Prec<V>::S* __restrict__ B, const uint8_t* __restrict__ flags,
+                                           const uint32_t* __restrict__ nbmask, const Args& a, uint32_t bx,
+                                           uint32_t by, uint32_t x0, uint32_t y0, uint32_t z0, uint32_t zc) {
     using P = Prec<V>;
     using S = typename P::S;
     using T = typename P::T;
     using I = uint32_t;
-    constexpr int RX = BX + 2, NI = two_cells(BX, BY);
+    constexpr int NI = BX ? two_cells(BX, BY) : two_cap(Q, (int)sizeof(S));
+    const uint32_t TX = BX ? (uint32_t)BX : bx, TY = BX ? (uint32_t)BY : by;  // tile cells
+    const uint32_t RX = TX + 2u;                                              // grown row
     __shared__ S ring[ZRing<Q>::planes() * NI];
     __shared__ uint32_t mring[2 * NI];  // the step t + 1 cells' masks or flags, two planes
 
     const uint32_t tid = threadIdx.x;
-    uint32_t tx, ty, tz;
-    if (g.xcd) {
-        // workgroup i runs on XCD i mod 8, which takes pairs [j kx, (j + 1) kx)
-        const uint32_t j = blockIdx.x & 7u, m = blockIdx.x >> 3;
-        tx = m % g.ntx;
-        const uint32_t pr = j * g.kx + m / g.ntx;
-        if (pr >= g.nty * g.nzc) return;  // past the last pair (the whole workgroup)
-        ty = pr % g.nty;
-        tz = pr / g.nty;
-    } else {
-        tx = blockIdx.x % g.ntx;
-        const uint32_t r = blockIdx.x / g.ntx;
-        ty = r % g.nty;
-        tz = r / g.nty;
-    }
     const uint32_t X = a.X, Y = a.Y, Z = a.Z;
     const I XY = X * Y, ps = (I)a.pstride;
-    const uint32_t x0 = tx * (uint32_t)BX, y0 = ty * (uint32_t)BY, z0 = tz * g.zc;
-    const uint32_t nplanes = std::min(g.zc, Z - z0) + 2u;
+    const uint32_t nplanes = std::min(zc, Z - z0) + 2u;
 
     // step t + 1: this thread's cell of the grown tile (wrapped coordinates)
-    const bool in_i = tid < (uint32_t)NI;
+    const bool in_i = tid < (BX ? (uint32_t)NI : RX * (TY + 2u));
     const uint32_t ix = tid % RX, iy = tid / RX;
     const uint32_t gx = (x0 + ix + X - 1u) % X, gy = (y0 + iy + Y - 1u) % Y;
     // step t + 2: this thread's cell of the tile
-    const uint32_t ox = tid % (uint32_t)BX, oy = tid / (uint32_t)BX;
-    const bool in_o = oy < (uint32_t)BY && y0 + oy < Y;
+    const uint32_t ox = tid % TX, oy = tid / TX;
+    const bool in_o = oy < TY && y0 + oy < Y && x0 + ox < X;
     const uint32_t px = x0 + ox, py = y0 + oy;
-    const I li = (oy + 1u) * RX + ox + 1u;
+    // (threads without a cell, which take no part in step t + 2, read cell 0)
+    const I li = BX || in_o ? (oy + 1u) * RX + ox + 1u : 0u;
 
     // Loads of step t, issued an iteration ahead of the plane that uses them.
     // SPLIT issues the directions with c_z = +1 two iterations ahead instead,
@@ -288,7 +279,7 @@ __global__ __launch_bounds__(two_threads(BX, BY), 1) void k_pull2(const typename
         if (!__all(self_solid)) {
             const Seams<I> sm = seams<I>(px, py, zo, a);
             T f[Q];
-            ring_gather<Q, 0, V, NB, NI, RX>(f, ring, li, pa, oa, b0, c1, mo, sm);
+            ring_gather<Q, 0, V, NB, NI>(f, ring, li, RX, pa, oa, b0, c1, mo, sm);
             if (!self_solid) {
                 const T rho = bgk<Q, P>(f, a, true);
                 if (MOV && a.bc.moving) moving_wall_terms<Q, P>(f, rho, sm, a);
@@ -376,17 +367,49 @@ __global__ __launch_bounds__(two_threads(BX, BY), 1) void k_pull2(const typename
     }
 }
 
+// Threads of a workgroup: one per grown cell, in whole wavefronts.
+__host__ __device__ constexpr int pull2_threads(int q, int sbytes, int bx, int by) {
+    return bx ? two_threads(bx, by) : (two_cap(q, sbytes) + 63) / 64 * 64;
+}
+
+template <int Q, int V, int NB, bool MOV, int BX, int BY, bool W, bool SPLIT>
+__global__ __launch_bounds__(pull2_threads(Q, (int)sizeof(typename Prec<V>::S), BX, BY), 1) void k_pull2(
+    const typename Prec<V>::S* __restrict__ A, typename Prec<V>::S* __restrict__ B,
+    const uint8_t* __restrict__ flags, const uint32_t* __restrict__ nbmask, FusedArgs<typename Prec<V>::T> a,
+    TwoGeom g) {
+    uint32_t tx, ty, tz;
+    if (g.xcd) {
+        // workgroup i runs on XCD i mod 8, which takes pairs [j kx, (j + 1) kx)
+        const uint32_t j = blockIdx.x & 7u, m = blockIdx.x >> 3;
+        tx = m % g.ntx;
+        const uint32_t pr = j * g.kx + m / g.ntx;
+        if (pr >= g.nty * g.nzc) return;  // past the last pair (the whole workgroup)
+        ty = pr % g.nty;
+        tz = pr / g.nty;
+    } else {
+        tx = blockIdx.x % g.ntx;
+        const uint32_t r = blockIdx.x / g.ntx;
+        ty = r % g.nty;
+        tz = r / g.nty;
+    }
+    const uint32_t bx = BX ? (uint32_t)BX : g.bx, by = BX ? (uint32_t)BY : g.by;
+    pull2_tile<Q, V, NB, MOV, BX, BY, W, SPLIT>(A, B, flags, nbmask, a, bx, by, tx * bx, ty * by, tz * g.zc, g.zc);
+}
+
 }  // namespace
 
+// Tiles BX cells wide in their compiled shape; BX = 0: any shape.
 template <int Q, int V, int BX, bool W>
 bool launch_pull2_bx(const FusedArgs<typename Prec<V>::T>& a, const TwoGeom& g, bool nb, bool mov,
                      const typename Prec<V>::S* A, typename Prec<V>::S* B, const uint8_t* flags,
                      const uint32_t* nbmask, hipStream_t stream) {
-    constexpr int sb = (int)sizeof(typename Prec<V>::S), BY = two_rows(Q, sb, BX);
-    if constexpr (BY == 0) {
+    constexpr int sb = (int)sizeof(typename Prec<V>::S), BY = BX ? two_rows(Q, sb, BX) : 0;
+    if constexpr (BX != 0 && BY == 0) {
         return false;
     } else {
-        const dim3 grid(two_blocks(g)), block(two_threads(BX, BY));
+        // a tile of any shape must fit the ring and the workgroup
+        if (BX == 0 && ((int)((g.bx + 2) * (g.by + 2)) > two_cap(Q, sb) || g.bx < 1 || g.by < 1)) return false;
+        const dim3 grid(two_blocks(g)), block(pull2_threads(Q, sb, BX, BY));
 #define PLB_TWO(NBv, MVv)                                                                               \
     hipLaunchKernelGGL((k_pull2<Q, V, NBv, MVv, BX, BY, W, two_split(Q, sb, NBv != 0)>), grid, block, 0, \
                        stream, A, B, flags, nbmask, a, g)
@@ -403,10 +426,15 @@ template <int Q, int V>
 bool launch_pull2(const FusedArgs<typename Prec<V>::T>& a, const TwoGeom& g, bool nb, bool mov,
                   const typename Prec<V>::S* A, typename Prec<V>::S* B, const uint8_t* flags,
                   const uint32_t* nbmask, hipStream_t stream) {
-    if (g.bx == 64 && !g.wide) return launch_pull2_bx<Q, V, 64, false>(a, g, nb, mov, A, B, flags, nbmask, stream);
-    if (g.bx == 64) return launch_pull2_bx<Q, V, 64, true>(a, g, nb, mov, A, B, flags, nbmask, stream);
-    if (g.bx == 32 && !g.wide) return launch_pull2_bx<Q, V, 32, false>(a, g, nb, mov, A, B, flags, nbmask, stream);
-    if (g.bx == 32) return launch_pull2_bx<Q, V, 32, true>(a, g, nb, mov, A, B, flags, nbmask, stream);
+    const bool w = g.wide != 0;
+    auto go = [&](auto bxc) {
+        constexpr int BX = decltype(bxc)::value;
+        return w ? launch_pull2_bx<Q, V, BX, true>(a, g, nb, mov, A, B, flags, nbmask, stream)
+                 : launch_pull2_bx<Q, V, BX, false>(a, g, nb, mov, A, B, flags, nbmask, stream);
+    };
+    if (g.any) return go(std::integral_constant<int, 0>());
+    if (g.bx == 64) return go(std::integral_constant<int, 64>());
+    if (g.bx == 32) return go(std::integral_constant<int, 32>());
     return false;
 }
 

@@ -1,0 +1,66 @@
+"""Two pull steps per launch on rows that are no whole number of 32-cell tiles
+(automatic from 2^18 cells): tiles of a shape of their own, the last of a row
+or column cut short, rows of a few cells, walls on each axis with a moving
+wall, periodic seams, solids and every storage type, against the oracle's
+corrected step and against one step per launch, bit for bit."""
+import numpy as np
+import pytest
+
+import plbpd_amd as P
+from plbpd_amd import capi
+from oracle.pyoracle import Boundary, NOSLIP, PERIODIC
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # q, X, Y, Z, walled axis or None, solids, index64
+    (19, 70, 61, 63, 2, True, 0),
+    (19, 131, 47, 43, 1, False, 0),
+    (19, 5, 230, 229, 0, False, 0),
+    (19, 250, 37, 29, None, True, 1),
+    (19, 33, 90, 89, 2, False, 1),
+    (27, 101, 53, 50, 2, True, 0),
+    (27, 47, 75, 76, 0, False, 1),
+]
+
+
+@pytest.mark.parametrize("q,X,Y,Z,axis,solids,wide", CASES)
+@pytest.mark.parametrize("variant", ["f64", "f32s", "f16s", "f32"])
+def test_ragged_two_step_matches_oracle(orc, q, X, Y, Z, axis, solids, wide, variant):
+    print(f"\n[case] ragged two-step {variant} q={q} {X}x{Y}x{Z} walls={axis} solids={solids}", flush=True)
+    types, vel = [PERIODIC] * 6, {}
+    if axis is not None:
+        types[2 * axis] = types[2 * axis + 1] = NOSLIP
+        vel = {2 * axis: (0.02, 0.01, -0.01), 2 * axis + 1: (0.0, 0.0, 0.0)}
+    ob, pb = Boundary(type=types, vel=vel), P.boundary(types, vel)
+    mask = (np.random.default_rng(8).random((Z, Y, X)) < 0.12).astype(np.uint8) if solids else None
+    tau, F, init, steps = 0.62, (2e-5, -1e-6, 1e-6), (P.INIT_PERTURBED, 5, 2e-3), 5
+    o = orc.cor_state(variant, q, X, Y, Z)
+    orc.cor_init(o, 1.0, (0.01, 0.0, 0.0), init)
+    orc.cor_run(o, tau, F, ob, steps, mask)
+    fluid = orc.cor_flags(q, X, Y, Z, ob, mask) == 0
+    raws = []
+    for two in (-1, 0):
+        with P.State(q, X, Y, Z, variant, P.FUSED) as st:
+            st.set_tuning(capi.TUNE_TWO_STEP, two)
+            st.set_tuning(capi.TUNE_INDEX64, wide)
+            assert st.scheme() == ("pull2" if two else "pull")
+            st.set_boundary(pb, mask)
+            st.initialize(1.0, (0.01, 0.0, 0.0), init, pb)
+            st.configure(tau, F, pb)
+            st.step(steps)
+            raw = st.download_raw()
+        raws.append(raw.view(np.uint16) if variant == "f16s" else raw)
+    exp = o["f"].view(np.uint16) if variant == "f16s" else o["f"]
+    assert np.array_equal(raws[0][fluid], exp[fluid])
+    assert np.array_equal(raws[0][fluid], raws[1][fluid])
+
+
+def test_ragged_two_step_rule():
+    """Thin lattices and those below 2^18 cells keep one step per launch."""
+    for q, X, Y, Z, want in ((19, 70, 61, 63, "pull2"), (19, 600, 1, 500, "pull"), (19, 500, 600, 1, "pull"),
+                             (19, 61, 64, 64, "pull"), (27, 75, 70, 70, "pull2")):
+        with P.State(q, X, Y, Z, "f32s", P.FUSED) as st:
+            assert st.scheme() == want, (q, X, Y, Z)
+    with P.State(19, 70, 61, 63, "f64", P.FUSED) as st:
+        st.set_tuning(capi.TUNE_TWO_TILE_X, 32)
+        assert st.scheme() == "pull"
