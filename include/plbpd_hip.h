@@ -376,8 +376,10 @@ int plb_batch_get_mapping(const plb_batch* b, int* xcd_runs);
  * the call leaves the simulation that many steps times 60 further on (an
  * even count); initialise the batch again to start from its initial state. */
 int plb_batch_autotune(plb_batch* b, int steps, double* results, int max_results, int* nresults);
-/* nsteps of all domains: one launch per step (graph-captured when
- * steps_per_graph > 0). */
+/* nsteps of all domains: one launch per step, or per two steps of the pull
+ * scheme (D3Q19 and D3Q27, from 2^18 cells in all, domains that are not thin;
+ * the same values bit for bit), graph-captured when steps_per_graph > 0.  The
+ * tiling and mapping are those of the one-step launches. */
 int plb_batch_step(plb_batch* b, int nsteps, int steps_per_graph);
 /* Baseline: the same steps with one launch per domain per step. */
 int plb_batch_step_per_domain(plb_batch* b, int nsteps);

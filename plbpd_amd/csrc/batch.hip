@@ -10,7 +10,8 @@
 // workgroup i takes tile i (a persistent block strides by the grid), so the
 // chip sweeps one window of memory; the XCD mapping instead hands each XCD a
 // contiguous run of tiles, so a domain's neighbouring rows share an L2
-// (batch_tiles).  The per-cell work is the step of fused.hip, pull (the
+// (batch_tiles).  Pairs of pull steps run as one launch of the two-step kernel
+// (batch_two.hpp) where two_step_plan finds that worth it.  The per-cell work is the step of fused.hip, pull (the
 // default) or push: the same collision, periodic wraps on periodic axes and
 // halfway bounce-back on the wall layers of no-slip faces (stationary or
 // moving).
@@ -18,11 +19,12 @@
 #include <cmath>
 #include <string>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
+#include "batch.hpp"
 #include "bgk.hpp"
-#include "fastdiv.hpp"
-#include "state.hpp"
+#include "fused_kernels.hpp"
 
 struct plb_batch;
 
@@ -30,15 +32,6 @@ namespace plb {
 namespace {
 
 constexpr int kMaxBlock = 256;
-
-template <class T>
-struct BDom {
-    uint32_t X, Y, Z, N;
-    FastDiv dX, dY;  // division by X and Y (cell -> coordinates)
-    uint64_t off;    // element offset of population 0 in the pool
-    uint64_t ps;     // elements between populations
-    T tau, om, omm, F0, F1, F2;
-};
 
 // Coordinates of cell c of a domain.
 template <class T>
@@ -388,6 +381,9 @@ struct plb_batch {
     void* doms;       // BDom<T> array on the device
     uint2* tiles;     // tile table on the device
     uint32_t ntiles;
+    BTile* two_tiles; // two-step launches: tile table on the device
+    uint32_t ntwo;    // its tiles; 0 = one step per launch
+    bool two_off;     // one step per launch while candidates for it are timed
     int tile;         // cells per tile
     int grid;         // persistent grid blocks (0 = one block per tile)
     hipStream_t stream;
@@ -414,6 +410,83 @@ int batch_layout(plb_batch* b, int tile) {
     PLB_HIP_TRY(hipMemcpy(b->tiles, t.data(), t.size() * sizeof(uint2), hipMemcpyHostToDevice));
     b->ntiles = (uint32_t)t.size();
     b->tile = tile;
+    return PLB_OK;
+}
+
+// The tiles of a two-step launch, or none where one step per launch is the
+// better choice.  A domain's cross-section is cut into tiles of two_shape(),
+// and its planes into chunks of at most zc, one zc for the batch: a chunk costs
+// its planes and the two grown ones, and a launch takes its work over the
+// compute units (one workgroup each) plus about half of its largest chunk, on
+// which the last of them wait.  Workgroups are dispatched in order, so the
+// largest chunks come first; workgroup i runs on XCD i mod 8, and within every
+// 256 workgroups XCD j takes a run of 32, whose tiles mostly belong to one
+// domain and share their borders in that XCD's L2 (the runs in turn from the
+// largest and from the smallest, to spread the work evenly).
+// Two steps per launch from 2^18 cells on, unless the grown borders (domains a
+// few layers thin) cost more than the saved pass: the rule of
+// fused_two_eligible.  512 domains of edges 16 to 96 (44.8 M cells, D3Q19
+// FP32-shifted): 1,162 -> 881 us per step (FP64 2,570 -> 1,628, FP16-shifted
+// 792 -> 673); 64 domains (6.1 M) 160 -> 140, 16 (1.1 M) 28.9 -> 28.6 (FP64 59
+// -> 48).
+int two_step_plan(plb_batch* b, int ncu) {
+    b->ntwo = 0;
+    if (b->q == 9 || b->total_cells < (1ull << 18)) return PLB_OK;
+    const int sb = (int)b->sbytes;
+    std::vector<TwoShape> shape(b->ndom);
+    int zmax = 1;
+    for (int d = 0; d < b->ndom; ++d) {
+        // 32-bit byte offsets within a domain
+        if ((uint64_t)b->q * b->ps[d] * sb > 0xffffffffull) return PLB_OK;
+        shape[d] = two_shape(b->q, sb, b->desc[d].x, b->desc[d].y);
+        zmax = std::max(zmax, b->desc[d].z);
+    }
+    const double cap = two_cap(b->q, sb);
+    // a short tile still pays its barriers and latencies
+    auto weight = [&](const TwoShape& t) { return 0.35 + 0.65 * (t.bx + 2) * (t.by + 2) / cap; };
+    double best = 0;
+    int zbest = zmax;
+    for (int zc = zmax; zc >= 4; zc = zc * 3 / 4) {
+        double total = 0, most = 0;
+        for (int d = 0; d < b->ndom; ++d) {
+            const plb_domain_desc& D = b->desc[d];
+            const TwoShape& t = shape[d];
+            const double n = (double)((D.x + t.bx - 1) / t.bx) * ((D.y + t.by - 1) / t.by), w = weight(t);
+            const int chunks = (D.z + zc - 1) / zc, c = (D.z + chunks - 1) / chunks;
+            total += n * w * (D.z + 2.0 * chunks);
+            most = std::max(most, w * (c + 2));
+        }
+        const double cost = std::max(total / ncu, most) + 0.5 * most;
+        if (best == 0 || cost < best) best = cost, zbest = zc;
+    }
+    std::vector<std::pair<double, BTile>> list;
+    double grown = 0;
+    for (int d = 0; d < b->ndom; ++d) {
+        const plb_domain_desc& D = b->desc[d];
+        const TwoShape& t = shape[d];
+        const int chunks = (D.z + zbest - 1) / zbest, c = (D.z + chunks - 1) / chunks;
+        for (int z = 0; z < D.z; z += c)
+            for (int y = 0; y < D.y; y += t.by)
+                for (int x = 0; x < D.x; x += t.bx) {
+                    const int planes = std::min(c, D.z - z) + 2;
+                    grown += (double)(t.bx + 2) * (t.by + 2) * planes;
+                    list.push_back({weight(t) * planes, BTile{(uint32_t)d, (uint32_t)x, (uint32_t)y, (uint32_t)z,
+                                                              (uint32_t)c, (uint32_t)t.bx, (uint32_t)t.by, 0}});
+                }
+    }
+    if (grown > 1.75 * (double)b->total_cells || list.size() >= (1ull << 31)) return PLB_OK;
+    std::stable_sort(list.begin(), list.end(), [](const auto& l, const auto& r) { return l.first > r.first; });
+    std::vector<BTile> order(list.size());
+    for (size_t g = 0; g < list.size(); g += 256) {
+        const size_t per = std::min<size_t>(256, list.size() - g) / 8;
+        for (size_t j = 0; j < 8; ++j)
+            for (size_t m = 0; m < per; ++m)
+                order[g + m * 8 + j] = list[g + ((g / 256) % 2 ? 7 - j : j) * per + m].second;
+        for (size_t i = g + 8 * per; i < std::min(list.size(), g + 256); ++i) order[i] = list[i].second;
+    }
+    PLB_HIP_TRY(hipMalloc(&b->two_tiles, order.size() * sizeof(BTile)));
+    PLB_HIP_TRY(hipMemcpy(b->two_tiles, order.data(), order.size() * sizeof(BTile), hipMemcpyHostToDevice));
+    b->ntwo = (uint32_t)order.size();
     return PLB_OK;
 }
 
@@ -500,6 +573,32 @@ int batch_launch(plb_batch* b, uint32_t t0, uint32_t t1, bool persistent_ok, int
 
 bool batch_pull(const plb_batch* b) { return b->scheme != PLB_SCHEME_PUSH; }
 
+// Whether pairs of steps run as one launch (post-collision storage is needed too).
+bool batch_two(const plb_batch* b) { return b->ntwo > 0 && !b->two_off && batch_pull(b); }
+
+int batch_launch_two(plb_batch* b) {
+    const int rc = with_qv_b(b->q, b->variant, [&](auto qc, auto vc) {
+        constexpr int Q = decltype(qc)::value;
+        constexpr int V = decltype(vc)::value;
+        using P = Prec<V>;
+        using T = typename P::T;
+        using S = typename P::S;
+        if constexpr (Q == 9) {
+            return fail(PLB_ERR_LOGIC, "no two-step kernel for D2Q9");
+        } else {
+            FusedBC<T> bc;
+            make_fused_bc<T>(b->bc, b->q, &bc);
+            if (!launch_batch2<Q, V>((const S*)b->buf[b->cur], (S*)b->buf[b->cur ^ 1], (const BDom<T>*)b->doms,
+                                     b->two_tiles, b->ntwo, bc, b->stream))
+                return fail(PLB_ERR_LOGIC, "no two-step kernel for this storage");
+            PLB_HIP_TRY(hipGetLastError());
+            return PLB_OK;
+        }
+    });
+    if (rc == PLB_OK) b->cur ^= 1;
+    return rc;
+}
+
 // Pull-scheme storage between steps is post-collision with the streaming of
 // the step pending (see fused_to_pre in fused.hip); the gather finishes it.
 int batch_to_pre(plb_batch* b) {
@@ -537,7 +636,13 @@ int batch_one_step(plb_batch* b, Launch&& launch) {
 
 int batch_step_plain(plb_batch* b, int nsteps) {
     for (int i = 0; i < nsteps; ++i) {
-        const int rc = batch_one_step(b, [&](int kind) { return batch_launch(b, 0, b->ntiles, true, kind); });
+        int rc;
+        if (i + 1 < nsteps && b->post && batch_two(b)) {
+            rc = batch_launch_two(b);
+            ++i;
+        } else {
+            rc = batch_one_step(b, [&](int kind) { return batch_launch(b, 0, b->ntiles, true, kind); });
+        }
         if (rc) return rc;
     }
     return PLB_OK;
@@ -597,6 +702,9 @@ int plb_batch_create(int q, int variant, int ndom, const plb_domain_desc* doms, 
     b->cur = 0;
     b->doms = nullptr;
     b->tiles = nullptr;
+    b->two_tiles = nullptr;
+    b->ntwo = 0;
+    b->two_off = false;
     b->grid = 0;
     b->map = 0;
     b->scheme = PLB_SCHEME_AUTO;
@@ -622,6 +730,10 @@ int plb_batch_create(int q, int variant, int ndom, const plb_domain_desc* doms, 
     if (rc) return bail(rc, plb_last_error());
     rc = variant == kF64 ? upload_doms<double>(b) : upload_doms<float>(b);
     if (rc) return bail(rc, plb_last_error());
+    int ncu = 0;
+    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || ncu <= 0) ncu = 256;
+    rc = two_step_plan(b, ncu);
+    if (rc) return bail(rc, plb_last_error());
     *out = b;
     return PLB_OK;
 }
@@ -631,7 +743,7 @@ int plb_batch_destroy(plb_batch* b) {
     (void)hipSetDevice(b->device);
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     if (b->graph) (void)hipGraphExecDestroy(b->graph);
-    void* ptrs[] = {b->buf[0], b->buf[1], b->doms, b->tiles};
+    void* ptrs[] = {b->buf[0], b->buf[1], b->doms, b->tiles, b->two_tiles};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -730,7 +842,16 @@ int plb_batch_step(plb_batch* b, int nsteps, int steps_per_graph) {
     if (reps > 0 && (!b->graph || b->graph_steps != steps_per_graph || b->graph_parity != b->cur)) {
         drop_batch_graph(b);
         PLB_HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-        const int lrc = batch_step_plain(b, steps_per_graph);
+        // two-step launches in a number that keeps the count of buffer swaps
+        // even (the graph must leave buf[cur] where it began)
+        int lrc = PLB_OK, left = steps_per_graph;
+        if (batch_two(b) && b->post && (steps_per_graph / 2) % 2 != 0) {
+            b->two_off = true;
+            lrc = batch_step_plain(b, 2);
+            b->two_off = false;
+            left -= 2;
+        }
+        if (lrc == PLB_OK) lrc = batch_step_plain(b, left);
         hipGraph_t g = nullptr;
         const hipError_t e = hipStreamEndCapture(b->stream, &g);
         if (lrc) {
@@ -785,6 +906,7 @@ int plb_batch_autotune(plb_batch* b, int steps, double* results, int max_results
     // every candidate runs an even number of steps (the total the caller sees
     // is even; the buffer parity is tracked in b->cur either way)
     const int even = steps + (steps & 1);
+    b->two_off = true;  // the tiling is that of the one-step launches
     for (int t : tiles) {
         for (int g : grids) {
           for (int m : {0, 1}) {
@@ -822,6 +944,7 @@ int plb_batch_autotune(plb_batch* b, int steps, double* results, int max_results
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
+    b->two_off = false;
     if (rc) return rc;
     if (nresults) *nresults = std::min(n, max_results);
     b->map = best_m;

@@ -1,0 +1,6 @@
+// The batched two-step kernels of D3Q27 (batch_two.hpp).
+#include "batch_two.hpp"
+
+namespace plb {
+PLB_BATCH2_INST_Q(27)
+}  // namespace plb

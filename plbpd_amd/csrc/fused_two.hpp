@@ -46,6 +46,10 @@ __device__ inline S* pop_elem(S* A, uint32_t k, uint32_t ps, uint32_t i) {
         return elem(A, k * ps + i);
 }
 
+// The arguments of one domain of a batch (batch_two.hpp).
+template <class T>
+struct BatchTileArgs;
+
 // Direction groups of the step t gathers: kAll, or, where the c_z = +1
 // directions are issued a plane ahead of the others, kUp (c_z = +1) and
 // kFlat (c_z = 0 and -1).
@@ -241,9 +245,18 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
     // Every thread loads, also past the grown tile (its wrapped coordinates
     // stay in the lattice; the values are not used): loads under a branch
     // made the compiler wait for loads in flight where the branches merge.
+    // A batch has no flags: its solid cells are the wall layers, known from
+    // the coordinates.
+    constexpr bool FLAGS = !std::is_same<Args, BatchTileArgs<T>>::value;
+    auto wall_cell = [&](uint32_t x, uint32_t y, uint32_t z) __attribute__((always_inline)) -> uint32_t {
+        return (a.bc.wall_lo[0] && x == 0) || (a.bc.wall_hi[0] && x + 1u == X) || (a.bc.wall_lo[1] && y == 0) ||
+               (a.bc.wall_hi[1] && y + 1u == Y) || (a.bc.wall_lo[2] && z == 0) || (a.bc.wall_hi[2] && z + 1u == Z);
+    };
     auto load_mask = [&](uint32_t n) __attribute__((always_inline)) -> uint32_t {
-        const I c = ((z0 + n + Z - 1u) % Z) * XY + gy * X + gx;
-        return NB ? nbmask[c] : (uint32_t)flags[c];
+        const uint32_t zn = (z0 + n + Z - 1u) % Z;
+        const I c = zn * XY + gy * X + gx;
+        if constexpr (!FLAGS) return wall_cell(gx, gy, zn);
+        else return NB ? nbmask[c] : (uint32_t)flags[c];
     };
     // the loads of plane n's directions of group G into fv
     auto fetch = [&](auto group, uint32_t n, S (&fv)[Q], uint32_t m) __attribute__((always_inline)) {
@@ -274,7 +287,11 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
         const uint32_t zo = z0 + n - 2u;
         const I c = zo * XY + py * X + px;
         const uint32_t pa = (n + 1u) % 3u, oa = (n + 2u) % 3u, b0 = (n + 1u) & 1u, c1 = n & 1u;
-        const uint32_t mo = mring[b0 * NI + li];
+        uint32_t mo;
+        if constexpr (FLAGS)
+            mo = mring[b0 * NI + li];
+        else
+            mo = wall_cell(px, py, zo);
         const bool self_solid = NB ? (mo & 1u) != 0 : mo != 0;
         if (!__all(self_solid)) {
             const Seams<I> sm = seams<I>(px, py, zo, a);
@@ -318,7 +335,7 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
             const uint32_t a3 = n % 3u, a2 = n & 1u;
             if (in_i) {
                 // the step t + 2 cells read this mask in the next iteration
-                mring[a2 * NI + tid] = mcur;
+                if (FLAGS) mring[a2 * NI + tid] = mcur;
                 const bool self_solid = NB ? (mcur & 1u) != 0 : mcur != 0;
                 if (!self_solid) step1(n, fv, a3, a2);
             }
@@ -347,7 +364,7 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
             S (&fc)[Q] = decltype(odd)::value ? fv1 : fv0;
             S (&fn)[Q] = decltype(odd)::value ? fv0 : fv1;
             const uint32_t a3 = n % 3u, a2 = n & 1u;
-            if (in_i) mring[a2 * NI + tid] = mc;
+            if (FLAGS && in_i) mring[a2 * NI + tid] = mc;
             const bool self_solid = NB ? (mc & 1u) != 0 : mc != 0;
             mc = load_mask(n + 2u);
             if (in_i && !self_solid) step1(n, fc, a3, a2);
