@@ -693,6 +693,10 @@ int plb_step(plb_state* s, int nsteps) {
             if ((rc = timed(s, PLB_STAGE_MOMENTS, [&] { return lit_moments(s, nullptr, nullptr); }))) return rc;
             if ((rc = timed(s, PLB_STAGE_RESET_VELOCITY, [&] { return lit_reset_velocity(s, bc); }))) return rc;
             if ((rc = timed(s, PLB_STAGE_RESET_DENSITY, [&] { return lit_reset_density(s, bc); }))) return rc;
+        } else if (i + 1 < nsteps && s->post_collision && fused_multi_steps(s) > 1) {
+            const int most = fused_multi_steps(s), n = nsteps - i < most ? nsteps - i : most;
+            if ((rc = timed(s, PLB_STAGE_FUSED, [&] { return fused_launch_multi(s, n); }))) return rc;
+            i += n - 1;
         } else if (i + 1 < nsteps && s->post_collision && fused_two_eligible(s)) {
             // two steps in one pass over the populations
             if ((rc = timed(s, PLB_STAGE_FUSED, [&] { return fused_launch_two(s); }))) return rc;
@@ -751,6 +755,17 @@ int plb_step_graph(plb_state* s, int nsteps, int steps_per_graph) {
             singles += 2;
         }
         int lrc = PLB_OK;
+        // D2Q9: an even number of launches of about equal step counts
+        const int most = !s->aa && s->post_collision ? fused_multi_steps(s) : 1;
+        if (most > 1) {
+            int launches = (steps_per_graph + most - 1) / most;
+            launches += launches & 1;
+            for (int i = 0; i < launches && lrc == PLB_OK; ++i) {
+                const int n = (singles + launches - i - 1) / (launches - i);
+                lrc = fused_launch_multi(s, n);
+                singles -= n;
+            }
+        }
         for (int i = 0; i < pairs && lrc == PLB_OK; ++i) lrc = fused_launch_two(s);
         for (int i = 0; i < singles && lrc == PLB_OK; ++i) lrc = fused_launch(s, true);
         hipGraph_t g = nullptr;

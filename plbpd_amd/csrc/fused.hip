@@ -670,7 +670,7 @@ int fused_initialize(plb_state* s, double rho0, const double u0[3], const plb_in
 
 namespace {
 
-enum KernelKind { kPush, kPull, kGather, kStreamOnly, kCollideOnly, kAaEven, kAaOdd, kAaGather, kPull2 };
+enum KernelKind { kPush, kPull, kGather, kStreamOnly, kCollideOnly, kAaEven, kAaOdd, kAaGather, kPull2, kMulti };
 
 // Chunks of a two-step launch along z, and the workgroup -> tile mapping.  A
 // workgroup holds a compute unit's LDS, so the launch runs in rounds of the
@@ -726,8 +726,18 @@ TwoGeom two_geom(const plb_state* s) {
     return g;
 }
 
+// Tile edge of a D2Q9 multi-step launch: 8 cells while those tiles find a
+// compute unit each, else 16, which computes fewer grown cells (8 steps of an
+// 8-cell tile 3.8 cells per output cell, of a 16-cell tile 2.2).  FP64, per
+// step, 8 / 16 cells: 100 x 25 1.26 / 1.63 us, 256 x 64 1.37 / 1.69, 301 x 97
+// 2.28 / 1.91, 512 x 256 6.0 / 3.6.
+int multi_tile(const plb_state* s) {
+    const uint64_t tiles = (uint64_t)((s->X + 7) / 8) * ((s->Z + 7) / 8) * s->Y;
+    return tiles <= (uint64_t)s->num_cu ? 8 : 16;
+}
+
 // Launch geometry and arguments shared by every fused-layout kernel.
-int launch_kind(plb_state* s, KernelKind kind) {
+int launch_kind(plb_state* s, KernelKind kind, int steps = 1) {
     if (!s->bc_set) return fail(PLB_ERR_LOGIC, "fused step before the boundary was set");
     // the row pull kernel (fused_row.hpp) takes rows of 64 * vec * wpr cells
     // (kRowShapes).  Automatic choice, from measurement on MI355X (256^3
@@ -842,6 +852,13 @@ int launch_kind(plb_state* s, KernelKind kind) {
                                             s->stream))
                         return fail(PLB_ERR_LOGIC, "no two-step kernel for this storage");
                 }
+                break;
+            case kMulti:
+                if constexpr (Q == 9)
+                    launch_multi9<V>(a, (uint32_t)steps, multi_tile(s), nb, a.bc.moving != 0, A, B, s->nbmask,
+                                     s->stream);
+                else
+                    return fail(PLB_ERR_LOGIC, "the multi-step kernel is for D2Q9");
                 break;
             case kPull:
                 if (vec) {
@@ -991,6 +1008,31 @@ int fused_launch_two(plb_state* s) {
     if (!s->post_collision || !fused_two_eligible(s))
         return fail(PLB_ERR_LOGIC, "two-step launch needs an eligible state in post-collision form");
     const int rc = launch_kind(s, kPull2);
+    s->moments_valid = false;
+    return rc;
+}
+
+// Steps per launch of a D2Q9 lattice.  Up to 2^22 cells a launch of several
+// steps measured faster than one launch per step (per step, one against
+// several): FP64 100 x 25 3.4 -> 1.3 us, 256 x 64 5.2 -> 1.4, 512 x 256 7.5 ->
+// 3.6, 1024 x 1024 31 -> 23, 2048 x 2048 113 -> 91; FP32-shifted 256 x 64 4.5 ->
+// 1.2, 1024 x 512 9.6 -> 7.7, 2048 x 2048 59 -> 58.  Above 2^18 cells, where
+// memory and not the launch is what a step waits for, FP32 arithmetic takes 4
+// steps, which recompute less (1024 x 512: 8.8 us with 8).
+int fused_multi_steps(const plb_state* s) {
+    if (s->q != 9 || s->tune_two == 0 || s->tune_index64 || s->aa || !fused_uses_pull(s) ||
+        s->mode != PLB_MODE_FUSED)
+        return 1;
+    const uint64_t cells = (uint64_t)s->X * (uint64_t)s->Y * (uint64_t)s->Z;
+    if (cells > (1ull << 22)) return 1;
+    if ((uint64_t)s->q * s->pstride * s->sbytes > 0xffffffffull) return 1;
+    return cells > (1ull << 18) && s->variant != kF64 ? 4 : kMultiSteps;
+}
+
+int fused_launch_multi(plb_state* s, int steps) {
+    if (!s->post_collision || steps < 1 || steps > fused_multi_steps(s))
+        return fail(PLB_ERR_LOGIC, "multi-step launch needs an eligible state in post-collision form");
+    const int rc = launch_kind(s, kMulti, steps);
     s->moments_valid = false;
     return rc;
 }

@@ -510,4 +510,12 @@ bool launch_pull2(const FusedArgs<typename Prec<V>::T>& a, const TwoGeom& g, boo
                   const typename Prec<V>::S* A, typename Prec<V>::S* B, const uint8_t* flags,
                   const uint32_t* nbmask, hipStream_t stream);
 
+// Up to kMultiSteps pull steps of a D2Q9 lattice in one launch
+// (fused_multi.hpp), in tiles of tile x tile cells (8 or 16).
+constexpr int kMultiSteps = 8;
+template <int V>
+void launch_multi9(const FusedArgs<typename Prec<V>::T>& a, uint32_t steps, int tile, bool nb, bool mov,
+                   const typename Prec<V>::S* A, typename Prec<V>::S* B, const uint32_t* nbmask,
+                   hipStream_t stream);
+
 }  // namespace plb

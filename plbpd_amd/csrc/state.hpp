@@ -141,6 +141,10 @@ int fused_flush_deferred(plb_state* s);
 // The two-step tile width for the state (32 or 64 cells), or 0 where none applies.
 int fused_two_tile_x(const plb_state* s);
 int fused_launch_two(plb_state* s);
+// D2Q9: the steps one launch can take (1: one step per launch), and that launch
+// from post-collision storage.
+int fused_multi_steps(const plb_state* s);
+int fused_launch_multi(plb_state* s, int steps);
 
 // literal mode (literal.hip)
 int lit_initialize(plb_state* s, double rho0, const double u0[3], const plb_init_spec* init,
