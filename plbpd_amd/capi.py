@@ -454,8 +454,8 @@ class Batch:
 
     def moments(self, d):
         dm = self.domains[d]
-        rho = np.zeros((dm["z"], dm["y"], dm["x"]), np.float64)
-        u = np.zeros((dm["z"], dm["y"], dm["x"], 3), np.float64)
+        rho = np.empty((dm["z"], dm["y"], dm["x"]), np.float64)
+        u = np.empty((dm["z"], dm["y"], dm["x"], 3), np.float64)
         check(lib().plb_batch_download_moments(self.h, int(d), _p(rho), _p(u)))
         return rho, u
 

@@ -25,6 +25,7 @@
 #include "batch.hpp"
 #include "bgk.hpp"
 #include "fused_kernels.hpp"
+#include "host_read.hpp"
 
 struct plb_batch;
 
@@ -307,37 +308,68 @@ __global__ void k_batch_init(typename Prec<V>::S* __restrict__ f, const BDom<typ
     }
 }
 
-// rho (N) and u (3N, AoS) of one domain, double; walls report rho_s, u_b.
-template <int Q, int V>
-__global__ void k_batch_moments(const typename Prec<V>::S* __restrict__ f, BDom<typename Prec<V>::T> D,
-                                FusedBC<double> bc, double rho_s, double* __restrict__ rho,
-                                double* __restrict__ u) {
+// rho and u (AoS) of the cells [first, first + count) of one domain, double,
+// to out (count rho, then 3 count u); walls report rho_s, u_b.  PEND: between
+// pull steps a cell's populations wait where the next step would gather them
+// (batch_pull_cell), and are read from there.  out is host memory: the three
+// components of a block's cells go through LDS, so that every store is a whole
+// run of lines.
+template <int Q, int V, bool PEND>
+__global__ __launch_bounds__(kMaxBlock) void k_batch_moments(const typename Prec<V>::S* __restrict__ f,
+                                                             BDom<typename Prec<V>::T> D, FusedBC<double> bc,
+                                                             double rho_s, uint32_t first, uint32_t count,
+                                                             double* __restrict__ out) {
     using P = Prec<V>;
     using T = typename P::T;
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= D.N) return;
-    const uint32_t x = c % D.X, y = (c / D.X) % D.Y, z = c / (D.X * D.Y);
-    int face = -1;
-    const bool on[6] = {bc.wall_hi[0] && x == D.X - 1, bc.wall_lo[0] && x == 0, bc.wall_hi[1] && y == D.Y - 1,
-                        bc.wall_lo[1] && y == 0, bc.wall_hi[2] && z == D.Z - 1, bc.wall_lo[2] && z == 0};
-    for (int fc = 0; fc < 6; ++fc)
-        if (on[fc]) face = fc;
-    if (face >= 0) {
-        rho[c] = rho_s;
-        for (int i = 0; i < 3; ++i) u[3 * (uint64_t)c + i] = bc.vel[1 + face][i];
-        return;
-    }
-    T fl[Q];
+    __shared__ double su[3 * kMaxBlock];
+    const uint32_t b0 = blockIdx.x * kMaxBlock, i = b0 + threadIdx.x;
+    if (i < count) {
+        const uint32_t c = first + i;
+        uint32_t x, y, z;
+        cell_xyz(D, c, x, y, z);
+        int face = -1;
+        const bool on[6] = {bc.wall_hi[0] && x == D.X - 1, bc.wall_lo[0] && x == 0, bc.wall_hi[1] && y == D.Y - 1,
+                            bc.wall_lo[1] && y == 0, bc.wall_hi[2] && z == D.Z - 1, bc.wall_lo[2] && z == 0};
+        for (int fc = 0; fc < 6; ++fc)
+            if (on[fc]) face = fc;
+        double rd = rho_s, ud[3];
+        if (face >= 0) {
+            for (int d = 0; d < 3; ++d) ud[d] = bc.vel[1 + face][d];
+        } else {
+            const typename P::S* a = f + D.off;
+            const uint32_t xo[3] = {x == 0 ? D.X - 1 : x - 1, x, x + 1 == D.X ? 0 : x + 1};
+            const uint32_t yo[3] = {y == 0 ? D.Y - 1 : y - 1, y, y + 1 == D.Y ? 0 : y + 1};
+            const uint32_t zo[3] = {z == 0 ? D.Z - 1 : z - 1, z, z + 1 == D.Z ? 0 : z + 1};
+            const bool wx[3] = {bc.wall_lo[0] && xo[0] == 0, false, bc.wall_hi[0] && xo[2] == D.X - 1};
+            const bool wy[3] = {bc.wall_lo[1] && yo[0] == 0, false, bc.wall_hi[1] && yo[2] == D.Y - 1};
+            const bool wz[3] = {bc.wall_lo[2] && zo[0] == 0, false, bc.wall_hi[2] && zo[2] == D.Z - 1};
+            T fl[Q];
 #pragma unroll
-    for (int k = 0; k < Q; ++k) fl[k] = P::load(f[D.off + (uint64_t)k * D.ps + c]);
-    T r, j0, j1, j2;
-    moment_sums<Q, T>(fl, r, j0, j1, j2);
-    if (P::shifted) r = (T)1 + r;
-    const T ri = (T)1 / r;
-    rho[c] = (double)r;
-    u[3 * (uint64_t)c] = (double)(j0 * ri);
-    u[3 * (uint64_t)c + 1] = (double)(j1 * ri);
-    u[3 * (uint64_t)c + 2] = (double)(j2 * ri);
+            for (int k = 0; k < Q; ++k) {
+                uint64_t src = (uint64_t)k * D.ps + c;
+                if (PEND) {
+                    const int cx = Lat<Q>::cx(k), cy = Lat<Q>::cy(k), cz = Lat<Q>::cz(k);
+                    const bool bb = wx[1 - cx] || wy[1 - cy] || wz[1 - cz];
+                    const uint32_t s = (zo[1 - cz] * D.Y + yo[1 - cy]) * D.X + xo[1 - cx];
+                    src = bb ? (uint64_t)rev<Q>(k) * D.ps + c : (uint64_t)k * D.ps + s;
+                }
+                fl[k] = P::load(a[src]);
+            }
+            T r, j0, j1, j2;
+            moment_sums<Q, T>(fl, r, j0, j1, j2);
+            if (P::shifted) r = (T)1 + r;
+            const T ri = (T)1 / r;
+            rd = (double)r;
+            ud[0] = (double)(j0 * ri);
+            ud[1] = (double)(j1 * ri);
+            ud[2] = (double)(j2 * ri);
+        }
+        out[i] = rd;
+        for (int d = 0; d < 3; ++d) su[3 * threadIdx.x + d] = ud[d];
+    }
+    __syncthreads();
+    const uint32_t n3 = 3u * (count - b0 < (uint32_t)kMaxBlock ? count - b0 : (uint32_t)kMaxBlock);
+    for (uint32_t t = threadIdx.x; t < n3; t += kMaxBlock) out[count + 3u * b0 + t] = su[t];
 }
 
 template <class Fn>
@@ -390,6 +422,7 @@ struct plb_batch {
     hipGraphExec_t graph;
     int graph_steps, graph_parity;
     uint64_t total_cells, fluid_cells;
+    plb::HostRing ring;  // pinned pieces of downloads
 };
 
 namespace plb {
@@ -746,6 +779,7 @@ int plb_batch_destroy(plb_batch* b) {
     void* ptrs[] = {b->buf[0], b->buf[1], b->doms, b->tiles, b->two_tiles};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    host_ring_free(&b->ring);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
     return PLB_OK;
@@ -954,14 +988,10 @@ int plb_batch_autotune(plb_batch* b, int steps, double* results, int max_results
 int plb_batch_download_moments(plb_batch* b, int d, double* rho, double* u) {
     if (!b || !rho || !u || d < 0 || d >= b->ndom) return fail(PLB_ERR_INVALID_ARGUMENT, "bad arguments");
     PLB_HIP_TRY(hipSetDevice(b->device));
-    const int prc = batch_to_pre(b);
-    if (prc) return prc;
     const uint64_t n = (uint64_t)b->desc[d].x * b->desc[d].y * b->desc[d].z;
-    double* dev = nullptr;
-    PLB_HIP_TRY(hipMalloc(&dev, n * 4 * sizeof(double)));
     FusedBC<double> bc;
     make_fused_bc<double>(b->bc, b->q, &bc);
-    int rc = with_qv_b(b->q, b->variant, [&](auto qc, auto vc) {
+    return with_qv_b(b->q, b->variant, [&](auto qc, auto vc) {
         constexpr int Q = decltype(qc)::value;
         constexpr int V = decltype(vc)::value;
         using P = Prec<V>;
@@ -971,24 +1001,30 @@ int plb_batch_download_moments(plb_batch* b, int d, double* rho, double* u) {
         D.Y = b->desc[d].y;
         D.Z = b->desc[d].z;
         D.N = (uint32_t)n;
+        D.dX = make_fastdiv(D.X);
+        D.dY = make_fastdiv(D.Y);
         D.off = b->off[d];
         D.ps = b->ps[d];
         D.tau = D.om = D.omm = D.F0 = D.F1 = D.F2 = (T)0;
-        hipLaunchKernelGGL((k_batch_moments<Q, V>), dim3(blocks_for(n, 256)), dim3(256), 0, b->stream,
-                           (const typename P::S*)b->buf[b->cur], D, bc, b->bc.rho_s, dev, dev + n);
-        PLB_HIP_TRY(hipGetLastError());
-        return PLB_OK;
+        const typename P::S* f = (const typename P::S*)b->buf[b->cur];
+        return host_read(
+            &b->ring, b->device, b->stream, n, 4 * sizeof(double),
+            [&](uint64_t first, uint64_t count, void* slot) {
+                const dim3 grid(blocks_for(count, kMaxBlock)), block(kMaxBlock);
+                if (b->post)
+                    hipLaunchKernelGGL((k_batch_moments<Q, V, true>), grid, block, 0, b->stream, f, D, bc,
+                                       b->bc.rho_s, (uint32_t)first, (uint32_t)count, (double*)slot);
+                else
+                    hipLaunchKernelGGL((k_batch_moments<Q, V, false>), grid, block, 0, b->stream, f, D, bc,
+                                       b->bc.rho_s, (uint32_t)first, (uint32_t)count, (double*)slot);
+                return hipGetLastError();
+            },
+            [&](uint64_t first, uint64_t count, const void* slot) {
+                const double* from = (const double*)slot;
+                std::memcpy(rho + first, from, count * sizeof(double));
+                std::memcpy(u + 3 * first, from + count, 3 * count * sizeof(double));
+            });
     });
-    hipError_t e = hipSuccess;
-    if (rc == PLB_OK) e = hipMemcpyAsync(rho, dev, n * sizeof(double), hipMemcpyDeviceToHost, b->stream);
-    if (rc == PLB_OK && e == hipSuccess)
-        e = hipMemcpyAsync(u, dev + n, 3 * n * sizeof(double), hipMemcpyDeviceToHost, b->stream);
-    const hipError_t e2 = hipStreamSynchronize(b->stream);
-    (void)hipFree(dev);
-    if (rc) return rc;
-    if (e != hipSuccess) return fail(PLB_ERR_HIP, hipGetErrorString(e));
-    if (e2 != hipSuccess) return fail(PLB_ERR_HIP, hipGetErrorString(e2));
-    return PLB_OK;
 }
 
 int plb_batch_cells(const plb_batch* b, uint64_t* total_cells, uint64_t* fluid_cells) {

@@ -5,6 +5,7 @@
 #include <string>
 #include <vector>
 
+#include "host_read.hpp"
 #include "state.hpp"
 
 namespace plb {
@@ -288,6 +289,7 @@ int plb_state_create(const plb_state_desc* d, plb_state** out) {
     s->moments_valid = false;
     s->scratch = nullptr;
     s->scratch_bytes = 0;
+    s->ring = new HostRing();
     s->graph = nullptr;
     s->graph_steps = 0;
     s->graph_parity = 0;
@@ -340,6 +342,7 @@ int plb_state_create(const plb_state_desc* d, plb_state** out) {
     };
     hipError_t e = hipStreamCreate(&s->stream);
     if (e != hipSuccess) {
+        delete s->ring;
         delete s;
         return fail(PLB_ERR_HIP, hipGetErrorString(e));
     }
@@ -376,6 +379,8 @@ int plb_state_destroy(plb_state* s) {
     void* ptrs[] = {s->buf[0], s->buf[1], s->rho, s->u, s->flags, s->nbmask, s->scratch};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    host_ring_free(s->ring);
+    delete s->ring;
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
     return PLB_OK;

@@ -10,6 +10,7 @@
 #include <string>
 #include <type_traits>
 
+#include "host_read.hpp"
 #include "state.hpp"
 
 namespace plb {
@@ -509,11 +510,11 @@ __global__ void k_moments_collide_push(LitDims g, R* __restrict__ n, R* __restri
     }
 }
 
-// Host AoS <-> device SoA with dtype conversion.  compact: host cells are
-// interior only (X*Y*Z); otherwise the full halo'd array.
+// Upload: host AoS -> device SoA with dtype conversion.  compact: host cells
+// are interior only (X*Y*Z); otherwise the full halo'd array.
 template <class H, class R>
-__global__ void k_transfer(LitDims g, H* __restrict__ host, R* __restrict__ dev, int vlen,
-                           int compact, int upload, uint64_t total) {
+__global__ void k_upload(LitDims g, const H* __restrict__ host, R* __restrict__ dev, int vlen, int compact,
+                         uint64_t total) {
     for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
          t += (uint64_t)gridDim.x * blockDim.x) {
         const int v = (int)(t % vlen);
@@ -523,12 +524,28 @@ __global__ void k_transfer(LitDims g, H* __restrict__ host, R* __restrict__ dev,
             const int x = (int)(hc % g.X), y = (int)((hc / g.X) % g.Y), z = (int)(hc / ((uint64_t)g.X * g.Y));
             c = g.cell(z + 1, y + 1, x + 1);
         }
-        if (upload)
-            dev[v * g.ncell + c] = (R)host[t];
-        else
-            host[t] = (H)dev[v * g.ncell + c];
+        dev[v * g.ncell + c] = (R)host[t];
     }
 }
+
+// Download: value v of cell c of the full halo'd array, or of the interior.
+template <class R>
+struct GetFull {
+    const R* dev;
+    uint64_t ncell;
+    __device__ R operator()(uint64_t c, uint32_t v) const { return dev[v * ncell + c]; }
+};
+template <class R>
+struct GetInterior {
+    const R* dev;
+    LitDims g;
+    FastDiv dX, dY;  // an interior of 2^32 cells is part of a state larger than any device
+    __device__ R operator()(uint64_t c, uint32_t v) const {
+        const uint32_t row = fdiv((uint32_t)c, dX), z = fdiv(row, dY);
+        const int x = (int)((uint32_t)c - row * dX.d), y = (int)(row - z * dY.d);
+        return dev[v * g.ncell + g.cell((int)z + 1, y + 1, x + 1)];
+    }
+};
 
 // FP64 sums over interior cells of rho and rho*u (two deterministic passes).
 template <class R>
@@ -871,37 +888,52 @@ int lit_transfer(plb_state* s, int field, int layout, int dtype, void* host, boo
     const int compact = layout == PLB_LAYOUT_COMPACT;
     const uint64_t cells = compact ? (uint64_t)s->X * s->Y * s->Z : s->ncell;
     const uint64_t total = cells * vlen;
+    if (!upload) {
+        return with_qr(s, [&](auto, auto rr) {
+            using R = decltype(rr);
+            auto read = [&](auto hh) {
+                using H = decltype(hh);
+                const size_t cell_bytes = vlen * sizeof(H);
+                const GetInterior<R> gi{(const R*)dev, g, make_fastdiv((uint32_t)s->X), make_fastdiv((uint32_t)s->Y)};
+                const GetFull<R> gf{(const R*)dev, g.ncell};
+                return host_read(
+                    s->ring, s->device, s->stream, cells, cell_bytes,
+                    [&](uint64_t first, uint64_t n, void* slot) {
+                        return compact ? host_fill<H>(gi, first, n, vlen, slot, s->stream)
+                                       : host_fill<H>(gf, first, n, vlen, slot, s->stream);
+                    },
+                    [&](uint64_t first, uint64_t n, const void* slot) {
+                        std::memcpy((char*)host + first * cell_bytes, slot, n * cell_bytes);
+                    });
+            };
+            return dtype == PLB_DTYPE_F64 ? read(double()) : read(float());
+        });
+    }
     const size_t hbytes = total * (dtype == PLB_DTYPE_F64 ? 8 : 4);
     void* stage = nullptr;
     PLB_HIP_TRY(hipMalloc(&stage, hbytes));
     int rc = PLB_OK;
-    if (upload) {
-        hipError_t e = hipMemcpyAsync(stage, host, hbytes, hipMemcpyHostToDevice, s->stream);
-        if (e != hipSuccess) rc = fail(PLB_ERR_HIP, std::string("upload: ") + hipGetErrorString(e));
-    }
+    hipError_t e = hipMemcpyAsync(stage, host, hbytes, hipMemcpyHostToDevice, s->stream);
+    if (e != hipSuccess) rc = fail(PLB_ERR_HIP, std::string("upload: ") + hipGetErrorString(e));
     if (rc == PLB_OK) {
         rc = with_qr(s, [&](auto, auto rr) {
             using R = decltype(rr);
             if (dtype == PLB_DTYPE_F64)
-                hipLaunchKernelGGL((k_transfer<double, R>), dim3(stride_blocks(total, kThreads)),
-                                   dim3(kThreads), 0, s->stream, g, (double*)stage, (R*)dev, vlen,
-                                   compact, upload ? 1 : 0, total);
+                hipLaunchKernelGGL((k_upload<double, R>), dim3(stride_blocks(total, kThreads)),
+                                   dim3(kThreads), 0, s->stream, g, (const double*)stage, (R*)dev, vlen,
+                                   compact, total);
             else
-                hipLaunchKernelGGL((k_transfer<float, R>), dim3(stride_blocks(total, kThreads)),
-                                   dim3(kThreads), 0, s->stream, g, (float*)stage, (R*)dev, vlen,
-                                   compact, upload ? 1 : 0, total);
+                hipLaunchKernelGGL((k_upload<float, R>), dim3(stride_blocks(total, kThreads)),
+                                   dim3(kThreads), 0, s->stream, g, (const float*)stage, (R*)dev, vlen,
+                                   compact, total);
             PLB_HIP_TRY(hipGetLastError());
             return PLB_OK;
         });
     }
-    if (rc == PLB_OK && !upload) {
-        hipError_t e = hipMemcpyAsync(host, stage, hbytes, hipMemcpyDeviceToHost, s->stream);
-        if (e != hipSuccess) rc = fail(PLB_ERR_HIP, std::string("download: ") + hipGetErrorString(e));
-    }
-    hipError_t e = hipStreamSynchronize(s->stream);
+    e = hipStreamSynchronize(s->stream);
     (void)hipFree(stage);
     if (rc == PLB_OK && e != hipSuccess) rc = fail(PLB_ERR_HIP, hipGetErrorString(e));
-    if (rc == PLB_OK && upload && field == PLB_FIELD_NTMP) s->lit_ntmp_folded = false;
+    if (rc == PLB_OK && field == PLB_FIELD_NTMP) s->lit_ntmp_folded = false;
     return rc;
 }
 

@@ -56,6 +56,8 @@ struct LitOp {
     plb_boundary bc;   // the periodic copies, the resets
 };
 
+struct HostRing;
+
 }  // namespace plb
 
 struct plb_state {
@@ -93,6 +95,7 @@ struct plb_state {
     bool moments_valid;
     void* scratch;  // reductions
     size_t scratch_bytes;
+    plb::HostRing* ring;  // pinned pieces of downloads (host_read.hpp)
     hipStream_t stream;
     // graph of a fixed number of fused steps
     hipGraphExec_t graph;
