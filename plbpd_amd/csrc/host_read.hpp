@@ -21,9 +21,9 @@
 
 namespace plb {
 
-// The pinned pieces of one state or batch: allocated by its first read (in the
-// size that read needs, and again for a larger one: at most 12 MB), freed with
-// it.  Two pieces per thread: one being written, one being read.
+// The pinned pieces of one state or batch: allocated by its first read (for
+// that read and for the velocities of as many cells, and again for a larger
+// one: at most 12 MB), freed with it.  Two pieces per thread: one being written, one being read.
 struct HostRing {
     static constexpr int kThreads = 3;
     static constexpr int kSlots = 2 * kThreads;
@@ -73,7 +73,10 @@ int host_read(HostRing* r, int device, hipStream_t stream, uint64_t items, size_
     const uint64_t most = HostRing::kSlotBytes / item_bytes, least = std::max<uint64_t>(1, std::min<uint64_t>(most, (128u << 10) / item_bytes));
     const uint64_t piece = std::max(least, std::min(most, (items + 7) / 8));
     const uint64_t pieces = (items + piece - 1) / piece;
-    const int rc = host_ring_ensure(r, piece * item_bytes);
+    // not once for a density and again for the velocities (24 bytes a cell)
+    // that are read after it: setting pinned memory up again costs 2 ms
+    const size_t velocities = (size_t)std::min<uint64_t>((items + 7) / 8, HostRing::kSlotBytes / 24) * 24;
+    const int rc = host_ring_ensure(r, std::max<size_t>(piece * item_bytes, velocities));
     if (rc) return rc;
     const size_t slot_bytes = r->slot_bytes;
     std::atomic<uint64_t> next{0};
