@@ -470,7 +470,7 @@ int two_step_plan(plb_batch* b, int ncu) {
     int zmax = 1;
     for (int d = 0; d < b->ndom; ++d) {
         // 32-bit byte offsets within a domain
-        if ((uint64_t)b->q * b->ps[d] * sb > 0xffffffffull) return PLB_OK;
+        if ((uint64_t)b->q * b->ps[d] * sb > kMaxBuffer) return PLB_OK;
         shape[d] = two_shape(b->q, sb, b->desc[d].x, b->desc[d].y);
         zmax = std::max(zmax, b->desc[d].z);
     }

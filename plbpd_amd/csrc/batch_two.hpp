@@ -20,7 +20,6 @@ struct BatchTileArgs {
     T tau, om, omm, F0, F1, F2;
     const FusedBC<T>& bc;
     const T (&wcub)[27][3];
-    int32_t nt_store;
 };
 
 template <class T>
@@ -30,15 +29,15 @@ struct BatchWalls {
 };
 
 template <int Q, int V, bool MOV>
-__global__ __launch_bounds__(pull2_threads(Q, (int)sizeof(typename Prec<V>::S), 0, 0), 1) void k_batch2(
+__global__ __launch_bounds__(two_threads(Q, (int)sizeof(typename Prec<V>::S)), 1) void k_batch2(
     const typename Prec<V>::S* __restrict__ A, typename Prec<V>::S* __restrict__ B,
     const BDom<typename Prec<V>::T>* __restrict__ doms, const BTile* __restrict__ tiles,
     BatchWalls<typename Prec<V>::T> w) {
     using T = typename Prec<V>::T;
     const BTile t = tiles[blockIdx.x];
     const BDom<T> D = doms[t.dom];
-    const BatchTileArgs<T> a{D.X, D.Y, D.Z, D.ps, D.tau, D.om, D.omm, D.F0, D.F1, D.F2, w.bc, w.wcub, 0};
-    pull2_tile<Q, V, 0, MOV, 0, 0, false, two_split(Q, (int)sizeof(typename Prec<V>::S), false)>(
+    const BatchTileArgs<T> a{D.X, D.Y, D.Z, D.ps, D.tau, D.om, D.omm, D.F0, D.F1, D.F2, w.bc, w.wcub};
+    pull2_tile<Q, V, 0, MOV, 1, two_split(Q, (int)sizeof(typename Prec<V>::S), false)>(
         A + D.off, B + D.off, nullptr, nullptr, a, t.bx, t.by, t.x0, t.y0, t.z0, t.zc);
 }
 
@@ -51,7 +50,7 @@ bool launch_batch2(const typename Prec<V>::S* A, typename Prec<V>::S* B, const B
     BatchWalls<T> w;
     w.bc = bc;
     fill_wall_cub<Q, T>(bc, w.wcub);
-    const dim3 grid(ntiles), block(pull2_threads(Q, (int)sizeof(typename Prec<V>::S), 0, 0));
+    const dim3 grid(ntiles), block(two_threads(Q, (int)sizeof(typename Prec<V>::S)));
     if (bc.moving)
         hipLaunchKernelGGL((k_batch2<Q, V, true>), grid, block, 0, stream, A, B, doms, tiles, w);
     else

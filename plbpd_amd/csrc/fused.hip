@@ -712,18 +712,17 @@ enum KernelKind { kPush, kPull, kGather, kStreamOnly, kCollideOnly, kAaEven, kAa
 // L2.  The runs hold kx = ceil(pairs / 8) pairs (the last may be shorter),
 // so the rounds are counted per XCD.
 TwoGeom two_geom(const plb_state* s) {
-    // rows of whole 64- or 32-cell tiles: the compiled shapes; other rows: the
-    // shape that two_shape finds
+    // rows of whole 64- or 32-cell tiles take those; other rows the shape that
+    // two_shape found
     TwoGeom g;
     int bx = fused_two_tile_x(s), by;
-    g.any = bx == 0;
-    if (g.any)
+    if (bx == 0)
         bx = s->two_any_bx, by = s->two_any_by;
     else
         by = two_rows(s->q, (int)s->sbytes, bx);
     g.bx = (uint32_t)bx;
     g.by = (uint32_t)by;
-    g.wide = (s->tune_index64 || (uint64_t)s->q * s->pstride * s->sbytes > 0xffffffffull) ? 1u : 0u;
+    g.buffers = two_buffers(s->q, (uint64_t)s->pstride * s->sbytes, s->tune_index64 ? 2 : 1);
     g.ntx = ((uint32_t)s->X + (uint32_t)bx - 1u) / (uint32_t)bx;
     g.nty = ((uint32_t)s->Y + (uint32_t)by - 1u) / (uint32_t)by;
     const uint64_t ntx = g.ntx, nty = g.nty, Z = (uint64_t)s->Z;
@@ -1021,7 +1020,7 @@ bool fused_two_eligible(const plb_state* s) {
     if (s->tune_two == 0 || s->aa || !fused_uses_pull(s) || s->mode != PLB_MODE_FUSED) return false;
     if (s->q != 19 && s->q != 27) return false;
     // offsets within one population array are 32-bit
-    if ((uint64_t)s->pstride * s->sbytes > 0xffffffffull) return false;
+    if ((uint64_t)s->pstride * s->sbytes > kMaxBuffer) return false;
     const uint64_t cells = (uint64_t)s->X * (uint64_t)s->Y * (uint64_t)s->Z;
     if (fused_two_tile_x(s) == 0) {
         // Rows that are no whole number of 32-cell tiles run in tiles of
@@ -1075,7 +1074,7 @@ int fused_multi_steps(const plb_state* s) {
         return 1;
     const uint64_t cells = (uint64_t)s->X * (uint64_t)s->Y * (uint64_t)s->Z;
     if (cells > (1ull << 22)) return 1;
-    if ((uint64_t)s->q * s->pstride * s->sbytes > 0xffffffffull) return 1;
+    if ((uint64_t)s->q * s->pstride * s->sbytes > kMaxBuffer) return 1;
     return cells > (1ull << 18) && s->variant != kF64 ? 4 : kMultiSteps;
 }
 

@@ -374,6 +374,34 @@ bool launch_pull_row(const FusedArgs<typename Prec<V>::T>& a, int vec, bool nts,
                      const typename Prec<V>::S* A, typename Prec<V>::S* B, const uint8_t* flags,
                      const uint32_t* nbmask, unsigned nblocks, hipStream_t stream);
 
+// Largest buffer (bytes) whose accesses the two-step and multi-step kernels
+// address by 32-bit offsets; the offsets past it mark lanes that do not store.
+constexpr uint64_t kMaxBuffer = 0xfffffff0ull;
+
+// The populations of buffer g of W: whole pairs of opposite directions, the
+// rest direction with the first.
+__host__ __device__ constexpr int two_group(int q, int w, int k) {
+    return w <= 1 || k == 0 ? 0 : (k - 1) / 2 * w / ((q - 1) / 2);
+}
+__host__ __device__ constexpr int two_group_first(int q, int w, int g) {
+    if (g == 0) return 0;
+    for (int k = 1; k < q; ++k)
+        if (two_group(q, w, k) >= g) return k;
+    return q;
+}
+// The buffers that arrays of `pop` bytes per population take, from `least` on.
+inline uint32_t two_buffers(int q, uint64_t pop, int least) {
+    for (int w = least; w <= 4; w *= 2) {
+        int most = 0;
+        for (int g = 0; g < w; ++g) {
+            const int n = two_group_first(q, w, g + 1) - two_group_first(q, w, g);
+            most = n > most ? n : most;
+        }
+        if ((uint64_t)most * pop <= kMaxBuffer) return (uint32_t)w;
+    }
+    return 0;
+}
+
 // Tiles of a two-step launch: ntx x nty tiles of bx x BY cells in every
 // chunk of zc planes, nzc chunks; xcd = 1 gives XCD j the j-th of eight runs
 // of kx (z-chunk, y-tile) pairs, so that tiles sharing their grown borders
@@ -384,8 +412,7 @@ struct TwoGeom {
     uint32_t kx;
     uint32_t bx;    // tile width (one workgroup per compute unit whatever the shape)
     uint32_t by;    // tile rows
-    uint32_t any;   // 1: a tile shape outside the compiled 64- and 32-cell ones (two_cap)
-    uint32_t wide;  // population arrays beyond 4 GiB: per-population base pointers
+    uint32_t buffers;  // buffers of up to 4 GiB that hold the array: 1, 2, 4, or 0 (pointers)
 };
 // Workgroups of a two-step launch (with the XCD mapping, eight runs of kx
 // pairs; the workgroups past the last pair return at once).
@@ -432,9 +459,8 @@ __host__ __device__ constexpr int zring_planes(int q) {
     return q == 19 ? ZRing<19>::planes() : (q == 27 ? ZRing<27>::planes() : (q == 9 ? ZRing<9>::planes() : 0));
 }
 
-// Cells of a grown tile, and threads of its workgroup (one cell each).
+// Cells of a grown tile.
 __host__ __device__ constexpr int two_cells(int bx, int by) { return (bx + 2) * (by + 2); }
-__host__ __device__ constexpr int two_threads(int bx, int by) { return (two_cells(bx, by) + 63) / 64 * 64; }
 // Whether the two-step kernel issues the step t gathers of the c_z = +1
 // directions an iteration earlier than the others (fused_two.hpp): D3Q19
 // with 4-byte storage, and with 8-byte storage around interior solids (nb).
@@ -446,19 +472,35 @@ __host__ __device__ constexpr bool two_split(int q, int sbytes, bool nb) {
     return q == 19 && (sbytes == 4 || (sbytes == 8 && nb));
 }
 
-// Rows per tile for a lattice, a storage width and a tile width: the largest
-// BY whose ring ((bx + 2) x (BY + 2) cells x (zring_planes(q) population
-// planes + two 4-byte mask planes)) fits the LDS of a compute unit (160 KiB
-// on gfx950; a workgroup takes all of it), within 1024 threads; 0 where no
-// BY >= 3 fits.  The split kernel with 4-byte storage takes at most 704
-// cells: 64 x 9 tiles (768 threads) ran slower than 64 x 8, and so did
+// Cells that a grown tile of any shape may have: the ring of that many cells
+// (zring_planes(q) population planes and two 4-byte mask planes) fits the LDS
+// of a compute unit (160 KiB on gfx950; a workgroup takes all of it), within
+// 1024 threads, one per cell.  The split kernel with 4-byte storage takes at
+// most 704 cells: 64 x 9 tiles (768 threads) ran slower than 64 x 8, and so did
 // 64 x 11 (858 threads in 128 VGPRs: D3Q19 256^3 FP32-shifted 356 / 307
 // against 341 / 288 us per step with solids / walls only).
+__host__ __device__ constexpr int two_cap(int q, int sbytes) {
+    const int lds = 160 * 1024 / (zring_planes(q) * sbytes + 8);
+    const int maxc = two_split(q, sbytes, true) && sbytes == 4 ? 704 : 1024;
+    if (lds >= maxc) return maxc;
+    // one slot more than cells where the last wavefront is cut short (two_slots)
+    return sbytes == 8 ? lds / 64 * 64 : lds - 1;
+}
+// Threads of a workgroup, and slots per plane of its ring: one per thread, so
+// that threads without a cell have a slot to write to as well, or as many as
+// fit the LDS, of which such threads share the last.
+__host__ __device__ constexpr int two_threads(int q, int sbytes) { return (two_cap(q, sbytes) + 63) / 64 * 64; }
+__host__ __device__ constexpr int two_slots(int q, int sbytes) {
+    const int lds = 160 * 1024 / (zring_planes(q) * sbytes + 8), t = two_threads(q, sbytes);
+    return t < lds ? t : lds;
+}
+// Rows per tile for a lattice, a storage width and a tile width: the largest
+// BY whose grown tile, (bx + 2) x (BY + 2) cells, is within two_cap(); 0 where
+// no BY >= 3 is.
 __host__ __device__ constexpr int two_rows(int q, int sbytes, int bx) {
     int best = 0;
-    const int maxc = two_split(q, sbytes, true) && sbytes == 4 ? 704 : 1024;
     for (int by = 1; by <= 40; ++by)
-        if (two_cells(bx, by) * (zring_planes(q) * sbytes + 8) <= 160 * 1024 && two_cells(bx, by) <= maxc) best = by;
+        if (two_cells(bx, by) <= two_cap(q, sbytes)) best = by;
     return best >= 3 ? best : 0;
 }
 // The tile width a lattice and storage width prefer: 32 for 8-byte storage,
@@ -469,13 +511,6 @@ __host__ __device__ constexpr int two_rows(int q, int sbytes, int bx) {
 // slower at 384^3).
 __host__ __device__ constexpr int two_tile_pref(int q, int sbytes) { return (void)q, sbytes == 8 ? 32 : 64; }
 
-// Cells of a grown tile, (bx + 2) x (by + 2), that a tile of any shape may
-// have: what fits the LDS, in whole wavefronts where the ring allows it.
-__host__ __device__ constexpr int two_cap(int q, int sbytes) {
-    const int lds = 160 * 1024 / (zring_planes(q) * sbytes + 8);
-    const int maxc = two_split(q, sbytes, true) && sbytes == 4 ? 704 : 1024;
-    return lds < maxc ? (lds > 448 && sbytes == 8 ? 448 : lds) : maxc;
-}
 // The tile shape for rows of X cells and Y rows: nx x ny equal tiles (the last
 // of a row or column may be short).  A launch costs the grown cells of every
 // tile, (bx + 2) x (by + 2) x nx x ny, and the lines its rows touch: a row of

@@ -72,18 +72,19 @@ __global__ __launch_bounds__(multi_threads(OX, OZ)) void k_multi9(const typename
     uint32_t m = 0;
     bool self_solid;
     S fv[9];
+    constexpr I sz = (I)sizeof(S);
+    const I psz = ps * sz;
+    const PopBuffers<9, 1> ra(A, psz), rb(B, psz);
     if (NB) {
         m = nbmask[c];
         self_solid = m & 1u;
-        constexpr I sz = (I)sizeof(S);
-        Seams<I> sb = sm;
-        sb.xm *= sz, sb.xp *= sz, sb.ym *= sz, sb.yp *= sz, sb.zm *= sz, sb.zp *= sz;
-        gather_mask<9, 0, V, false, kAll>(fv, A, c * sz, ps * sz, m, sb);
     } else {
         self_solid = (a.bc.wall_lo[0] && gx == 0) || (a.bc.wall_hi[0] && gx + 1u == X) ||
                      (a.bc.wall_lo[2] && gz == 0) || (a.bc.wall_hi[2] && gz + 1u == Z);
-        gather_walls<9, 0, V, false, kAll>(fv, A, c, ps, sm);
     }
+    Seams<I> sb = sm;
+    sb.xm *= sz, sb.xp *= sz, sb.ym *= sz, sb.yp *= sz, sb.zm *= sz, sb.zp *= sz;
+    gather<9, 0, V, NB, 1, kAll>(fv, ra, A, c * sz, psz, m, sb);
     T f[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k) f[k] = P::load_raw(fv[k]);
@@ -98,7 +99,8 @@ __global__ __launch_bounds__(multi_threads(OX, OZ)) void k_multi9(const typename
         }
         if (s == steps) {
             // the tile's own cells; zeros for those that are not fluid
-            if (on && x0 + ix - h < X && z0 + iz - h < Z) store_own<9, V, false>(f, B, c, ps, self_solid);
+            const bool own = on && x0 + ix - h < X && z0 + iz - h < Z;
+            store_own<9, V, 1>(f, rb, B, own ? c * sz : kNoStore, psz, self_solid);
             return;
         }
         if (on && !self_solid) {

@@ -33,18 +33,51 @@ namespace plb {
 
 namespace {
 
-// Element (population k, cell offset i) of a population array.  W = false:
-// one 32-bit element offset k * pstride + i from the array base (every byte
-// offset of the array fits 32 bits); W = true: the population's base pointer
-// (a 64-bit scalar) plus the 32-bit cell offset (every byte offset within one
-// population fits 32 bits), for arrays beyond 4 GiB.
-template <bool W, class S>
-__device__ inline S* pop_elem(S* A, uint32_t k, uint32_t ps, uint32_t i) {
-    if constexpr (W)
-        return elem(A + (uint64_t)k * ps, i);
-    else
-        return elem(A, k * ps + i);
+// Buffer accesses: a buffer's bytes [0, bytes), byte offset voff (per lane) +
+// soff (uniform).  A lane whose voff is kNoStore stores nothing: it lies past
+// every buffer's end (buffers end below it), and the memory unit drops stores
+// past the end of a buffer.
+constexpr uint32_t kNoStore = 0xfffffff8u;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+__device__ inline __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00027000);
 }
+template <class S>
+__device__ inline S buf_load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    if constexpr (sizeof(S) == 8)
+        return __builtin_bit_cast(S, __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0));
+    else if constexpr (sizeof(S) == 4)
+        return __builtin_bit_cast(S, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
+    else
+        return __builtin_bit_cast(S, __builtin_amdgcn_raw_buffer_load_b16(r, (int)voff, (int)soff, 0));
+}
+template <class S>
+__device__ inline void buf_store(__amdgpu_buffer_rsrc_t r, S v, uint32_t voff, uint32_t soff) {
+    if constexpr (sizeof(S) == 8)
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)voff, (int)soff, 0);
+    else if constexpr (sizeof(S) == 4)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, (int)voff, (int)soff, 0);
+    else
+        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, (int)voff, (int)soff, 0);
+}
+
+// A population array as W buffers, whole pairs of opposite directions each
+// (W = 0: none).  Two to four of them cost a few scalar registers; a buffer for
+// each pair, and pointers, cost D3Q27 384^3 FP32-shifted 1,841 and 1,711 us per
+// step (1,560 with two buffers).
+template <int Q, int W>
+struct PopBuffers {
+    __amdgpu_buffer_rsrc_t r[W ? W : 1];
+    __device__ PopBuffers(const void* A, uint32_t psz) {
+#pragma unroll
+        for (int g = 0; g < (W ? W : 1); ++g) {
+            const int first = two_group_first(Q, W, g), end = two_group_first(Q, W, g + 1);
+            r[g] = buffer_of(reinterpret_cast<const char*>(A) + (uint64_t)first * psz,
+                             W ? (uint32_t)(end - first) * psz : 0u);
+        }
+    }
+};
 
 // The arguments of one domain of a batch (batch_two.hpp).
 template <class T>
@@ -59,77 +92,57 @@ __device__ constexpr bool in_group() {
     return G == kAll || (Lat<Q>::cz(K) > 0) == (G == kUp);
 }
 
-// Step t loads without interior solids, for the directions of group G:
-// population k from x - c_k, or the cell's own slot rev(k) where x - c_k is
-// a wall layer (known from the coordinates, so no load waits on a flag).
-template <int Q, int K, int V, bool W, int G>
-__device__ inline void gather_walls(typename Prec<V>::S (&fv)[Q], const typename Prec<V>::S* __restrict__ A,
-                                    uint32_t c, uint32_t ps, const Seams<uint32_t>& s) {
-    if constexpr (K < Q && !in_group<Q, K, G>()) {
-        gather_walls<Q, K + 1, V, W, G>(fv, A, c, ps, s);
-    } else if constexpr (K < Q) {
-        const bool wall = pull_wall<Q, K>(s);
-        if constexpr (W) {
-            fv[K] = *pop_elem<W>(A, wall ? (uint32_t)rev_k<Q>(K) : (uint32_t)K, ps,
-                                 wall ? c : c + pull_offset<Q, K>(s));
-        } else {
-            const uint32_t moved = (uint32_t)K * ps + (c + pull_offset<Q, K>(s));
-            const uint32_t own = (uint32_t)rev_k<Q>(K) * ps + c;
-            fv[K] = *elem(A, wall ? own : moved);
-        }
-        gather_walls<Q, K + 1, V, W, G>(fv, A, c, ps, s);
-    }
-}
-
-// Step t loads around interior solids, for the directions of group G:
-// population k from x - c_k, or the cell's own slot rev(k) where the
-// neighbour mask m says x - c_k is not fluid (one load per population).
-template <int Q, int K, int V, bool W, int G>
-__device__ inline void gather_mask(typename Prec<V>::S (&fv)[Q], const typename Prec<V>::S* __restrict__ A,
-                                   uint32_t c, uint32_t ps, uint32_t m, const Seams<uint32_t>& s) {
-    if constexpr (K < Q && !in_group<Q, K, G>()) {
-        gather_mask<Q, K + 1, V, W, G>(fv, A, c, ps, m, s);
-    } else if constexpr (K < Q) {
-        constexpr uint32_t R = (uint32_t)rev_k<Q>(K);
-        const bool solid = ((m >> R) & 1u) != 0;
-        if constexpr (W) {
-            fv[K] = *pop_elem<W>(A, solid ? R : (uint32_t)K, ps, solid ? c : c + pull_offset<Q, K>(s));
-        } else {
-            // byte offsets (c, ps and the seams of s in bytes): the population
-            // parts are uniform (a selected population number times pstride
-            // would be a per-lane multiply) and the cell parts shared between
-            // directions; the mask bit, sign-extended to all ones, selects
-            // bit by bit
+// Step t loads for the directions of group G: population k from x - c_k, or
+// the cell's own slot rev(k) where that neighbour is not fluid, by the
+// neighbour mask m around interior solids (NB) and by the coordinates without
+// (so no load waits on a flag); one load per population.  c, psz (the bytes of
+// a population) and the seams s are in bytes.  Directions k and rev(k) are
+// neighbours in the array (1 and 2, 3 and 4, ...), so with the lower one's
+// base as the uniform part of the address, the two candidates differ by a
+// per-lane offset and psz only.  The array is W buffers of up to 4 GiB
+// (PopBuffers); W = 0: pointers (larger arrays, every byte offset of one
+// population within 32 bits).
+template <int Q, int K, int V, int NB, int W, int G>
+__device__ inline void gather(typename Prec<V>::S (&fv)[Q], const PopBuffers<Q, W>& ra,
+                              const typename Prec<V>::S* __restrict__ A, uint32_t c, uint32_t psz, uint32_t m,
+                              const Seams<uint32_t>& s) {
+    if constexpr (K < Q) {
+        if constexpr (in_group<Q, K, G>()) {
             using S = typename Prec<V>::S;
-            (void)solid;
-            const uint32_t moved = (uint32_t)K * ps + (c + pull_offset<Q, K>(s));
-            const uint32_t own = R * ps + c;
-            const uint32_t sel = (uint32_t)__builtin_amdgcn_sbfe((int)m, (int)R, 1);
-            fv[K] = *reinterpret_cast<const S*>(reinterpret_cast<const char*>(A) + (moved ^ ((moved ^ own) & sel)));
+            constexpr uint32_t R = (uint32_t)rev_k<Q>(K);
+            const bool solid = NB ? ((m >> R) & 1u) != 0 : pull_wall<Q, K>(s);
+            const uint32_t to = c + pull_offset<Q, K>(s);
+            if constexpr (W == 0) {
+                const char* p = reinterpret_cast<const char*>(A) + (uint64_t)(solid ? R : (uint32_t)K) * psz;
+                fv[K] = *reinterpret_cast<const S*>(p + (solid ? c : to));
+            } else {
+                constexpr uint32_t lower = (uint32_t)K < R ? (uint32_t)K : R;
+                const uint32_t moved = (uint32_t)K == lower ? to : to + psz, own = (uint32_t)K == lower ? c + psz : c;
+                const uint32_t off = K == 0 ? c : (solid ? own : moved);
+                constexpr int g = two_group(Q, W, K);
+                fv[K] = buf_load<S>(ra.r[g], off, (lower - (uint32_t)two_group_first(Q, W, g)) * psz);
+            }
         }
-        gather_mask<Q, K + 1, V, W, G>(fv, A, c, ps, m, s);
+        gather<Q, K + 1, V, NB, W, G>(fv, ra, A, c, psz, m, s);
     }
 }
 
-// Step t + 2 of a cell into its own slots (zeros for a cell that is not fluid).
-// Each population's base pointer is a scalar and the cell's byte offset is
-// shared by all of them.  (The compiler turns these into one 64-bit address
-// add per store, where per-population 32-bit offsets from the array base
-// kept about 30 loop-carried offsets in vector registers; forcing the base
-// into a scalar operand, as the cell kernel does, compiled this kernel to
-// more instructions.)
-template <int Q, int V, bool NT>
-__device__ inline void store_own(const typename Prec<V>::T (&f)[Q], typename Prec<V>::S* __restrict__ B, uint32_t c,
-                                 uint32_t ps, bool zero) {
+// Step t + 2 of a cell into its own slots (zeros where zero is set), at byte
+// offset voff of each population; kNoStore: no store (a lane's, without a
+// branch).
+template <int Q, int V, int W>
+__device__ inline void store_own(const typename Prec<V>::T (&f)[Q], const PopBuffers<Q, W>& rb,
+                                 typename Prec<V>::S* __restrict__ B, uint32_t voff, uint32_t psz, bool zero) {
     using P = Prec<V>;
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
         const typename P::S v = P::store_raw(zero ? (typename P::T)0 : f[k]);
-        typename P::S* p = pop_elem<true>(B, (uint32_t)k, ps, c);
-        if (NT)
-            __builtin_nontemporal_store(v, p);
-        else
-            *p = v;
+        if constexpr (W == 0) {
+            buf_store(buffer_of(reinterpret_cast<const char*>(B) + (uint64_t)k * psz, psz), v, voff, 0u);
+        } else {
+            const int g = two_group(Q, W, k);
+            buf_store(rb.r[g], v, voff, (uint32_t)(k - two_group_first(Q, W, g)) * psz);
+        }
     }
 }
 
@@ -195,10 +208,11 @@ __device__ inline void lds_barrier() {
 }
 
 // The sweep of one workgroup over the planes [z0, z0 + zc) of the tile of
-// bx x by cells at (x0, y0).  BX, BY: the tile shape where it is compiled in;
-// BX = 0: any shape of at most two_cap() grown cells (bx, by), the ring laid
-// out for that many.  a: FusedArgs, or the like for one domain of a batch.
-template <int Q, int V, int NB, bool MOV, int BX, int BY, bool W, bool SPLIT, class Args>
+// bx x by cells at (x0, y0), of any shape with at most two_cap() grown cells.
+// (With 64 x 8 and 32 x 11 tiles compiled in, D3Q19 256^3 ran 269 / 591 us per
+// step walls only, FP32-shifted / FP64, against 263 / 595 with the shape as an
+// argument.)  a: FusedArgs, or the like for one domain of a batch.
+template <int Q, int V, int NB, bool MOV, int W, bool SPLIT, class Args>
 __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict__ A,
                                            typename Prec<V>::S* __restrict__ B, const uint8_t* __restrict__ flags,
                                            const uint32_t* __restrict__ nbmask, const Args& a, uint32_t bx,
@@ -207,9 +221,9 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
     using S = typename P::S;
     using T = typename P::T;
     using I = uint32_t;
-    constexpr int NI = BX ? two_cells(BX, BY) : two_cap(Q, (int)sizeof(S));
-    const uint32_t TX = BX ? (uint32_t)BX : bx, TY = BX ? (uint32_t)BY : by;  // tile cells
-    const uint32_t RX = TX + 2u;                                              // grown row
+    constexpr int NI = two_slots(Q, (int)sizeof(S)), NT = two_threads(Q, (int)sizeof(S));
+    static_assert(NI == NT || two_cap(Q, (int)sizeof(S)) < NI, "a slot for the threads without a cell");
+    const uint32_t RX = bx + 2u;  // grown row
     __shared__ S ring[ZRing<Q>::planes() * NI];
     __shared__ uint32_t mring[2 * NI];  // the step t + 1 cells' masks or flags, two planes
 
@@ -219,15 +233,15 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
     const uint32_t nplanes = std::min(zc, Z - z0) + 2u;
 
     // step t + 1: this thread's cell of the grown tile (wrapped coordinates)
-    const bool in_i = tid < (BX ? (uint32_t)NI : RX * (TY + 2u));
+    const uint32_t slot = NI == NT ? tid : std::min(tid, (uint32_t)NI - 1u);  // in the ring
     const uint32_t ix = tid % RX, iy = tid / RX;
     const uint32_t gx = (x0 + ix + X - 1u) % X, gy = (y0 + iy + Y - 1u) % Y;
     // step t + 2: this thread's cell of the tile
-    const uint32_t ox = tid % TX, oy = tid / TX;
-    const bool in_o = oy < TY && y0 + oy < Y && x0 + ox < X;
+    const uint32_t ox = tid % bx, oy = tid / bx;
+    const bool in_o = oy < by && y0 + oy < Y && x0 + ox < X;
     const uint32_t px = x0 + ox, py = y0 + oy;
-    // (threads without a cell, which take no part in step t + 2, read cell 0)
-    const I li = BX || in_o ? (oy + 1u) * RX + ox + 1u : 0u;
+    // (a thread without a cell reads those of the first one and stores nothing)
+    const I li = in_o ? (oy + 1u) * RX + ox + 1u : RX + 1u;
 
     // Loads of step t, issued an iteration ahead of the plane that uses them.
     // SPLIT issues the directions with c_z = +1 two iterations ahead instead,
@@ -259,52 +273,59 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
         else return NB ? nbmask[c] : (uint32_t)flags[c];
     };
     // the loads of plane n's directions of group G into fv
+    constexpr I sz = (I)sizeof(S);
+    const I psz = ps * sz;
+    const PopBuffers<Q, W> ra(A, psz), rb(B, psz);
     auto fetch = [&](auto group, uint32_t n, S (&fv)[Q], uint32_t m) __attribute__((always_inline)) {
         constexpr int G = decltype(group)::value;
         const uint32_t zi = (z0 + n + Z - 1u) % Z;
         const I c = zi * XY + gy * X + gx;
-        const Seams<I> sm = seams<I>(gx, gy, zi, a);
-        if (NB && !W) {
-            // in bytes: one vector add per cell part, none per direction
-            constexpr I sz = (I)sizeof(S);
-            Seams<I> sb = sm;
-            sb.xm *= sz, sb.xp *= sz, sb.ym *= sz, sb.yp *= sz, sb.zm *= sz, sb.zp *= sz;
-            gather_mask<Q, 0, V, W, G>(fv, A, c * sz, ps * sz, m, sb);
-        } else if (NB) {
-            gather_mask<Q, 0, V, W, G>(fv, A, c, ps, m, sm);
-        } else {
-            gather_walls<Q, 0, V, W, G>(fv, A, c, ps, sm);
-        }
+        Seams<I> sb = seams<I>(gx, gy, zi, a);
+        sb.xm *= sz, sb.xp *= sz, sb.ym *= sz, sb.yp *= sz, sb.zm *= sz, sb.zp *= sz;
+        gather<Q, 0, V, NB, W, G>(fv, ra, A, c * sz, psz, m, sb);
     };
     using All = std::integral_constant<int, kAll>;
     using Up = std::integral_constant<int, kUp>;
     using Flat = std::integral_constant<int, kFlat>;
 
-    // Step t + 2 of the tile's cell at plane n - 2 of the chunk (iteration n):
-    // from the ring planes of iterations n - 2, n - 1 and n, with the mask of
-    // its step t + 1 cell (stored in mring by iteration n - 1).
+    // Step t + 2 of the tile's cell at plane n - 2 of the chunk (iteration n;
+    // none in the first two): from the ring planes of iterations n - 2, n - 1
+    // and n, with the mask of its step t + 1 cell (stored in mring by
+    // iteration n - 1).
     auto step2 = [&](uint32_t n) __attribute__((always_inline)) {
         const uint32_t zo = z0 + n - 2u;
-        const I c = zo * XY + py * X + px;
         const uint32_t pa = (n + 1u) % 3u, oa = (n + 2u) % 3u, b0 = (n + 1u) & 1u, c1 = n & 1u;
+        if (n < 2u) return;
+        // One straight run of instructions from the ring's reads to the
+        // stores, threads without a cell and cells that are not fluid
+        // included (what they compute is dropped): the compiler then spreads
+        // the stores over the arithmetic, and in step 1 the next plane's loads,
+        // instead of issuing them in bursts at the end of a branch.  The
+        // kernel is bound by neither alone (D3Q19 256^3 FP32-shifted around
+        // solids: vector unit 65% busy, memory unit 67%), so what counts is
+        // that both work at the same time: 341 -> 317 us per step with solids,
+        // 287 -> 268 walls only; FP64 647 -> 630 / 601 -> 589; D3Q27 384^3
+        // FP32-shifted 1,634 -> 1,560, FP64 3,638 -> 3,455.  (Stores in every
+        // wavefront and plane, dropped where there is nothing to store, so that
+        // no wait for a load counts a path without them: no faster on large
+        // lattices, 2-10% slower on small ones.)
         uint32_t mo;
         if constexpr (FLAGS)
             mo = mring[b0 * NI + li];
         else
             mo = wall_cell(px, py, zo);
-        const bool self_solid = NB ? (mo & 1u) != 0 : mo != 0;
-        if (!__all(self_solid)) {
+        const bool zero = NB ? (mo & 1u) != 0 : mo != 0;
+        if (__any(in_o && !zero)) {
             const Seams<I> sm = seams<I>(px, py, zo, a);
             T f[Q];
             ring_gather<Q, 0, V, NB, NI>(f, ring, li, RX, pa, oa, b0, c1, mo, sm);
-            if (!self_solid) {
-                const T rho = bgk<Q, P>(f, a, true);
-                if (MOV && a.bc.moving) moving_wall_terms<Q, P>(f, rho, sm, a);
-            }
-            if (a.nt_store)
-                store_own<Q, V, true>(f, B, c, ps, self_solid);
-            else
-                store_own<Q, V, false>(f, B, c, ps, self_solid);
+            const T rho = bgk<Q, P>(f, a, true);
+            if (MOV && a.bc.moving) moving_wall_terms<Q, P>(f, rho, sm, a);
+            // Around interior solids a cell that is not fluid stores zeros, so
+            // that lines are written whole (but a wavefront of such cells
+            // nothing); wall cells alone store nothing.
+            const bool store = in_o && (NB || !zero);
+            store_own<Q, V, W>(f, rb, B, store ? (zo * XY + py * X + px) * sz : kNoStore, psz, NB && zero);
         }
     };
     // Step t + 1 of this thread's cell at plane n from the loads in fv, into
@@ -315,7 +336,7 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
         for (int k = 0; k < Q; ++k) f[k] = P::load_raw(fv[k]);
         const T rho = bgk<Q, P>(f, a, true);
         if (MOV && a.bc.moving) moving_wall_terms<Q, P>(f, rho, seams<I>(gx, gy, (z0 + n + Z - 1u) % Z, a), a);
-        ring_store<Q, 0, V, NI>(f, ring, tid, a3, a2);
+        ring_store<Q, 0, V, NI>(f, ring, slot, a3, a2);
     };
 
     if constexpr (!SPLIT) {
@@ -333,15 +354,13 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
             mnext = load_mask(n + 1u);
             // ring slots of plane n (relative plane numbers: only n mod 3 and mod 2 matter)
             const uint32_t a3 = n % 3u, a2 = n & 1u;
-            if (in_i) {
-                // the step t + 2 cells read this mask in the next iteration
-                if (FLAGS) mring[a2 * NI + tid] = mcur;
-                const bool self_solid = NB ? (mcur & 1u) != 0 : mcur != 0;
-                if (!self_solid) step1(n, fv, a3, a2);
-            }
+            // the step t + 2 cells read this mask in the next iteration
+            if (FLAGS) mring[a2 * NI + slot] = mcur;
+            // (a wavefront of solid cells has nothing to compute)
+            if (!__all(NB ? (mcur & 1u) != 0 : mcur != 0)) step1(n, fv, a3, a2);
             fetch(All{}, n + 1u, fv, mnext);
             lds_barrier();
-            if (n >= 2u && in_o) step2(n);
+            step2(n);
             lds_barrier();
         };
         uint32_t m0 = load_mask(0), m1 = 0;
@@ -356,7 +375,9 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
         // (its c_z = +1 directions are in flight) with the mask mn of plane
         // n + 1, loaded an iteration ago; the mask of plane n + 2 into mc and
         // its c_z = +1 directions into fc; the step t + 2 cell of plane
-        // n - 1.  The loop runs it twice per trip with the register sets
+        // n - 1.  Step t + 1 runs in every wavefront, also one of solid cells:
+        // behind a vote the loads would not spread over it (317 -> 332 us per
+        // step).  The loop runs it twice per trip with the register sets
         // swapped (odd: fc = fv1, fn = fv0), so that no register that a load
         // in flight writes is copied.
         S fv0[Q], fv1[Q];
@@ -364,14 +385,13 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
             S (&fc)[Q] = decltype(odd)::value ? fv1 : fv0;
             S (&fn)[Q] = decltype(odd)::value ? fv0 : fv1;
             const uint32_t a3 = n % 3u, a2 = n & 1u;
-            if (FLAGS && in_i) mring[a2 * NI + tid] = mc;
-            const bool self_solid = NB ? (mc & 1u) != 0 : mc != 0;
+            if (FLAGS) mring[a2 * NI + slot] = mc;
             mc = load_mask(n + 2u);
-            if (in_i && !self_solid) step1(n, fc, a3, a2);
             fetch(Flat{}, n + 1u, fn, mn);
+            step1(n, fc, a3, a2);
             fetch(Up{}, n + 2u, fc, mc);
             lds_barrier();
-            if (n >= 2u && in_o) step2(n);
+            step2(n);
             lds_barrier();
         };
         uint32_t m0 = load_mask(0), m1 = load_mask(1);
@@ -384,13 +404,8 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
     }
 }
 
-// Threads of a workgroup: one per grown cell, in whole wavefronts.
-__host__ __device__ constexpr int pull2_threads(int q, int sbytes, int bx, int by) {
-    return bx ? two_threads(bx, by) : (two_cap(q, sbytes) + 63) / 64 * 64;
-}
-
-template <int Q, int V, int NB, bool MOV, int BX, int BY, bool W, bool SPLIT>
-__global__ __launch_bounds__(pull2_threads(Q, (int)sizeof(typename Prec<V>::S), BX, BY), 1) void k_pull2(
+template <int Q, int V, int NB, bool MOV, int W>
+__global__ __launch_bounds__(two_threads(Q, (int)sizeof(typename Prec<V>::S)), 1) void k_pull2(
     const typename Prec<V>::S* __restrict__ A, typename Prec<V>::S* __restrict__ B,
     const uint8_t* __restrict__ flags, const uint32_t* __restrict__ nbmask, FusedArgs<typename Prec<V>::T> a,
     TwoGeom g) {
@@ -409,50 +424,37 @@ __global__ __launch_bounds__(pull2_threads(Q, (int)sizeof(typename Prec<V>::S), 
         ty = r % g.nty;
         tz = r / g.nty;
     }
-    const uint32_t bx = BX ? (uint32_t)BX : g.bx, by = BX ? (uint32_t)BY : g.by;
-    pull2_tile<Q, V, NB, MOV, BX, BY, W, SPLIT>(A, B, flags, nbmask, a, bx, by, tx * bx, ty * by, tz * g.zc, g.zc);
+    pull2_tile<Q, V, NB, MOV, W, two_split(Q, (int)sizeof(typename Prec<V>::S), NB != 0)>(
+        A, B, flags, nbmask, a, g.bx, g.by, tx * g.bx, ty * g.by, tz * g.zc, g.zc);
 }
 
 }  // namespace
-
-// Tiles BX cells wide in their compiled shape; BX = 0: any shape.
-template <int Q, int V, int BX, bool W>
-bool launch_pull2_bx(const FusedArgs<typename Prec<V>::T>& a, const TwoGeom& g, bool nb, bool mov,
-                     const typename Prec<V>::S* A, typename Prec<V>::S* B, const uint8_t* flags,
-                     const uint32_t* nbmask, hipStream_t stream) {
-    constexpr int sb = (int)sizeof(typename Prec<V>::S), BY = BX ? two_rows(Q, sb, BX) : 0;
-    if constexpr (BX != 0 && BY == 0) {
-        return false;
-    } else {
-        // a tile of any shape must fit the ring and the workgroup
-        if (BX == 0 && ((int)((g.bx + 2) * (g.by + 2)) > two_cap(Q, sb) || g.bx < 1 || g.by < 1)) return false;
-        const dim3 grid(two_blocks(g)), block(pull2_threads(Q, sb, BX, BY));
-#define PLB_TWO(NBv, MVv)                                                                               \
-    hipLaunchKernelGGL((k_pull2<Q, V, NBv, MVv, BX, BY, W, two_split(Q, sb, NBv != 0)>), grid, block, 0, \
-                       stream, A, B, flags, nbmask, a, g)
-        if (nb && mov) PLB_TWO(1, true);
-        else if (nb) PLB_TWO(1, false);
-        else if (mov) PLB_TWO(0, true);
-        else PLB_TWO(0, false);
-#undef PLB_TWO
-        return true;
-    }
-}
 
 template <int Q, int V>
 bool launch_pull2(const FusedArgs<typename Prec<V>::T>& a, const TwoGeom& g, bool nb, bool mov,
                   const typename Prec<V>::S* A, typename Prec<V>::S* B, const uint8_t* flags,
                   const uint32_t* nbmask, hipStream_t stream) {
-    const bool w = g.wide != 0;
-    auto go = [&](auto bxc) {
-        constexpr int BX = decltype(bxc)::value;
-        return w ? launch_pull2_bx<Q, V, BX, true>(a, g, nb, mov, A, B, flags, nbmask, stream)
-                 : launch_pull2_bx<Q, V, BX, false>(a, g, nb, mov, A, B, flags, nbmask, stream);
+    constexpr int sb = (int)sizeof(typename Prec<V>::S);
+    // the tile must fit the ring and the workgroup
+    if (g.bx < 1 || g.by < 1 || (uint64_t)(g.bx + 2) * (g.by + 2) > (uint64_t)two_cap(Q, sb)) return false;
+    const dim3 grid(two_blocks(g)), block(two_threads(Q, sb));
+    auto go = [&](auto nbc, auto mvc, auto wc) {
+        hipLaunchKernelGGL((k_pull2<Q, V, decltype(nbc)::value, decltype(mvc)::value, decltype(wc)::value>), grid,
+                           block, 0, stream, A, B, flags, nbmask, a, g);
     };
-    if (g.any) return go(std::integral_constant<int, 0>());
-    if (g.bx == 64) return go(std::integral_constant<int, 64>());
-    if (g.bx == 32) return go(std::integral_constant<int, 32>());
-    return false;
+    auto by_walls = [&](auto wc) {
+        using N0 = std::integral_constant<int, 0>;
+        using N1 = std::integral_constant<int, 1>;
+        if (nb) mov ? go(N1{}, std::true_type{}, wc) : go(N1{}, std::false_type{}, wc);
+        else mov ? go(N0{}, std::true_type{}, wc) : go(N0{}, std::false_type{}, wc);
+    };
+    switch (g.buffers) {
+        case 1: by_walls(std::integral_constant<int, 1>()); break;
+        case 2: by_walls(std::integral_constant<int, 2>()); break;
+        case 4: by_walls(std::integral_constant<int, 4>()); break;
+        default: by_walls(std::integral_constant<int, 0>()); break;
+    }
+    return true;
 }
 
 #define PLB_TWO_INST(Q, V)                                                                                  \

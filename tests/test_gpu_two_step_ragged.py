@@ -64,3 +64,30 @@ def test_ragged_two_step_rule():
     with P.State(19, 70, 61, 63, "f64", P.FUSED) as st:
         st.set_tuning(capi.TUNE_TWO_TILE_X, 32)
         assert st.scheme() == "pull"
+
+
+@pytest.mark.parametrize("q,pad", [(19, 70 << 20), (19, 100 << 20), (19, 160 << 20), (27, 50 << 20), (27, 100 << 20),
+                                   (27, 130 << 20)])
+def test_two_step_array_sizes(q, pad):
+    """Arrays addressed as two and four buffers and by pointers (populations
+    set far apart on a small lattice): the values of the array that one
+    buffer holds, bit for bit."""
+    X, Y, Z = 64, 10, 9
+    types, vel = [PERIODIC] * 4 + [NOSLIP] * 2, {P.UP: (0.02, 0.0, 0.0), P.DOWN: (0.0, 0.0, 0.0)}
+    pb = P.boundary(types, vel)
+    for solids in (True, False):
+        print(f"\n[case] two-step array sizes q={q} pad={pad} solids={solids}", flush=True)
+        mask = (np.random.default_rng(8).random((Z, Y, X)) < 0.12).astype(np.uint8) if solids else None
+        out = []
+        for p in (-1, pad):
+            with P.State(q, X, Y, Z, "f32s", P.FUSED, pop_pad=p) as st:
+                st.set_tuning(capi.TUNE_TWO_STEP, 1)
+                assert st.scheme() == "pull2"
+                st.set_boundary(pb, mask)
+                st.initialize(1.0, (0.01, 0.0, 0.0), (P.INIT_PERTURBED, 5, 2e-3), pb)
+                st.configure(0.62, (2e-5, -1e-6, 1e-6), pb)
+                st.step(7)
+                out.append((st.download_raw()[1:-1], st.moments()))
+        fluid = slice(None) if mask is None else mask[1:-1] == 0
+        assert np.array_equal(out[0][0][fluid], out[1][0][fluid])
+        assert all(np.array_equal(a, b) for a, b in zip(out[0][1], out[1][1]))
