@@ -517,7 +517,7 @@ int plb_stream(plb_state* s, const char* stream_type) {
         const plb_boundary* per = q[0].kind == kLitPeriodic ? &q[0].bc : nullptr;
         const LitOp* r = &c - 2;
         return timed(s, PLB_STAGE_COLLIDE, [&] {
-            return lit_moments_collide_push(s, c.tau, c.force, per, &r[0].bc, &r[1].bc, nullptr);
+            return lit_moments_collide_push(s, c.tau, c.force, per, &r[0].bc, &r[1].bc, nullptr, true);
         });
     }
     // every other request finds the deferred calls done, as the reference's does
@@ -679,7 +679,7 @@ int plb_step(plb_state* s, int nsteps) {
             const bool fold = s->tune_lit_fuse != 0;
             if (fold && i > 0) {
                 if ((rc = timed(s, PLB_STAGE_COLLIDE,
-                                [&] { return lit_moments_collide_push(s, s->tau, F, bc, bc, bc, bc); })))
+                                [&] { return lit_moments_collide_push(s, s->tau, F, bc, bc, bc, bc, i + 1 == nsteps); })))
                     return rc;
             } else if (fold) {
                 if ((rc = timed(s, PLB_STAGE_COLLIDE, [&] { return lit_collide_push(s, s->tau, F); })))

@@ -461,6 +461,19 @@ __device__ inline bool near_noslip(const MomentStores& ms, const LitDims& g, int
            (ms.hi[1] && y >= g.Y - 1) || (ms.lo[2] && z <= 2) || (ms.hi[2] && z >= g.Z - 1);
 }
 
+// Whether the cell lies on a no-slip face.
+__device__ inline bool on_noslip(const MomentStores& ms, const LitDims& g, int x, int y, int z) {
+    return (ms.lo[0] && x == 1) || (ms.hi[0] && x == g.X) || (ms.lo[1] && y == 1) || (ms.hi[1] && y == g.Y) ||
+           (ms.lo[2] && z == 1) || (ms.hi[2] && z == g.Z);
+}
+// Whether c - c_k of interior cell c lies in the halo: a slot no push writes.
+template <int Q>
+__device__ inline bool from_halo(const LitDims& g, int k, int x, int y, int z) {
+    const int cx = Lat<Q>::cx(k), cy = Lat<Q>::cy(k), cz = Lat<Q>::cz(k);
+    return (cx > 0 && x == 1) || (cx < 0 && x == g.X) || (cy > 0 && y == 1) || (cy < 0 && y == g.Y) ||
+           (cz > 0 && z == 1) || (cz < 0 && z == g.Z);
+}
+
 // The previous step's periodic copies, moments and resets (Boundary,
 // CalcMoments) folded into this step's collision and push, inside plb_step or
 // for staged calls that the C ABI deferred until the push.
@@ -472,10 +485,17 @@ __device__ inline bool near_noslip(const MomentStores& ms, const LitDims& g, int
 // periodic copies in and leaving the dead rho and u stores out took the step
 // of plb_step from 252 to 221 us (D3Q19 128^3 FP64: 38 instead of 42 values
 // per cell, two launches fewer) and from 10.6 to 8.1 us (D2Q9 256 x 64 FP64).
+//
+// In-place stores: all of the outer layer where the caller can see ntmp
+// afterwards (keep_all).  Where plb_step goes on with another of these kernels
+// (the same per and no-slip faces, nothing read in between), the push of that
+// step overwrites every slot (c, k) with c - c_k interior before anything
+// reads it, and of the others it reads (c, k) itself only where no periodic
+// copy takes its place, and the no-slip pass only those of its face cells.
 template <int Q, class R>
 __global__ void k_moments_collide_push(LitDims g, R* __restrict__ n, R* __restrict__ rho, R* __restrict__ u,
-                                       R* __restrict__ t, Periodic per, FaceResets<R> fr, MomentStores ms, R tau,
-                                       R om, R omm, R F0, R F1, R F2) {
+                                       R* __restrict__ t, Periodic per, FaceResets<R> fr, MomentStores ms,
+                                       int keep_all, R tau, R om, R omm, R F0, R F1, R F2) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int y = blockIdx.y + 1, z = blockIdx.z + 1;
     if (x > g.X) return;
@@ -497,13 +517,13 @@ __global__ void k_moments_collide_push(LitDims g, R* __restrict__ n, R* __restri
         u[g.ncell + c] = um[1];
         u[2 * g.ncell + c] = um[2];
     }
-    const bool keep = outer_layer(g, x, y, z);
+    const bool outer = outer_layer(g, x, y, z), all = keep_all && outer, face = on_noslip(ms, g, x, y, z);
     R uu[3], usq;
     updated_u(um[0], um[1], um[2], rl, tau, F0, F1, F2, uu, usq);
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
         const R v = collide_value<Q, R>(k, nv[k], rl, uu, usq, om, omm);
-        if (keep) n[k * g.ncell + c] = v;
+        if (all || (outer && from_halo<Q>(g, k, x, y, z) && (face || shift_of<Q>(sh, k) == 0))) n[k * g.ncell + c] = v;
         const int64_t off = (int64_t)Lat<Q>::cx(k) + (int64_t)Lat<Q>::cy(k) * g.nx +
                             (int64_t)Lat<Q>::cz(k) * g.nx * g.ny;
         t[k * g.ncell + (uint64_t)((int64_t)c + off)] = v;
@@ -708,7 +728,8 @@ FaceResets<R> face_resets(const plb_boundary* bc_vel, const plb_boundary* bc_rho
 }  // namespace
 
 int lit_moments_collide_push(plb_state* s, double tau, const double F[3], const plb_boundary* bc_per,
-                             const plb_boundary* bc_vel, const plb_boundary* bc_rho, const plb_boundary* bc_noslip) {
+                             const plb_boundary* bc_vel, const plb_boundary* bc_rho, const plb_boundary* bc_noslip,
+                             bool keep_all) {
     const LitDims g = dims_of(s);
     const int rc = with_qr(s, [&](auto qc, auto rr) {
         constexpr int Q = decltype(qc)::value;
@@ -724,7 +745,7 @@ int lit_moments_collide_push(plb_state* s, double tau, const double F[3], const 
         }
         hipLaunchKernelGGL((k_moments_collide_push<Q, R>), interior_grid(s), dim3(interior_block(s)), 0, s->stream,
                            g, (R*)s->buf[s->cur], (R*)s->rho, (R*)s->u, (R*)s->buf[s->cur ^ 1], per,
-                           face_resets<R>(bc_vel, bc_rho), ms, tr, om, omm, (R)F[0], (R)F[1], (R)F[2]);
+                           face_resets<R>(bc_vel, bc_rho), ms, keep_all ? 1 : 0, tr, om, omm, (R)F[0], (R)F[1], (R)F[2]);
         PLB_HIP_TRY(hipGetLastError());
         return PLB_OK;
     });

@@ -158,9 +158,11 @@ int lit_collide_push(plb_state* s, double tau, const double F[3]);
 // bc_per: the periodic copies folded in (null: none); bc_vel: the faces whose
 // velocity is reset; bc_rho: those whose density is; bc_noslip: the no-slip
 // faces of this step, when nothing else reads rho or u before the next
-// moments (null: every rho and u is stored)
+// moments (null: every rho and u is stored); keep_all: ntmp can be seen after
+// this step (else another of these calls with the same boundary follows)
 int lit_moments_collide_push(plb_state* s, double tau, const double F[3], const plb_boundary* bc_per,
-                             const plb_boundary* bc_vel, const plb_boundary* bc_rho, const plb_boundary* bc_noslip);
+                             const plb_boundary* bc_vel, const plb_boundary* bc_rho, const plb_boundary* bc_noslip,
+                             bool keep_all);
 int lit_noslip(plb_state* s, const plb_boundary* bc);
 // The same pass for faces within the documented size limit of the entry point.
 int lit_noslip_noalloc(plb_state* s, const plb_boundary* bc);

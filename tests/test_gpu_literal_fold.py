@@ -89,3 +89,24 @@ def test_step_stores_the_densities_noslip_reads(orc, q, X, Y, Z, axis):
             orc.lit_run(o, 0.75, (1e-4, 0.0, -2e-5), ob, n)
             st.step(n)
             _same(st, o, n)
+
+
+@pytest.mark.parametrize("q,X,Y,Z", [(9, 70, 1, 4), (19, 5, 4, 6), (19, 1, 2, 3), (27, 66, 3, 4)])
+@pytest.mark.parametrize("faces", ["PPNNNN", "NNPPNN", "UUPPNN", "PPNUUN", "PPPPUU", "NNNNUU", "UUUUUU", "PPPPNU"])
+def test_step_keeps_what_the_next_step_reads(orc, q, X, Y, Z, faces):
+    """plb_step: inside the run a collision leaves in place only the slots that
+    no push fills and that no periodic copy replaces or a no-slip pass reads;
+    walls, seams and bare faces meet at every kind of edge here."""
+    print(f"\n[case] literal step q={q} {X}x{Y}x{Z} faces {faces}", flush=True)
+    types = [{"P": PERIODIC, "N": NOSLIP, "U": UNSET}[f] for f in faces]
+    vel = {f: (0.01 * (f + 1), -0.005 * f, 0.004) for f in range(6) if types[f] == NOSLIP}
+    ob, pb = _bc(types, vel, 1.01)
+    o = orc.lit_state(q, X, Y, Z)
+    orc.lit_init(o, 1.0, (0.01, 0.0, 0.0), (P.INIT_PERTURBED, 5, 1e-2), ob)
+    with P.State(q, X, Y, Z, "f64", P.LITERAL) as st:
+        st.initialize(1.0, (0.01, 0.0, 0.0), (P.INIT_PERTURBED, 5, 1e-2), pb)
+        st.configure(0.75, (1e-4, 0.0, -2e-5), pb)
+        for n in (2, 3, 1, 4):
+            orc.lit_run(o, 0.75, (1e-4, 0.0, -2e-5), ob, n)
+            st.step(n)
+            _same(st, o, n)
