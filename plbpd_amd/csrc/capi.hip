@@ -286,6 +286,7 @@ int plb_state_create(const plb_state_desc* d, plb_state** out) {
     s->collide_pending = false;
     s->fused_deferred = false;
     s->lit_ntmp_folded = false;
+    s->lit_saved = 0;
     s->moments_valid = false;
     s->scratch = nullptr;
     s->scratch_bytes = 0;
@@ -323,18 +324,14 @@ int plb_state_create(const plb_state_desc* d, plb_state** out) {
     for (double& v : s->stage_ms) v = 0.0;
 
     const uint64_t X = d->x, Y = d->y, Z = d->z;
-    size_t mom_bytes;
     if (s->aa) s->tune_scheme = PLB_SCHEME_AA;
     if (d->mode == PLB_MODE_LITERAL) {
         s->ncell = (X + 2) * (Y + 2) * (Z + 2);
-        s->pstride = s->ncell;
-        mom_bytes = s->ncell * s->sbytes;
     } else {
         s->ncell = X * Y * Z;
         fused_two_plan(s);
         const size_t pad = d->pop_pad >= 0 ? (size_t)d->pop_pad : (size_t)(2048 + 64);
         s->pstride = ((s->ncell + 63) / 64) * 64 + pad;
-        mom_bytes = s->ncell * sizeof(double);
     }
     auto cleanup = [&](int code, const std::string& msg) {
         plb_state_destroy(s);
@@ -346,22 +343,47 @@ int plb_state_create(const plb_state_desc* d, plb_state** out) {
         delete s;
         return fail(PLB_ERR_HIP, hipGetErrorString(e));
     }
-    const size_t pop_bytes = s->pstride * s->q * s->sbytes;
-    for (int b = 0; b < (s->aa ? 1 : 2); ++b) {
-        e = hipMalloc(&s->buf[b], pop_bytes);
-        if (e != hipSuccess) return cleanup(PLB_ERR_OOM, "population buffer: " + std::string(hipGetErrorString(e)));
-        e = hipMemset(s->buf[b], 0, pop_bytes);
-        if (e != hipSuccess) return cleanup(PLB_ERR_HIP, hipGetErrorString(e));
+    // what a failure is reported as
+    std::string what;
+    int code = PLB_ERR_OOM;
+    auto allocate = [&]() -> hipError_t {
+        const size_t pop_bytes = s->pstride * s->q * s->sbytes;
+        const size_t mom_bytes =
+            d->mode == PLB_MODE_LITERAL ? lit_cells(s) * s->sbytes : s->ncell * sizeof(double);
+        for (int b = 0; b < (s->aa ? 1 : 2); ++b) {
+            what = "population buffer: ";
+            code = PLB_ERR_OOM;
+            hipError_t e = hipMalloc(&s->buf[b], pop_bytes);
+            if (e != hipSuccess) return e;
+            what.clear();
+            code = PLB_ERR_HIP;
+            e = hipMemset(s->buf[b], 0, pop_bytes);
+            if (e != hipSuccess) return e;
+        }
+        code = PLB_ERR_OOM;
+        hipError_t e = hipMalloc(&s->rho, mom_bytes);
+        if (e == hipSuccess) e = hipMalloc(&s->u, 3 * mom_bytes);
+        if (e == hipSuccess) e = hipMemset(s->rho, 0, mom_bytes);
+        if (e == hipSuccess) e = hipMemset(s->u, 0, 3 * mom_bytes);
+        return e;
+    };
+    if (d->mode == PLB_MODE_LITERAL) lit_layout(s, false);
+    e = allocate();
+    if (e == hipErrorOutOfMemory && d->mode == PLB_MODE_LITERAL) {
+        // once more in the packed layout
+        (void)hipGetLastError();
+        for (void** p : {&s->buf[0], &s->buf[1], &s->rho, &s->u}) {
+            if (*p) (void)hipFree(*p);
+            *p = nullptr;
+        }
+        lit_layout(s, true);
+        e = allocate();
     }
-    e = hipMalloc(&s->rho, mom_bytes);
-    if (e == hipSuccess) e = hipMalloc(&s->u, 3 * mom_bytes);
-    if (e == hipSuccess) e = hipMemset(s->rho, 0, mom_bytes);
-    if (e == hipSuccess) e = hipMemset(s->u, 0, 3 * mom_bytes);
     if (e == hipSuccess && s->mode == PLB_MODE_FUSED) {
         e = hipMalloc(&s->flags, s->ncell);
         if (e == hipSuccess) e = hipMemset(s->flags, 0, s->ncell);
     }
-    if (e != hipSuccess) return cleanup(PLB_ERR_OOM, hipGetErrorString(e));
+    if (e != hipSuccess) return cleanup(code, what + hipGetErrorString(e));
     *out = s;
     return PLB_OK;
 }
@@ -390,7 +412,7 @@ int plb_state_bytes(const plb_state* s, size_t* bytes) {
     if (!s || !bytes) return fail(PLB_ERR_INVALID_ARGUMENT, "null argument");
     size_t b = (s->aa ? 1 : 2) * s->pstride * s->q * s->sbytes;
     if (s->mode == PLB_MODE_LITERAL)
-        b += 4 * s->ncell * s->sbytes;
+        b += 4 * lit_cells(s) * s->sbytes;
     else
         b += 4 * s->ncell * sizeof(double) + s->ncell + (s->nbmask ? 4 * s->ncell : 0);
     *bytes = b + s->scratch_bytes;
@@ -517,7 +539,7 @@ int plb_stream(plb_state* s, const char* stream_type) {
         const plb_boundary* per = q[0].kind == kLitPeriodic ? &q[0].bc : nullptr;
         const LitOp* r = &c - 2;
         return timed(s, PLB_STAGE_COLLIDE, [&] {
-            return lit_moments_collide_push(s, c.tau, c.force, per, &r[0].bc, &r[1].bc, nullptr, true);
+            return lit_moments_collide_push(s, c.tau, c.force, per, &r[0].bc, &r[1].bc, nullptr, false);
         });
     }
     // every other request finds the deferred calls done, as the reference's does
@@ -556,7 +578,7 @@ int plb_apply_noslip(plb_state* s, const plb_boundary* bc) {
     int rc = s && s->mode == PLB_MODE_LITERAL ? enter(s) : enter_keep(s);
     if (rc) return rc;
     if (!bc) return fail(PLB_ERR_INVALID_ARGUMENT, "null boundary");
-    if (s->mode == PLB_MODE_LITERAL) return timed(s, PLB_STAGE_NOSLIP, [&] { return lit_noslip(s, bc); });
+    if (s->mode == PLB_MODE_LITERAL) return timed(s, PLB_STAGE_NOSLIP, [&] { return lit_noslip(s, bc, true); });
     // folded into the fused kernel; the boundary must be the one it uses
     for (int f = 0; f < 6; ++f)
         if (bc->type[f] == kNoslip && !bc->has_vel[f])
@@ -679,7 +701,7 @@ int plb_step(plb_state* s, int nsteps) {
             const bool fold = s->tune_lit_fuse != 0;
             if (fold && i > 0) {
                 if ((rc = timed(s, PLB_STAGE_COLLIDE,
-                                [&] { return lit_moments_collide_push(s, s->tau, F, bc, bc, bc, bc, i + 1 == nsteps); })))
+                                [&] { return lit_moments_collide_push(s, s->tau, F, bc, bc, bc, bc, i + 1 < nsteps); })))
                     return rc;
             } else if (fold) {
                 if ((rc = timed(s, PLB_STAGE_COLLIDE, [&] { return lit_collide_push(s, s->tau, F); })))
@@ -688,7 +710,8 @@ int plb_step(plb_state* s, int nsteps) {
                 if ((rc = timed(s, PLB_STAGE_COLLIDE, [&] { return lit_collide(s, s->tau, F); }))) return rc;
                 if ((rc = timed(s, PLB_STAGE_STREAM, [&] { return lit_push(s); }))) return rc;
             }
-            if ((rc = timed(s, PLB_STAGE_NOSLIP, [&] { return lit_noslip(s, bc); }))) return rc;
+            if ((rc = timed(s, PLB_STAGE_NOSLIP, [&] { return lit_noslip(s, bc, !fold || i + 1 == nsteps); })))
+                return rc;
             if (fold && i + 1 < nsteps) continue;
             if ((rc = timed(s, PLB_STAGE_PERIODIC, [&] { return lit_periodic(s, bc); }))) return rc;
             if (fold) {

@@ -1,6 +1,6 @@
 // Literal mode: the reference's staged step (PLBPD.cpp:23-30), one kernel per
-// reference operator, on halo'd structure-of-arrays buffers:
-//   n[k * ncell + c],  c = (z*(Y+2) + y)*(X+2) + x,  x in [0, X+1] etc.
+// reference operator, on halo'd structure-of-arrays buffers: rho[c], u[i * ncell
+// + c] and n[at(k) + c], c = (z*(Y+2) + y)*nx + x, x in [0, X+1] etc. (LitDims).
 // A collision and the push after it can run as one kernel (k_collide_push),
 // which can also take the previous step's moments and resets
 // (k_moments_collide_push); every buffer ends as after the separate kernels.
@@ -18,12 +18,36 @@ namespace {
 
 constexpr unsigned kThreads = 256;
 
+// Device layout.  Population k of cell c lies at at(k) + c, at(k) = k * ps +
+// base - (c_kx * sx + c_ky * sy + c_kz * sz).  With (sx, sy, sz) = (1, nx, nx * ny)
+// the slot (x + c_k, k), which a push from cell x fills, lies at x's own place
+// in array k, so that a wavefront of the collide+push kernels writes the same
+// cells of every array: whole lines, as rows start on a line (nx and ps whole
+// lines, base such that x = 1 begins one); its reads of (x, k) are shifted
+// instead, by a cell along the row at most, and a line that two wavefronts read
+// is in the cache.  With (0, 0, 0), base 0 and nx = X + 2 (lit_layout's packed
+// form) a slot lies at its own cell, and the pushes' stores share lines.
 struct LitDims {
     int X, Y, Z;
-    int nx, ny;      // X+2, Y+2
-    uint64_t ncell;  // (X+2)(Y+2)(Z+2)
+    int nx, ny;         // cells from row to row (X + 2 or more), Y + 2
+    uint64_t ncell;     // nx * ny * (Z + 2)
+    uint64_t ps, base;  // elements between the population arrays, and before the first
+    int64_t sx, sy, sz;
     __host__ __device__ uint64_t cell(int z, int y, int x) const {
         return ((uint64_t)z * ny + y) * nx + x;
+    }
+    __host__ __device__ int64_t at(int k, int cx, int cy, int cz) const {
+        return (int64_t)(k * ps + base) - (cx * sx + cy * sy + cz * sz);
+    }
+    template <int Q>
+    __device__ int64_t at(int k) const {
+        return at(k, Lat<Q>::cx(k), Lat<Q>::cy(k), Lat<Q>::cz(k));
+    }
+    // where a push from cell c puts population k, less c: the slot of c + c_k
+    template <int Q>
+    __device__ int64_t to(int k) const {
+        const int cx = Lat<Q>::cx(k), cy = Lat<Q>::cy(k), cz = Lat<Q>::cz(k);
+        return at(k, cx, cy, cz) + cx + (int64_t)cy * nx + (int64_t)cz * nx * ny;
     }
 };
 
@@ -32,9 +56,15 @@ LitDims dims_of(const plb_state* s) {
     d.X = s->X;
     d.Y = s->Y;
     d.Z = s->Z;
-    d.nx = s->X + 2;
+    d.nx = s->lit_nx;
     d.ny = s->Y + 2;
-    d.ncell = s->ncell;
+    d.ncell = lit_cells(s);
+    d.ps = s->pstride;
+    d.base = s->lit_base;
+    const int64_t on = s->lit_base != 0;
+    d.sx = on;
+    d.sy = on * d.nx;
+    d.sz = on * d.nx * d.ny;
     return d;
 }
 
@@ -68,6 +98,7 @@ __global__ void k_init(LitDims g, R* n, R* ntmp, R* rho, R* u, double rho0, doub
     const int x = (int)(c % g.nx);
     const int y = (int)((c / g.nx) % g.ny);
     const int z = (int)(c / ((uint64_t)g.nx * g.ny));
+    if (x > g.X + 1) return;
     const int xi = (x - 1 + g.X) % g.X, yi = (y - 1 + g.Y) % g.Y, zi = (z - 1 + g.Z) % g.Z;
     const double u0[3] = {u0x, u0y, u0z};
     double uc[3];
@@ -79,8 +110,8 @@ __global__ void k_init(LitDims g, R* n, R* ntmp, R* rho, R* u, double rho0, doub
     const R usq = ur[0] * ur[0] + ur[1] * ur[1] + ur[2] * ur[2];
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
-        n[k * g.ncell + c] = feq_ref<Q, R>(k, r0, ur, usq);
-        ntmp[k * g.ncell + c] = (R)0;
+        n[g.at<Q>(k) + (int64_t)c] = feq_ref<Q, R>(k, r0, ur, usq);
+        ntmp[g.at<Q>(k) + (int64_t)c] = (R)0;
     }
 }
 
@@ -129,51 +160,54 @@ __global__ void k_collide(LitDims g, R* __restrict__ n, const R* __restrict__ rh
     updated_u(u[c], u[g.ncell + c], u[2 * g.ncell + c], rl, tau, F0, F1, F2, uu, usq);
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
-        R* p = n + k * g.ncell + c;
+        R* p = n + g.at<Q>(k) + c;
         *p = collide_value<Q, R>(k, *p, rl, uu, usq, om, omm);
     }
 }
 
-// Whether interior cell (x, y, z) lies on the outer interior layer (a face
-// layer of Boundary.cpp:113-148 on any axis).  The collide+push kernels store
-// their in-place post-collision values only there.  Off that layer, the
-// value the reference leaves in place (it becomes ntmp after the swap) is
-// the one the same kernel pushed to c + c_k, and nothing reads it before the
-// next push overwrites it: the next push writes ntmp(c', k) for every c' with
-// c' - c_k interior, which is every cell off the outer layer.  Between the
-// two pushes only a read of ntmp or a change of n at those pushed slots
-// (a collision in place, an upload) needs the values, and k_ntmp_restore
-// copies them back from n first.  No-slip and periodic copies never change
-// a slot n(c + c_k, k) of such a cell: no-slip writes n(f + c_kp, kp) for face
-// cells f, periodic copies write n(c', k) with c' - c_k in the halo.
-__device__ inline bool outer_layer(const LitDims& g, int x, int y, int z) {
-    return x == 1 || x == g.X || y == 1 || y == g.Y || z == 1 || z == g.Z;
+// Whether c - c_k of interior cell c lies in the halo: a slot no push writes.
+template <int Q>
+__device__ inline bool from_halo(const LitDims& g, int k, int x, int y, int z) {
+    const int cx = Lat<Q>::cx(k), cy = Lat<Q>::cy(k), cz = Lat<Q>::cz(k);
+    return (cx > 0 && x == 1) || (cx < 0 && x == g.X) || (cy > 0 && y == 1) || (cy < 0 && y == g.Y) ||
+           (cz > 0 && z == 1) || (cz < 0 && z == g.Z);
+}
+// Whether an interior cell lies on one of the faces of the bit mask (face f:
+// the layer at coordinate X|Y|Z, f even, or 1, f odd, of axis f / 2).
+__device__ inline bool on_faces(unsigned faces, const LitDims& g, int x, int y, int z) {
+    return ((faces & 1u) && x == g.X) || ((faces & 2u) && x == 1) || ((faces & 4u) && y == g.Y) ||
+           ((faces & 8u) && y == 1) || ((faces & 16u) && z == g.Z) || ((faces & 32u) && z == 1);
 }
 
-// ntmp(c, k) = n(c + c_k, k) for the interior cells off the outer layer: the
-// in-place values the collide+push kernels did not store (see outer_layer).
+// The post-collision values that the reference leaves in place, ntmp after the
+// swap.  The collide+push kernels store there only the slots (c, k) with
+// c - c_k in the halo, which no push writes and the reference's stage order
+// reads back (Q1).  The next push overwrites every other slot before anything
+// reads it; until then its value is the one the same kernel pushed to
+// n(c + c_k, k), which only a no-slip pass changes, and only for its face cells
+// c (it writes n(f + c_kp, kp) for face cells f; periodic copies write n(c', k)
+// with c' - c_k in the halo): that pass saves what it is about to overwrite
+// (k_noslip).  So k_ntmp_restore can put every value in place, before anything
+// reads ntmp (a download) or changes n (a collision by itself, an upload).
+// On the faces of `saved` the no-slip passes have done so, k = 0 apart.
 template <int Q, class R>
-__global__ void k_ntmp_restore(LitDims g, const R* __restrict__ n, R* __restrict__ t) {
+__global__ void k_ntmp_restore(LitDims g, unsigned saved, const R* __restrict__ n, R* __restrict__ t) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int y = blockIdx.y + 1, z = blockIdx.z + 1;
-    if (x > g.X || outer_layer(g, x, y, z)) return;
+    if (x > g.X) return;
     const uint64_t c = g.cell(z, y, x);
+    const bool done = on_faces(saved, g, x, y, z);
 #pragma unroll
-    for (int k = 0; k < Q; ++k) {
-        const int64_t off = (int64_t)Lat<Q>::cx(k) + (int64_t)Lat<Q>::cy(k) * g.nx +
-                            (int64_t)Lat<Q>::cz(k) * g.nx * g.ny;
-        t[k * g.ncell + c] = n[k * g.ncell + (uint64_t)((int64_t)c + off)];
-    }
+    for (int k = 0; k < Q; ++k)
+        if ((k == 0 || !done) && !from_halo<Q>(g, k, x, y, z))
+            t[g.at<Q>(k) + (int64_t)c] = n[g.to<Q>(k) + (int64_t)c];
 }
 
 // The collision followed by Streaming::_push_kernel (Streaming.cpp:63-74) in
 // one pass: each post-collision value is stored at x + c_k in t, as k_push
-// copies it, and in place on the outer layer, as k_collide leaves it (it
-// becomes ntmp after the swap; the next push leaves those entries, and the
-// reference's stage order reads some of them back, Q1).  Every value a caller
-// or a later stage can read equals the one k_collide then k_push give (see
-// outer_layer); the push's re-read of n and the in-place stores off the outer
-// layer are saved.
+// copies it, and in place where no push will write (see k_ntmp_restore).  Every
+// value a caller or a later stage can read equals the one k_collide then
+// k_push give; the push's re-read of n and most in-place stores are saved.
 template <int Q, class R>
 __global__ void k_collide_push(LitDims g, R* __restrict__ n, const R* __restrict__ rho,
                                const R* __restrict__ u, R* __restrict__ t, R tau, R om, R omm, R F0, R F1,
@@ -183,16 +217,14 @@ __global__ void k_collide_push(LitDims g, R* __restrict__ n, const R* __restrict
     if (x > g.X) return;
     const uint64_t c = g.cell(z, y, x);
     const R rl = rho[c];
-    const bool keep = outer_layer(g, x, y, z);
     R uu[3], usq;
     updated_u(u[c], u[g.ncell + c], u[2 * g.ncell + c], rl, tau, F0, F1, F2, uu, usq);
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
-        const R v = collide_value<Q, R>(k, n[k * g.ncell + c], rl, uu, usq, om, omm);
-        if (keep) n[k * g.ncell + c] = v;
-        const int64_t off = (int64_t)Lat<Q>::cx(k) + (int64_t)Lat<Q>::cy(k) * g.nx +
-                            (int64_t)Lat<Q>::cz(k) * g.nx * g.ny;
-        t[k * g.ncell + (uint64_t)((int64_t)c + off)] = v;
+        R* p = n + g.at<Q>(k) + c;
+        const R v = collide_value<Q, R>(k, *p, rl, uu, usq, om, omm);
+        if (from_halo<Q>(g, k, x, y, z)) *p = v;
+        t[g.to<Q>(k) + (int64_t)c] = v;
     }
 }
 
@@ -205,9 +237,7 @@ __global__ void k_push(LitDims g, const R* __restrict__ n, R* __restrict__ t) {
     const uint64_t c = g.cell(z, y, x);
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
-        const int64_t off = (int64_t)Lat<Q>::cx(k) + (int64_t)Lat<Q>::cy(k) * g.nx +
-                            (int64_t)Lat<Q>::cz(k) * g.nx * g.ny;
-        t[k * g.ncell + (uint64_t)((int64_t)c + off)] = n[k * g.ncell + c];
+        t[g.to<Q>(k) + (int64_t)c] = n[g.at<Q>(k) + (int64_t)c];
     }
 }
 
@@ -235,6 +265,10 @@ template <class R>
 struct NoslipFaces {
     FaceBox box[2];
     R ub[2][3];
+    // t, if not null: ntmp, in which the values about to be overwritten are
+    // put in place (k_ntmp_restore), but for the faces of `saved`
+    R* t;
+    unsigned saved;
 };
 
 // Boundary::_apply_noslip (Boundary.cpp:189-221) for one face, as the serial
@@ -283,13 +317,20 @@ __global__ void k_noslip(LitDims g, NoslipFaces<R> fs, R* __restrict__ n, const 
     // c_k = -c_kp
     const R cu_k = (R)(-cxp) * ub0 + (R)(-cyp) * ub1 + (R)(-czp) * ub2;
     const R t_y = (R)2 * wk * rho[cy] * cu_k * cs2inv;
-    const R v = n[k * g.ncell + cc];
-    n[kp * g.ncell + cy] = v - t_y;
+    R* const own = n + g.at(k, -cxp, -cyp, -czp) + cc;
+    R* const dst = n + g.at(kp, cxp, cyp, czp) + cy;
+    const R v = *own;
+    if (fs.t) {
+        // (c, kp) was pushed to *dst, and (y, k) to *own
+        if (!on_faces(fs.saved, g, x, y, z)) fs.t[g.at(kp, cxp, cyp, czp) + (int64_t)cc] = *dst;
+        if (in_face && !on_faces(fs.saved, g, yx, yy, yz)) fs.t[g.at(k, -cxp, -cyp, -czp) + (int64_t)cy] = v;
+    }
+    *dst = v - t_y;
     if (in_face) {
         // op (y, k): its own term t(y, c_kp of it = c_k) is t_y, then c's
         const R cu_kp = (R)cxp * ub0 + (R)cyp * ub1 + (R)czp * ub2;
         const R t_c = (R)2 * wk * rho[cc] * cu_kp * cs2inv;
-        n[k * g.ncell + cc] = (v - t_y) - t_c;
+        *own = (v - t_y) - t_c;
     }
 }
 
@@ -316,12 +357,13 @@ template <int Q, class R>
 __global__ void k_periodic(LitDims g, Periodic per, R* __restrict__ n) {
     const int axis = (int)blockIdx.z, k = 1 + (int)blockIdx.y;
     if (axis == 0 ? !per.ew : !per.ns) return;
-    int cx = 0, cy = 0;
+    int cx = 0, cy = 0, cz = 0;
 #pragma unroll
     for (int j = 1; j < Q; ++j)
         if (j == k) {
             cx = Lat<Q>::cx(j);
             cy = Lat<Q>::cy(j);
+            cz = Lat<Q>::cz(j);
         }
     const int ck = axis == 0 ? cx : cy;
     if (ck == 0) return;
@@ -335,7 +377,8 @@ __global__ void k_periodic(LitDims g, Periodic per, R* __restrict__ n) {
     if (axis == 0 && per.ns && ((cy > 0 && a == 1) || (cy < 0 && a == g.Y))) return;
     const uint64_t dst = axis == 0 ? g.cell(z, a, to) : g.cell(z, to, a);
     const uint64_t src = axis == 0 ? g.cell(z, a, from) : g.cell(z, from, a);
-    n[k * g.ncell + dst] = n[k * g.ncell + src];
+    R* const nk = n + g.at(k, cx, cy, cz);
+    nk[dst] = nk[src];
 }
 
 // Where an interior cell finds its population k when the periodic copies are
@@ -343,23 +386,27 @@ __global__ void k_periodic(LitDims g, Periodic per, R* __restrict__ n) {
 // copy that stands would take it from, relative to the cell's own slot (0
 // away from the seams).  The copies read halo slots only, which the folded
 // kernels do not write.
-struct SeamShift {
-    int64_t xp, xm, yp, ym;  // for c_x > 0, c_x < 0, c_y > 0, c_y < 0
+struct Seam {
+    uint32_t xp, xm;  // x from which c_x > 0, c_x < 0 come
+    int64_t yp, ym;   // and the shift of the row (uniform) for c_y > 0, c_y < 0
 };
-__device__ inline SeamShift seam_shift(const LitDims& g, const Periodic& per, int x, int y) {
-    SeamShift s;
-    s.xp = per.ew && x == 1 ? (int64_t)g.X : 0;
-    s.xm = per.ew && x == g.X ? -(int64_t)g.X : 0;
+__device__ inline Seam seam_of(const LitDims& g, const Periodic& per, int x, int y) {
+    Seam s;
+    s.xp = per.ew && x == 1 ? (uint32_t)g.X + 1u : (uint32_t)x;
+    s.xm = per.ew && x == g.X ? 0u : (uint32_t)x;
     s.yp = per.ns && y == 1 ? (int64_t)g.Y * g.nx : 0;
     s.ym = per.ns && y == g.Y ? -(int64_t)g.Y * g.nx : 0;
     return s;
 }
 template <int Q>
-__device__ inline int64_t shift_of(const SeamShift& s, int k) {
-    const int cx = Lat<Q>::cx(k), cy = Lat<Q>::cy(k);
-    const int64_t ox = cx > 0 ? s.xp : (cx < 0 ? s.xm : 0);
-    const int64_t oy = cy > 0 ? s.yp : (cy < 0 ? s.ym : 0);
-    return oy != 0 ? oy : ox;
+__device__ inline int64_t seam_row(const Seam& s, int k) {
+    const int cy = Lat<Q>::cy(k);
+    return cy > 0 ? s.yp : (cy < 0 ? s.ym : 0);
+}
+template <int Q>
+__device__ inline uint32_t seam_x(const Seam& s, int k, uint32_t x) {
+    const int cx = Lat<Q>::cx(k);
+    return cx == 0 || seam_row<Q>(s, k) != 0 ? x : (cx > 0 ? s.xp : s.xm);
 }
 
 // CalcMoments::_get_local_moments (CalcMoments.hpp:22-37): rho = sum_k n_k,
@@ -438,7 +485,7 @@ __global__ void k_moments(LitDims g, const R* __restrict__ n, R* __restrict__ rh
     const uint64_t c = g.cell(z, y, x);
     MomentSum<Q, R> m;
 #pragma unroll
-    for (int k = 0; k < Q; ++k) m.add(k, __builtin_nontemporal_load(n + k * g.ncell + c));
+    for (int k = 0; k < Q; ++k) m.add(k, __builtin_nontemporal_load(n + g.at<Q>(k) + c));
     R rl, um[3];
     m.finish(rl, um);
     apply_resets(fr, g, x, y, z, rl, um);
@@ -454,24 +501,11 @@ __global__ void k_moments(LitDims g, const R* __restrict__ n, R* __restrict__ rh
 // the face layers of the no-slip faces and of the layers next to them.
 struct MomentStores {
     int all;
-    int lo[3], hi[3];  // no-slip on the low / high face of each axis
+    unsigned noslip;  // the no-slip faces, a bit each
 };
-__device__ inline bool near_noslip(const MomentStores& ms, const LitDims& g, int x, int y, int z) {
-    return (ms.lo[0] && x <= 2) || (ms.hi[0] && x >= g.X - 1) || (ms.lo[1] && y <= 2) ||
-           (ms.hi[1] && y >= g.Y - 1) || (ms.lo[2] && z <= 2) || (ms.hi[2] && z >= g.Z - 1);
-}
-
-// Whether the cell lies on a no-slip face.
-__device__ inline bool on_noslip(const MomentStores& ms, const LitDims& g, int x, int y, int z) {
-    return (ms.lo[0] && x == 1) || (ms.hi[0] && x == g.X) || (ms.lo[1] && y == 1) || (ms.hi[1] && y == g.Y) ||
-           (ms.lo[2] && z == 1) || (ms.hi[2] && z == g.Z);
-}
-// Whether c - c_k of interior cell c lies in the halo: a slot no push writes.
-template <int Q>
-__device__ inline bool from_halo(const LitDims& g, int k, int x, int y, int z) {
-    const int cx = Lat<Q>::cx(k), cy = Lat<Q>::cy(k), cz = Lat<Q>::cz(k);
-    return (cx > 0 && x == 1) || (cx < 0 && x == g.X) || (cy > 0 && y == 1) || (cy < 0 && y == g.Y) ||
-           (cz > 0 && z == 1) || (cz < 0 && z == g.Z);
+__device__ inline bool near_noslip(unsigned faces, const LitDims& g, int x, int y, int z) {
+    return ((faces & 1u) && x >= g.X - 1) || ((faces & 2u) && x <= 2) || ((faces & 4u) && y >= g.Y - 1) ||
+           ((faces & 8u) && y <= 2) || ((faces & 16u) && z >= g.Z - 1) || ((faces & 32u) && z <= 2);
 }
 
 // The previous step's periodic copies, moments and resets (Boundary,
@@ -486,84 +520,91 @@ __device__ inline bool from_halo(const LitDims& g, int k, int x, int y, int z) {
 // of plb_step from 252 to 221 us (D3Q19 128^3 FP64: 38 instead of 42 values
 // per cell, two launches fewer) and from 10.6 to 8.1 us (D2Q9 256 x 64 FP64).
 //
-// In-place stores: all of the outer layer where the caller can see ntmp
-// afterwards (keep_all).  Where plb_step goes on with another of these kernels
-// (the same per and no-slip faces, nothing read in between), the push of that
-// step overwrites every slot (c, k) with c - c_k interior before anything
-// reads it, and of the others it reads (c, k) itself only where no periodic
-// copy takes its place, and the no-slip pass only those of its face cells.
+// In-place stores: as in k_collide_push, and fewer still (next_known) where
+// plb_step goes on with another of these kernels, the same per and no-slip
+// faces and nothing read in between: of the slots no push writes, that step
+// reads (c, k) itself only where no periodic copy takes its place, and its
+// no-slip pass only those of its face cells.  All of the outer layer's values
+// in place (38 one-lane stores per row of a lattice periodic in x, each into
+// lines of its own) and stores along c_k cost 191 us per step at 128^3 FP64;
+// the stores that remain, 157; whole lines (LitDims), 136 (FP32 77 -> 72,
+// 256^3 FP64 1,260 -> 1,107, D3Q27 64^3 27.6 -> 24.3): 4.7 TB/s of the 38 values
+// per cell at 128^3, 4.6 at 256^3, bound by memory.
 template <int Q, class R>
 __global__ void k_moments_collide_push(LitDims g, R* __restrict__ n, R* __restrict__ rho, R* __restrict__ u,
                                        R* __restrict__ t, Periodic per, FaceResets<R> fr, MomentStores ms,
-                                       int keep_all, R tau, R om, R omm, R F0, R F1, R F2) {
+                                       int next_known, R tau, R om, R omm, R F0, R F1, R F2) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int y = blockIdx.y + 1, z = blockIdx.z + 1;
     if (x > g.X) return;
     const uint64_t c = g.cell(z, y, x);
-    const SeamShift sh = seam_shift(g, per, x, y);
+    // addresses: a uniform row of the population's array, and x
+    const int64_t row = (int64_t)g.cell(z, y, 0);
+    const Seam sm = seam_of(g, per, x, y);
     R nv[Q];
     MomentSum<Q, R> m;
 #pragma unroll
-    for (int k = 0; k < Q; ++k) {
-        nv[k] = n[k * g.ncell + (uint64_t)((int64_t)c + shift_of<Q>(sh, k))];
-        m.add(k, nv[k]);
-    }
+    for (int k = 0; k < Q; ++k)
+        nv[k] = (n + g.at<Q>(k) + row + seam_row<Q>(sm, k))[seam_x<Q>(sm, k, (uint32_t)x)];
+#pragma unroll
+    for (int k = 0; k < Q; ++k) m.add(k, nv[k]);
     R rl, um[3];
     m.finish(rl, um);
     apply_resets(fr, g, x, y, z, rl, um);
-    if (ms.all || near_noslip(ms, g, x, y, z)) rho[c] = rl;
+    if (ms.all || near_noslip(ms.noslip, g, x, y, z)) rho[c] = rl;
     if (ms.all) {
         u[c] = um[0];
         u[g.ncell + c] = um[1];
         u[2 * g.ncell + c] = um[2];
     }
-    const bool outer = outer_layer(g, x, y, z), all = keep_all && outer, face = on_noslip(ms, g, x, y, z);
     R uu[3], usq;
     updated_u(um[0], um[1], um[2], rl, tau, F0, F1, F2, uu, usq);
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
-        const R v = collide_value<Q, R>(k, nv[k], rl, uu, usq, om, omm);
-        if (all || (outer && from_halo<Q>(g, k, x, y, z) && (face || shift_of<Q>(sh, k) == 0))) n[k * g.ncell + c] = v;
-        const int64_t off = (int64_t)Lat<Q>::cx(k) + (int64_t)Lat<Q>::cy(k) * g.nx +
-                            (int64_t)Lat<Q>::cz(k) * g.nx * g.ny;
-        t[k * g.ncell + (uint64_t)((int64_t)c + off)] = v;
+        nv[k] = collide_value<Q, R>(k, nv[k], rl, uu, usq, om, omm);
+        (t + g.to<Q>(k) + row)[(uint32_t)x] = nv[k];
+    }
+    const bool any = !next_known || on_faces(ms.noslip, g, x, y, z);
+#pragma unroll
+    for (int k = 1; k < Q; ++k) {
+        const bool own = any || (seam_row<Q>(sm, k) == 0 && seam_x<Q>(sm, k, (uint32_t)x) == (uint32_t)x);
+        if (own && from_halo<Q>(g, k, x, y, z)) (n + g.at<Q>(k) + row)[(uint32_t)x] = nv[k];
     }
 }
+
+// Where value v of cell 0 of a field lies.
+struct ValueSlots {
+    int64_t off[27];
+};
 
 // Upload: host AoS -> device SoA with dtype conversion.  compact: host cells
 // are interior only (X*Y*Z); otherwise the full halo'd array.
 template <class H, class R>
-__global__ void k_upload(LitDims g, const H* __restrict__ host, R* __restrict__ dev, int vlen, int compact,
-                         uint64_t total) {
+__global__ void k_upload(LitDims g, const H* __restrict__ host, R* __restrict__ dev, ValueSlots sl, int vlen,
+                         int compact, uint64_t total) {
     for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
          t += (uint64_t)gridDim.x * blockDim.x) {
         const int v = (int)(t % vlen);
         const uint64_t hc = t / vlen;
-        uint64_t c = hc;
-        if (compact) {
-            const int x = (int)(hc % g.X), y = (int)((hc / g.X) % g.Y), z = (int)(hc / ((uint64_t)g.X * g.Y));
-            c = g.cell(z + 1, y + 1, x + 1);
-        }
-        dev[v * g.ncell + c] = (R)host[t];
+        const int o = compact ? 1 : 0, X = g.X + 2 - 2 * o, Y = g.ny - 2 * o;
+        const int x = (int)(hc % X), y = (int)((hc / X) % Y), z = (int)(hc / ((uint64_t)X * Y));
+        dev[sl.off[v] + (int64_t)g.cell(z + o, y + o, x + o)] = (R)host[t];
     }
 }
 
-// Download: value v of cell c of the full halo'd array, or of the interior.
+// Download: value v of cell c of the full halo'd array (o = 0), or of the
+// interior (o = 1).
 template <class R>
-struct GetFull {
-    const R* dev;
-    uint64_t ncell;
-    __device__ R operator()(uint64_t c, uint32_t v) const { return dev[v * ncell + c]; }
-};
-template <class R>
-struct GetInterior {
+struct GetValue {
     const R* dev;
     LitDims g;
-    FastDiv dX, dY;  // an interior of 2^32 cells is part of a state larger than any device
+    ValueSlots sl;
+    FastDiv dX, dY;  // a row, a column of 2^32 cells in all is part of a state larger than any device
+    int o;
     __device__ R operator()(uint64_t c, uint32_t v) const {
         const uint32_t row = fdiv((uint32_t)c, dX), z = fdiv(row, dY);
         const int x = (int)((uint32_t)c - row * dX.d), y = (int)(row - z * dY.d);
-        return dev[v * g.ncell + g.cell((int)z + 1, y + 1, x + 1)];
+        return dev[sl.off[v] + (int64_t)g.cell((int)z + o, y + o, x + o)];
     }
 };
 
@@ -624,8 +665,7 @@ dim3 interior_grid(const plb_state* s) {
     return dim3((unsigned)((s->X + b - 1) / b), (unsigned)s->Y, (unsigned)s->Z);
 }
 
-// Stores the in-place values the last collide+push kernel left out (see
-// outer_layer), before anything reads ntmp or changes n.
+// Stores the in-place values the last collide+push kernel left out, before anything reads ntmp or changes n.
 int lit_ntmp_restore(plb_state* s) {
     if (!s->lit_ntmp_folded) return PLB_OK;
     const LitDims g = dims_of(s);
@@ -633,7 +673,7 @@ int lit_ntmp_restore(plb_state* s) {
         constexpr int Q = decltype(qc)::value;
         using R = decltype(rr);
         hipLaunchKernelGGL((k_ntmp_restore<Q, R>), interior_grid(s), dim3(interior_block(s)), 0, s->stream, g,
-                           (const R*)s->buf[s->cur], (R*)s->buf[s->cur ^ 1]);
+                           s->lit_saved, (const R*)s->buf[s->cur], (R*)s->buf[s->cur ^ 1]);
         PLB_HIP_TRY(hipGetLastError());
         return PLB_OK;
     });
@@ -644,6 +684,26 @@ int lit_ntmp_restore(plb_state* s) {
 }  // namespace
 
 // ------------------------------------------------------------ launchers ----
+// Device layout of a state (LitDims).  Rows of whole lines take up to an
+// eighth more memory for the pitch (where it would be more, only buffers below
+// 1 GiB get it), and two planes for the shift.  packed: the smallest form.
+void lit_layout(plb_state* s, bool packed) {
+    const uint64_t line = 128 / s->sbytes, X2 = (uint64_t)s->X + 2, ny = (uint64_t)s->Y + 2, nz = (uint64_t)s->Z + 2;
+    uint64_t nx = (X2 + line - 1) / line * line;
+    if (nx * 8 > X2 * 9 && nx * ny * nz * s->q * s->sbytes > (1ull << 30)) nx = X2;
+    if (packed) {
+        s->lit_nx = (int)X2;
+        s->lit_base = 0;
+        s->pstride = X2 * ny * nz;
+        return;
+    }
+    const uint64_t far = nx * ny + nx + 1;  // of a direction's shift
+    s->lit_nx = (int)nx;
+    s->lit_base = (far + line - 1) / line * line + line - 1;
+    s->pstride = (s->lit_base + nx * ny * nz + far + line - 1) / line * line;
+}
+uint64_t lit_cells(const plb_state* s) { return (uint64_t)s->lit_nx * (s->Y + 2) * (s->Z + 2); }
+
 int lit_initialize(plb_state* s, double rho0, const double u0[3], const plb_init_spec* init,
                    const double* tg_dev) {
     const LitDims g = dims_of(s);
@@ -708,6 +768,7 @@ int lit_collide_push(plb_state* s, double tau, const double F[3]) {
     if (rc == PLB_OK) {
         s->cur ^= 1;  // std::swap(simdata.ntmp, simdata.n)
         s->lit_ntmp_folded = true;
+        s->lit_saved = 0;
     }
     return rc;
 }
@@ -729,7 +790,7 @@ FaceResets<R> face_resets(const plb_boundary* bc_vel, const plb_boundary* bc_rho
 
 int lit_moments_collide_push(plb_state* s, double tau, const double F[3], const plb_boundary* bc_per,
                              const plb_boundary* bc_vel, const plb_boundary* bc_rho, const plb_boundary* bc_noslip,
-                             bool keep_all) {
+                             bool next_known) {
     const LitDims g = dims_of(s);
     const int rc = with_qr(s, [&](auto qc, auto rr) {
         constexpr int Q = decltype(qc)::value;
@@ -739,19 +800,18 @@ int lit_moments_collide_push(plb_state* s, double tau, const double F[3], const 
         const Periodic per = bc_per ? periodic_of(bc_per) : Periodic{0, 0};
         MomentStores ms;
         ms.all = bc_noslip == nullptr;
-        for (int a = 0; a < 3; ++a) {
-            ms.hi[a] = bc_noslip && bc_noslip->type[2 * a] == kNoslip;
-            ms.lo[a] = bc_noslip && bc_noslip->type[2 * a + 1] == kNoslip;
-        }
+        ms.noslip = 0;
+        for (int f = 0; bc_noslip && f < 6; ++f) ms.noslip |= bc_noslip->type[f] == kNoslip ? 1u << f : 0u;
         hipLaunchKernelGGL((k_moments_collide_push<Q, R>), interior_grid(s), dim3(interior_block(s)), 0, s->stream,
                            g, (R*)s->buf[s->cur], (R*)s->rho, (R*)s->u, (R*)s->buf[s->cur ^ 1], per,
-                           face_resets<R>(bc_vel, bc_rho), ms, keep_all ? 1 : 0, tr, om, omm, (R)F[0], (R)F[1], (R)F[2]);
+                           face_resets<R>(bc_vel, bc_rho), ms, next_known ? 1 : 0, tr, om, omm, (R)F[0], (R)F[1], (R)F[2]);
         PLB_HIP_TRY(hipGetLastError());
         return PLB_OK;
     });
     if (rc == PLB_OK) {
         s->cur ^= 1;  // std::swap(simdata.ntmp, simdata.n)
         s->lit_ntmp_folded = true;
+        s->lit_saved = 0;
     }
     return rc;
 }
@@ -768,12 +828,12 @@ int lit_push(plb_state* s) {
     });
     if (rc == PLB_OK) {
         s->cur ^= 1;  // std::swap(simdata.ntmp, simdata.n)
-        s->lit_ntmp_folded = false;  // the push wrote every cell off the outer layer
+        s->lit_ntmp_folded = false;  // the push wrote every slot that was not in place
     }
     return rc;
 }
 
-int lit_noslip(plb_state* s, const plb_boundary* bc) {
+int lit_noslip(plb_state* s, const plb_boundary* bc, bool ntmp_read) {
     const LitDims g = dims_of(s);
     const int dims[3] = {s->X, s->Y, s->Z};
     for (int f = 0; f < 6;) {
@@ -789,6 +849,7 @@ int lit_noslip(plb_state* s, const plb_boundary* bc) {
         // with two layers each would write into the layer the other reads.
         const bool both = f % 2 == 0 && bc->type[f + 1] == kNoslip && bc->has_vel[f + 1] && dims[f / 2] >= 3;
         const int nf = both ? 2 : 1;
+        const bool save = s->lit_ntmp_folded && ntmp_read;
         const int rc = with_qr(s, [&](auto qc, auto rr) {
             constexpr int Q = decltype(qc)::value;
             using R = decltype(rr);
@@ -798,6 +859,8 @@ int lit_noslip(plb_state* s, const plb_boundary* bc) {
                 fs.box[i] = face_box(fi, s->X, s->Y, s->Z);
                 for (int d = 0; d < 3; ++d) fs.ub[i][d] = (R)bc->vel[fi][d];
             }
+            fs.t = save ? (R*)s->buf[s->cur ^ 1] : nullptr;
+            fs.saved = s->lit_saved;
             // a face of 2^32 cells is part of a state larger than any device
             const uint32_t total = (uint32_t)fs.box[0].count();
             const R cs2inv = (R)1 / (R)(1.0 / 3.0);
@@ -808,6 +871,7 @@ int lit_noslip(plb_state* s, const plb_boundary* bc) {
             return PLB_OK;
         });
         if (rc) return rc;
+        for (int i = 0; save && i < nf; ++i) s->lit_saved |= 1u << (f + i);
         f += nf;
     }
     return PLB_OK;
@@ -825,7 +889,7 @@ int lit_noslip_noalloc(plb_state* s, const plb_boundary* bc) {
                                                       " bytes exceeds the no-allocation limit of 16 MiB; use "
                                                       "plb_apply_noslip");
     }
-    return lit_noslip(s, bc);
+    return lit_noslip(s, bc, true);
 }
 
 int lit_periodic(plb_state* s, const plb_boundary* bc) {
@@ -906,7 +970,16 @@ int lit_transfer(plb_state* s, int field, int layout, int dtype, void* host, boo
         case PLB_FIELD_NTMP: vlen = s->q; dev = s->buf[s->cur ^ 1]; break;
         default: return fail(PLB_ERR_INVALID_ARGUMENT, "unknown field");
     }
-    const int compact = layout == PLB_LAYOUT_COMPACT;
+    ValueSlots sl;
+    const bool pop = field == PLB_FIELD_N || field == PLB_FIELD_NTMP;
+    const int slots = with_q(s->q, [&](auto qc) {
+        using L = Lat<decltype(qc)::value>;
+        for (int v = 0; v < vlen; ++v)
+            sl.off[v] = pop ? g.at(v, L::cx(v), L::cy(v), L::cz(v)) : (int64_t)(v * g.ncell);
+        return PLB_OK;
+    });
+    if (slots) return slots;
+    const int compact = layout == PLB_LAYOUT_COMPACT ? 1 : 0;
     const uint64_t cells = compact ? (uint64_t)s->X * s->Y * s->Z : s->ncell;
     const uint64_t total = cells * vlen;
     if (!upload) {
@@ -915,13 +988,12 @@ int lit_transfer(plb_state* s, int field, int layout, int dtype, void* host, boo
             auto read = [&](auto hh) {
                 using H = decltype(hh);
                 const size_t cell_bytes = vlen * sizeof(H);
-                const GetInterior<R> gi{(const R*)dev, g, make_fastdiv((uint32_t)s->X), make_fastdiv((uint32_t)s->Y)};
-                const GetFull<R> gf{(const R*)dev, g.ncell};
+                const GetValue<R> get{(const R*)dev, g, sl, make_fastdiv((uint32_t)(s->X + 2 - 2 * compact)),
+                                      make_fastdiv((uint32_t)(s->Y + 2 - 2 * compact)), compact};
                 return host_read(
                     s->ring, s->device, s->stream, cells, cell_bytes,
                     [&](uint64_t first, uint64_t n, void* slot) {
-                        return compact ? host_fill<H>(gi, first, n, vlen, slot, s->stream)
-                                       : host_fill<H>(gf, first, n, vlen, slot, s->stream);
+                        return host_fill<H>(get, first, n, vlen, slot, s->stream);
                     },
                     [&](uint64_t first, uint64_t n, const void* slot) {
                         std::memcpy((char*)host + first * cell_bytes, slot, n * cell_bytes);
@@ -941,11 +1013,11 @@ int lit_transfer(plb_state* s, int field, int layout, int dtype, void* host, boo
             using R = decltype(rr);
             if (dtype == PLB_DTYPE_F64)
                 hipLaunchKernelGGL((k_upload<double, R>), dim3(stride_blocks(total, kThreads)),
-                                   dim3(kThreads), 0, s->stream, g, (const double*)stage, (R*)dev, vlen,
+                                   dim3(kThreads), 0, s->stream, g, (const double*)stage, (R*)dev, sl, vlen,
                                    compact, total);
             else
                 hipLaunchKernelGGL((k_upload<float, R>), dim3(stride_blocks(total, kThreads)),
-                                   dim3(kThreads), 0, s->stream, g, (const float*)stage, (R*)dev, vlen,
+                                   dim3(kThreads), 0, s->stream, g, (const float*)stage, (R*)dev, sl, vlen,
                                    compact, total);
             PLB_HIP_TRY(hipGetLastError());
             return PLB_OK;

@@ -65,6 +65,8 @@ struct plb_state {
     int variant, mode, device;
     size_t ncell;    // literal: halo'd cells; fused: compact cells
     size_t pstride;  // elements between population arrays
+    int lit_nx;       // literal: cells from row to row on the device
+    size_t lit_base;  // literal: elements before the first population array (0: the packed layout)
     size_t sbytes;   // bytes per stored population value
     void* buf[2];    // population buffers
     int cur;         // buf[cur] holds n (SimData::n), buf[cur ^ 1] ntmp
@@ -89,9 +91,12 @@ struct plb_state {
     // and collide, in that order, each of the first four directly after the
     // one before it); any other call runs them first, in order
     std::vector<plb::LitOp> lit_queue;
-    // literal: the last collide+push kernel stored its in-place values on the
-    // outer layer only; ntmp off that layer is n(c + c_k, k) until restored
+    // literal: the last collide+push kernel stored in place only the slots no
+    // push writes; the rest of ntmp is n(c + c_k, k) until restored, but for
+    // the cells of the faces in lit_saved (a bit each), which a no-slip pass put
+    // in place before it changed n
     bool lit_ntmp_folded;
+    unsigned lit_saved;
     bool moments_valid;
     void* scratch;  // reductions
     size_t scratch_bytes;
@@ -150,6 +155,10 @@ int fused_multi_steps(const plb_state* s);
 int fused_launch_multi(plb_state* s, int steps);
 
 // literal mode (literal.hip)
+// The device layout of a literal state: rows of whole lines, or packed.
+void lit_layout(plb_state* s, bool packed);
+// Cells per moment field on the device.
+uint64_t lit_cells(const plb_state* s);
 int lit_initialize(plb_state* s, double rho0, const double u0[3], const plb_init_spec* init,
                    const double* tg_dev);
 int lit_collide(plb_state* s, double tau, const double F[3]);
@@ -158,12 +167,13 @@ int lit_collide_push(plb_state* s, double tau, const double F[3]);
 // bc_per: the periodic copies folded in (null: none); bc_vel: the faces whose
 // velocity is reset; bc_rho: those whose density is; bc_noslip: the no-slip
 // faces of this step, when nothing else reads rho or u before the next
-// moments (null: every rho and u is stored); keep_all: ntmp can be seen after
-// this step (else another of these calls with the same boundary follows)
+// moments (null: every rho and u is stored); next_known: another of these
+// calls with the same boundary follows, and ntmp is not seen before
 int lit_moments_collide_push(plb_state* s, double tau, const double F[3], const plb_boundary* bc_per,
                              const plb_boundary* bc_vel, const plb_boundary* bc_rho, const plb_boundary* bc_noslip,
-                             bool keep_all);
-int lit_noslip(plb_state* s, const plb_boundary* bc);
+                             bool next_known);
+// ntmp_read: ntmp can be seen before the next push.
+int lit_noslip(plb_state* s, const plb_boundary* bc, bool ntmp_read);
 // The same pass for faces within the documented size limit of the entry point.
 int lit_noslip_noalloc(plb_state* s, const plb_boundary* bc);
 int lit_periodic(plb_state* s, const plb_boundary* bc);

@@ -110,3 +110,35 @@ def test_step_keeps_what_the_next_step_reads(orc, q, X, Y, Z, faces):
             orc.lit_run(o, 0.75, (1e-4, 0.0, -2e-5), ob, n)
             st.step(n)
             _same(st, o, n)
+
+
+@pytest.mark.parametrize("q,X,Y,Z", [(9, 20, 1, 2), (9, 5, 1, 1), (19, 6, 5, 4), (19, 2, 1, 3), (19, 66, 2, 2),
+                                     (27, 3, 4, 1)])
+@pytest.mark.parametrize("passes", [["UUUUNN"], ["NNUUNN", "UUNNUU"], ["UUUUNU", "UUUUNN", "NNNNNN"],
+                                    ["UNNUUU", "UNNUUU"], ["PPUUNN", "UUPPNU"]])
+def test_noslip_passes_save_what_they_overwrite(orc, q, X, Y, Z, passes):
+    """The values a collision leaves in place, read after one and more no-slip
+    passes over the same and other faces, and after the collision or push that
+    follows them."""
+    bcs = []
+    for faces in passes:
+        types = [{"P": PERIODIC, "N": NOSLIP, "U": UNSET}[f] for f in faces]
+        bcs.append(_bc(types, {f: (0.01 * (f + 1), -0.005 * f, 0.004) for f in range(6) if types[f] == NOSLIP}))
+    tau, F = 0.7, (1e-4, -2e-5, 3e-5)
+    for end in range(len(passes) + 2):
+        print(f"\n[case] literal no-slip passes q={q} {X}x{Y}x{Z} {passes} end {end}", flush=True)
+        o = orc.lit_state(q, X, Y, Z)
+        orc.lit_init(o, 1.0, (0.01, 0.0, 0.0), (P.INIT_PERTURBED, 17, 1e-2), bcs[0][0])
+        with P.State(q, X, Y, Z, "f64", P.LITERAL) as st:
+            st.initialize(1.0, (0.01, 0.0, 0.0), (P.INIT_PERTURBED, 17, 1e-2), bcs[0][1])
+            for _ in range(2):
+                orc.lit_collide(o, tau, F), st.collide(tau, F)
+                orc.lit_push(o), st.stream("push")
+                for i, (ob, pb) in enumerate(bcs):
+                    if i < end:
+                        orc.lit_noslip(o, ob), st.apply_noslip(pb)
+                        orc.lit_periodic(o, ob), st.apply_periodicity(pb)
+            if end > len(passes):
+                orc.lit_collide(o, tau, F), st.collide(tau, F)
+                st.synchronize()
+            _same(st, o, end)
