@@ -274,7 +274,9 @@ int plb_bench_pattern(int device, int q, int x, int y, int z, int sbytes, int ve
                             /* are ordinary (its shifted lines are shared with   */
                             /* the next wavefront); the row pull kernel's are    */
                             /* non-temporal without interior solids.            */
-#define PLB_TUNE_NT_STORE 2 /* non-temporal population stores (0/1; default 1) */
+#define PLB_TUNE_NT_STORE 2 /* non-temporal population stores (0/1; default 1); */
+                            /* the two-step kernel's and, on rows of no whole    */
+                            /* lines, the cell kernels' are ordinary             */
 #define PLB_TUNE_SCHEME 3   /* streaming scheme of the fused step:              */
 #define PLB_SCHEME_AUTO 0   /*   pull (default; moving walls included)         */
 #define PLB_SCHEME_PUSH 1   /*   collide, then scatter to neighbours            */
@@ -304,9 +306,9 @@ int plb_bench_pattern(int device, int q, int x, int y, int z, int sbytes, int ve
                               /* otherwise (default) each XCD takes one of eight  */
                               /* contiguous runs of its (z-chunk, y-tile) pairs   */
 #define PLB_TUNE_INDEX64 7    /* 1: the cell kernels' 64-bit index instantiations, and */
-                              /* the two-step kernel's per-population base pointers,   */
-                              /* even where 32-bit byte offsets fit (they run by       */
-                              /* themselves for buffers over 4 GiB); default 0         */
+                              /* the two-step kernel's form for arrays beyond one      */
+                              /* 4 GiB buffer, even where 32-bit byte offsets fit      */
+                              /* (they run by themselves where they do not); default 0 */
 #define PLB_TUNE_LITERAL_FUSE 8 /* literal mode: 1 (default) runs a collision and the */
                                 /* push that follows it as one kernel (same values in */
                                 /* n and ntmp, one pass fewer over n), and does each  */

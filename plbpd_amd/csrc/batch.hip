@@ -459,8 +459,9 @@ int batch_layout(plb_batch* b, int tile) {
 // Two steps per launch from 2^18 cells on, unless the grown borders (domains a
 // few layers thin) cost more than the saved pass: the rule of
 // fused_two_eligible.  512 domains of edges 16 to 96 (44.8 M cells, D3Q19
-// FP32-shifted): 1,162 -> 881 us per step (FP64 2,570 -> 1,628, FP16-shifted
-// 792 -> 673); 64 domains (6.1 M) 160 -> 140, 16 (1.1 M) 28.9 -> 28.6 (FP64 59
+// FP32-shifted): one step per launch 1,162 us per step, two 881, and 830 since
+// the kernel's steps run straight through (FP64 2,570 and 1,628, FP16-shifted
+// 792 and 673 before that); 64 domains (6.1 M) 160 -> 140, 16 (1.1 M) 28.9 -> 28.6 (FP64 59
 // -> 48).
 int two_step_plan(plb_batch* b, int ncu) {
     b->ntwo = 0;

@@ -429,9 +429,14 @@ __host__ __device__ constexpr uint32_t two_blocks(const TwoGeom& g) {
 // more per group would let the step t + 1 cells of the next plane be written
 // while the step t + 2 cells of this one are read, with one workgroup barrier
 // per plane instead of two; for D3Q19 FP32-shifted its 64 x 7 tiles ran 354 /
-// 309 us per step at 256^3 with solids / walls only, against 341 / 288 for
-// two barriers and 64 x 8 tiles.)
-template <int Q>
+// 309 us per step at 256^3 with solids / walls only, when two barriers and
+// 64 x 8 tiles took 341 / 288.)
+//
+// HOLD: a step t + 2 cell takes what it reads of its own plane and the one
+// below as soon as its plane is in the ring, and holds it in registers (14 of
+// D3Q19's 19 values, 18 of D3Q27's 27) until the plane above is there: the
+// c_z = +1 group then keeps two planes, the others one.
+template <int Q, bool HOLD>
 struct ZRing {
     __host__ __device__ static constexpr int grp(int k) {
         return Lat<Q>::cz(k) > 0 ? 0 : (Lat<Q>::cz(k) == 0 ? 1 : 2);
@@ -446,17 +451,31 @@ struct ZRing {
         for (int j = 0; j < k; ++j) n += grp(j) == grp(k);
         return n;
     }
-    __host__ __device__ static constexpr int slots(int g) { return g == 0 ? 3 : 2; }
+    __host__ __device__ static constexpr int slots(int g) { return (g == 0 ? 3 : 2) - (HOLD ? 1 : 0); }
     __host__ __device__ static constexpr int base(int g) {
         int b = 0;
         for (int h = 0; h < g; ++h) b += size(h) * slots(h);
         return b;
     }
-    // population planes the ring holds per cell (43 for D3Q19, 63 for D3Q27)
+    // population planes the ring holds per cell (43 or 24 for D3Q19, 63 or 36 for D3Q27)
     __host__ __device__ static constexpr int planes() { return base(3); }
 };
-__host__ __device__ constexpr int zring_planes(int q) {
-    return q == 19 ? ZRing<19>::planes() : (q == 27 ? ZRing<27>::planes() : (q == 9 ? ZRing<9>::planes() : 0));
+// Whether the two-step kernel holds (ZRing): for 8-byte storage, whose tiles
+// the LDS limits (D3Q19 32 x 11 -> 32 x 13 cells, D3Q27 32 x 7 -> 32 x 13), and
+// D3Q27 in 4-byte storage.  Per step, three planes kept / held: D3Q19 FP64 256^3
+// 636 / 594 us with solids, 553 / 515 walls only, 250 x 191 x 133 270 / 199;
+// D3Q27 FP64 256^3 1,007 / 800, 384^3 3,457 / 2,828; D3Q27 FP32-shifted 256^3
+// 467 / 442 (solids 579 / 518), 384^3 1,560 / 1,486.  D3Q19 in 4-byte storage,
+// whose tiles the registers limit, was 1% faster at 256^3 and 13% slower at 250
+// x 191 x 133; 2-byte storage the same (and D3Q27 spilled).
+__host__ __device__ constexpr bool two_hold(int q, int sbytes) { return sbytes == 8 || (q == 27 && sbytes == 4); }
+// Bytes of LDS per cell: the ring's planes, and the masks of two planes or one.
+__host__ __device__ constexpr int two_lds(int q, int sbytes) {
+    const bool h = two_hold(q, sbytes);
+    const int planes = q == 19 ? (h ? ZRing<19, true>::planes() : ZRing<19, false>::planes())
+                               : (q == 27 ? (h ? ZRing<27, true>::planes() : ZRing<27, false>::planes())
+                                          : ZRing<9, false>::planes());
+    return planes * sbytes + (h ? 4 : 8);
 }
 
 // Cells of a grown tile.
@@ -473,15 +492,18 @@ __host__ __device__ constexpr bool two_split(int q, int sbytes, bool nb) {
 }
 
 // Cells that a grown tile of any shape may have: the ring of that many cells
-// (zring_planes(q) population planes and two 4-byte mask planes) fits the LDS
+// (two_lds(): its population planes and one or two 4-byte mask planes) fits the LDS
 // of a compute unit (160 KiB on gfx950; a workgroup takes all of it), within
 // 1024 threads, one per cell.  The split kernel with 4-byte storage takes at
 // most 704 cells: 64 x 9 tiles (768 threads) ran slower than 64 x 8, and so did
-// 64 x 11 (858 threads in 128 VGPRs: D3Q19 256^3 FP32-shifted 356 / 307
-// against 341 / 288 us per step with solids / walls only).
+// 64 x 11 (858 threads in 128 VGPRs: D3Q19 256^3 FP32-shifted 356 / 307 us
+// per step with solids / walls only, when 64 x 8 took 341 / 288).  8-byte storage
+// takes 512 (256 VGPRs a thread; with 768 threads it spilled: D3Q19 256^3 995
+// against 594 us per step with solids), D3Q27 in 4-byte storage 640 (768: 501
+// against 457 at 256^3 walls only).
 __host__ __device__ constexpr int two_cap(int q, int sbytes) {
-    const int lds = 160 * 1024 / (zring_planes(q) * sbytes + 8);
-    const int maxc = two_split(q, sbytes, true) && sbytes == 4 ? 704 : 1024;
+    const int lds = 160 * 1024 / two_lds(q, sbytes);
+    const int maxc = sbytes == 8 ? 512 : sbytes == 4 ? (q == 27 ? 640 : 704) : 1024;
     if (lds >= maxc) return maxc;
     // one slot more than cells where the last wavefront is cut short (two_slots)
     return sbytes == 8 ? lds / 64 * 64 : lds - 1;
@@ -491,13 +513,14 @@ __host__ __device__ constexpr int two_cap(int q, int sbytes) {
 // fit the LDS, of which such threads share the last.
 __host__ __device__ constexpr int two_threads(int q, int sbytes) { return (two_cap(q, sbytes) + 63) / 64 * 64; }
 __host__ __device__ constexpr int two_slots(int q, int sbytes) {
-    const int lds = 160 * 1024 / (zring_planes(q) * sbytes + 8), t = two_threads(q, sbytes);
+    const int lds = 160 * 1024 / two_lds(q, sbytes), t = two_threads(q, sbytes);
     return t < lds ? t : lds;
 }
 // Rows per tile for a lattice, a storage width and a tile width: the largest
 // BY whose grown tile, (bx + 2) x (BY + 2) cells, is within two_cap(); 0 where
 // no BY >= 3 is.
 __host__ __device__ constexpr int two_rows(int q, int sbytes, int bx) {
+    if (q == 27 && sbytes == 8 && bx > 32) return 0;  // 64 x 5 tiles: more grown cells than 32 x 13
     int best = 0;
     for (int by = 1; by <= 40; ++by)
         if (two_cells(bx, by) <= two_cap(q, sbytes)) best = by;

@@ -12,9 +12,9 @@
 // so none waits for another.  One cell per thread for the whole launch (its
 // neighbour mask and seams stay in registers); the LDS copy has two buffers, so
 // a step needs one barrier.  256 x 64 cells, 200 steps and the read-out: FP64
-// 1,074 -> 377 us; a step takes 1.2 to 1.4 us there, bound by the
-// instructions of the two wavefronts per SIMD and by their latency.  Values pass through the storage type between
-// steps, as they would through memory.
+// 1,074 -> 321 us; a step takes 1.2 to 1.4 us there, bound by the
+// instructions of the two wavefronts per SIMD and by their latency.  Values
+// pass through the storage type between steps, as they would through memory.
 #pragma once
 
 #include "fused_two.hpp"

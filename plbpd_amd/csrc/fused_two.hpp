@@ -147,22 +147,21 @@ __device__ inline void store_own(const typename Prec<V>::T (&f)[Q], const PopBuf
 }
 
 // Ring plane of direction k in its group's slot: element offset of cell 0.
-template <int Q, int K, int NI>
+template <int Q, int K, int NI, bool H>
 __device__ inline uint32_t ring_at(uint32_t slot) {
-    using Z = ZRing<Q>;
+    using Z = ZRing<Q, H>;
     constexpr int g = Z::grp(K);
     return ((uint32_t)Z::base(g) + slot * (uint32_t)Z::size(g) + (uint32_t)Z::idx(K)) * (uint32_t)NI;
 }
 
 // Step t + 1 of a cell into the ring: direction k to its group's slot for
-// this plane (a3 = plane mod 3 for the c_z = +1 group, a2 = plane mod 2 for
-// the others).
-template <int Q, int K, int V, int NI>
+// this plane (up for the c_z = +1 group, fl for the others).
+template <int Q, int K, int V, int NI, bool H>
 __device__ inline void ring_store(const typename Prec<V>::T (&f)[Q], typename Prec<V>::S* ring, uint32_t cell,
-                                  uint32_t a3, uint32_t a2) {
+                                  uint32_t up, uint32_t fl) {
     if constexpr (K < Q) {
-        ring[ring_at<Q, K, NI>(ZRing<Q>::grp(K) == 0 ? a3 : a2) + cell] = Prec<V>::store_raw(f[K]);
-        ring_store<Q, K + 1, V, NI>(f, ring, cell, a3, a2);
+        ring[ring_at<Q, K, NI, H>(ZRing<Q, H>::grp(K) == 0 ? up : fl) + cell] = Prec<V>::store_raw(f[K]);
+        ring_store<Q, K + 1, V, NI, H>(f, ring, cell, up, fl);
     }
 }
 
@@ -171,28 +170,33 @@ __device__ inline void ring_store(const typename Prec<V>::T (&f)[Q], typename Pr
 // rev(k) in plane zo where x - c_k is not fluid.  Slots: pa = the c_z = +1
 // group's slot of plane zo - 1, oa = its slot of plane zo, b0 = the other
 // groups' slot of plane zo, c1 = the c_z = -1 group's slot of plane zo + 1.
-// RX: cells per grown row.
-template <int Q, int K, int V, int NB, int NI>
+// RX: cells per grown row.  P: kAll, or the directions with c_z = -1 (kDown),
+// or the others (kHeld).
+enum : int { kDown = 3, kHeld = 4 };
+template <int Q, int K, int V, int NB, int NI, bool H, int P>
 __device__ inline void ring_gather(typename Prec<V>::T (&f)[Q], const typename Prec<V>::S* ring, uint32_t li,
                                    uint32_t RX, uint32_t pa, uint32_t oa, uint32_t b0, uint32_t c1, uint32_t m,
                                    const Seams<uint32_t>& s) {
     if constexpr (K < Q) {
-        using Z = ZRing<Q>;
+        using Z = ZRing<Q, H>;
         constexpr int R = rev_k<Q>(K);
-        constexpr int cx = Lat<Q>::cx(K), cy = Lat<Q>::cy(K);
+        constexpr int cx = Lat<Q>::cx(K), cy = Lat<Q>::cy(K), cz = Lat<Q>::cz(K);
         constexpr int g = Z::grp(K), gr = Z::grp(R);
-        const uint32_t moved = ring_at<Q, K, NI>(g == 0 ? pa : (g == 1 ? b0 : c1)) + li - ((uint32_t)cx + (uint32_t)cy * RX);
-        const uint32_t own = ring_at<Q, R, NI>(gr == 0 ? oa : b0) + li;
-        if constexpr (NB != 0) {
-            // own - moved is uniform (li cancels) and, like every ring index,
-            // far inside the signed 24-bit range: one 24-bit multiply-add by
-            // the mask bit instead of a compare and a select
-            const int d = __mul24((int)((m >> R) & 1u), (int)(own - moved));
-            f[K] = Prec<V>::load_raw(ring[moved + (uint32_t)d]);
-        } else {
-            f[K] = Prec<V>::load_raw(ring[pull_wall<Q, K>(s) ? own : moved]);
+        if constexpr (P == kAll || (cz < 0) == (P == kDown)) {
+            const uint32_t moved =
+                ring_at<Q, K, NI, H>(g == 0 ? pa : (g == 1 ? b0 : c1)) + li - ((uint32_t)cx + (uint32_t)cy * RX);
+            const uint32_t own = ring_at<Q, R, NI, H>(gr == 0 ? oa : b0) + li;
+            if constexpr (NB != 0) {
+                // own - moved is uniform (li cancels) and, like every ring index,
+                // far inside the signed 24-bit range: one 24-bit multiply-add by
+                // the mask bit instead of a compare and a select
+                const int d = __mul24((int)((m >> R) & 1u), (int)(own - moved));
+                f[K] = Prec<V>::load_raw(ring[moved + (uint32_t)d]);
+            } else {
+                f[K] = Prec<V>::load_raw(ring[pull_wall<Q, K>(s) ? own : moved]);
+            }
         }
-        ring_gather<Q, K + 1, V, NB, NI>(f, ring, li, RX, pa, oa, b0, c1, m, s);
+        ring_gather<Q, K + 1, V, NB, NI, H, P>(f, ring, li, RX, pa, oa, b0, c1, m, s);
     }
 }
 
@@ -224,8 +228,9 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
     constexpr int NI = two_slots(Q, (int)sizeof(S)), NT = two_threads(Q, (int)sizeof(S));
     static_assert(NI == NT || two_cap(Q, (int)sizeof(S)) < NI, "a slot for the threads without a cell");
     const uint32_t RX = bx + 2u;  // grown row
-    __shared__ S ring[ZRing<Q>::planes() * NI];
-    __shared__ uint32_t mring[2 * NI];  // the step t + 1 cells' masks or flags, two planes
+    constexpr bool HOLD = two_hold(Q, (int)sizeof(S));
+    __shared__ S ring[ZRing<Q, HOLD>::planes() * NI];
+    __shared__ uint32_t mring[(HOLD ? 1 : 2) * NI];  // the step t + 1 cells' masks or flags
 
     const uint32_t tid = threadIdx.x;
     const uint32_t X = a.X, Y = a.Y, Z = a.Z;
@@ -289,54 +294,97 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
     using Flat = std::integral_constant<int, kFlat>;
 
     // Step t + 2 of the tile's cell at plane n - 2 of the chunk (iteration n;
-    // none in the first two): from the ring planes of iterations n - 2, n - 1
-    // and n, with the mask of its step t + 1 cell (stored in mring by
-    // iteration n - 1).
+    // none in the first two), zo in the lattice: its values from the ring planes
+    // of iterations n - 2, n - 1 and n, with the mask of its step t + 1 cell
+    // (stored in mring by iteration n - 1), then its collision and its stores.
+    //
+    // One straight run of instructions from the ring's reads to the
+    // stores, threads without a cell and cells that are not fluid
+    // included (what they compute is dropped): the compiler then spreads
+    // the stores over the arithmetic, and in step 1 the next plane's loads,
+    // instead of issuing them in bursts at the end of a branch.  The
+    // kernel is bound by neither alone (D3Q19 256^3 FP32-shifted around
+    // solids: vector unit 65% busy, memory unit 67%), so what counts is
+    // that both work at the same time: 341 -> 317 us per step with solids,
+    // 287 -> 268 walls only; FP64 647 -> 630 / 601 -> 589; D3Q27 384^3
+    // FP32-shifted 1,634 -> 1,560, FP64 3,638 -> 3,455.  (Stores in every
+    // wavefront and plane, dropped where there is nothing to store, so that
+    // no wait for a load counts a path without them: no faster on large
+    // lattices, 2-10% slower on small ones.)
+    auto mask2 = [&](uint32_t slot0, uint32_t z) __attribute__((always_inline)) -> uint32_t {
+        if constexpr (FLAGS) return mring[slot0 * NI + li];
+        else return wall_cell(px, py, z);
+    };
+    auto finish = [&](uint32_t zo, bool zero, const Seams<I>& sm, T (&f)[Q]) __attribute__((always_inline)) {
+        const T rho = bgk<Q, P>(f, a, true);
+        if (MOV && a.bc.moving) moving_wall_terms<Q, P>(f, rho, sm, a);
+        // Around interior solids a cell that is not fluid stores zeros, so
+        // that lines are written whole (but a wavefront of such cells
+        // nothing); wall cells alone store nothing.
+        const bool store = in_o && (NB || !zero);
+        store_own<Q, V, W>(f, rb, B, store ? (zo * XY + py * X + px) * sz : kNoStore, psz, NB && zero);
+    };
     auto step2 = [&](uint32_t n) __attribute__((always_inline)) {
         const uint32_t zo = z0 + n - 2u;
-        const uint32_t pa = (n + 1u) % 3u, oa = (n + 2u) % 3u, b0 = (n + 1u) & 1u, c1 = n & 1u;
         if (n < 2u) return;
-        // One straight run of instructions from the ring's reads to the
-        // stores, threads without a cell and cells that are not fluid
-        // included (what they compute is dropped): the compiler then spreads
-        // the stores over the arithmetic, and in step 1 the next plane's loads,
-        // instead of issuing them in bursts at the end of a branch.  The
-        // kernel is bound by neither alone (D3Q19 256^3 FP32-shifted around
-        // solids: vector unit 65% busy, memory unit 67%), so what counts is
-        // that both work at the same time: 341 -> 317 us per step with solids,
-        // 287 -> 268 walls only; FP64 647 -> 630 / 601 -> 589; D3Q27 384^3
-        // FP32-shifted 1,634 -> 1,560, FP64 3,638 -> 3,455.  (Stores in every
-        // wavefront and plane, dropped where there is nothing to store, so that
-        // no wait for a load counts a path without them: no faster on large
-        // lattices, 2-10% slower on small ones.)
-        uint32_t mo;
-        if constexpr (FLAGS)
-            mo = mring[b0 * NI + li];
-        else
-            mo = wall_cell(px, py, zo);
+        const uint32_t b0 = (n + 1u) & 1u;
+        const uint32_t mo = mask2(b0, zo);
         const bool zero = NB ? (mo & 1u) != 0 : mo != 0;
         if (__any(in_o && !zero)) {
             const Seams<I> sm = seams<I>(px, py, zo, a);
             T f[Q];
-            ring_gather<Q, 0, V, NB, NI>(f, ring, li, RX, pa, oa, b0, c1, mo, sm);
-            const T rho = bgk<Q, P>(f, a, true);
-            if (MOV && a.bc.moving) moving_wall_terms<Q, P>(f, rho, sm, a);
-            // Around interior solids a cell that is not fluid stores zeros, so
-            // that lines are written whole (but a wavefront of such cells
-            // nothing); wall cells alone store nothing.
-            const bool store = in_o && (NB || !zero);
-            store_own<Q, V, W>(f, rb, B, store ? (zo * XY + py * X + px) * sz : kNoStore, psz, NB && zero);
+            ring_gather<Q, 0, V, NB, NI, HOLD, kAll>(f, ring, li, RX, (n + 1u) % 3u, (n + 2u) % 3u, b0, n & 1u, mo, sm);
+            finish(zo, zero, sm, f);
+        }
+    };
+    // HOLD: the cell's values in two parts.  read2 completes the cell of plane
+    // n - 1 (fo, its mask mo) with the c_z = -1 directions from plane n, and takes
+    // the other directions of the cell of plane n (hold, its mask mhold).
+    T hold[Q], fo[Q];
+    uint32_t mhold = 1u, mo = 1u;
+    auto read2 = [&](uint32_t n) __attribute__((always_inline)) {
+        const uint32_t up = (n + 1u) & 1u, zh = (z0 + n + Z - 1u) % Z;  // the c_z = +1 group's slot of plane n - 1
+#pragma unroll
+        for (int k = 0; k < Q; ++k)
+            if (Lat<Q>::cz(k) >= 0) fo[k] = hold[k];
+        mo = mhold;
+        ring_gather<Q, 0, V, NB, NI, true, kDown>(fo, ring, li, RX, up, up, 0u, 0u, mo,
+                                                  seams<I>(px, py, (z0 + n + Z - 2u) % Z, a));
+        mhold = mask2(0u, zh);
+        ring_gather<Q, 0, V, NB, NI, true, kHeld>(hold, ring, li, RX, up, up, 0u, 0u, mhold, seams<I>(px, py, zh, a));
+    };
+    auto collide2 = [&](uint32_t n) __attribute__((always_inline)) {
+        if (n < 2u) return;
+        const uint32_t zo = z0 + n - 2u;
+        const bool zero = NB ? (mo & 1u) != 0 : mo != 0;
+        if (__any(in_o && !zero)) finish(zo, zero, seams<I>(px, py, zo, a), fo);
+    };
+    // The second half of an iteration: plane n is in the ring.  HOLD with
+    // 4-byte storage collides after the barrier, next to the loads and the
+    // collision of the next plane (D3Q27 FP32-shifted 256^3 457 us per step
+    // against 477, 384^3 1,527 / 1,542; FP64, which waits on its stores there,
+    // 602 / 571 at D3Q19 256^3, 3,085 / 3,017 at D3Q27 384^3).
+    auto second = [&](uint32_t n) __attribute__((always_inline)) {
+        lds_barrier();
+        if constexpr (!HOLD) {
+            step2(n);
+            lds_barrier();
+        } else {
+            read2(n);
+            if (sizeof(S) == 8) collide2(n);
+            lds_barrier();
+            if (sizeof(S) != 8) collide2(n);
         }
     };
     // Step t + 1 of this thread's cell at plane n from the loads in fv, into
-    // the ring slots a3 (c_z = +1 group) and a2 (the others).
-    auto step1 = [&](uint32_t n, const S (&fv)[Q], uint32_t a3, uint32_t a2) __attribute__((always_inline)) {
+    // its ring slots (relative plane numbers: only n mod 3 and mod 2 matter).
+    auto step1 = [&](uint32_t n, const S (&fv)[Q]) __attribute__((always_inline)) {
         T f[Q];
 #pragma unroll
         for (int k = 0; k < Q; ++k) f[k] = P::load_raw(fv[k]);
         const T rho = bgk<Q, P>(f, a, true);
         if (MOV && a.bc.moving) moving_wall_terms<Q, P>(f, rho, seams<I>(gx, gy, (z0 + n + Z - 1u) % Z, a), a);
-        ring_store<Q, 0, V, NI>(f, ring, slot, a3, a2);
+        ring_store<Q, 0, V, NI, HOLD>(f, ring, slot, HOLD ? n & 1u : n % 3u, HOLD ? 0u : n & 1u);
     };
 
     if constexpr (!SPLIT) {
@@ -352,16 +400,12 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
             // (plane numbers wrap modulo Z, so the loads past the chunk's
             // last plane stay in bounds; their values are not used)
             mnext = load_mask(n + 1u);
-            // ring slots of plane n (relative plane numbers: only n mod 3 and mod 2 matter)
-            const uint32_t a3 = n % 3u, a2 = n & 1u;
-            // the step t + 2 cells read this mask in the next iteration
-            if (FLAGS) mring[a2 * NI + slot] = mcur;
+            // the step t + 2 cells read this mask
+            if (FLAGS) mring[(HOLD ? 0u : n & 1u) * NI + slot] = mcur;
             // (a wavefront of solid cells has nothing to compute)
-            if (!__all(NB ? (mcur & 1u) != 0 : mcur != 0)) step1(n, fv, a3, a2);
+            if (!__all(NB ? (mcur & 1u) != 0 : mcur != 0)) step1(n, fv);
             fetch(All{}, n + 1u, fv, mnext);
-            lds_barrier();
-            step2(n);
-            lds_barrier();
+            second(n);
         };
         uint32_t m0 = load_mask(0), m1 = 0;
         fetch(All{}, 0, fv, m0);
@@ -384,15 +428,12 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
         auto plane = [&](auto odd, uint32_t n, uint32_t& mc, uint32_t& mn) __attribute__((always_inline)) {
             S (&fc)[Q] = decltype(odd)::value ? fv1 : fv0;
             S (&fn)[Q] = decltype(odd)::value ? fv0 : fv1;
-            const uint32_t a3 = n % 3u, a2 = n & 1u;
-            if (FLAGS) mring[a2 * NI + slot] = mc;
+            if (FLAGS) mring[(HOLD ? 0u : n & 1u) * NI + slot] = mc;
             mc = load_mask(n + 2u);
             fetch(Flat{}, n + 1u, fn, mn);
-            step1(n, fc, a3, a2);
+            step1(n, fc);
             fetch(Up{}, n + 2u, fc, mc);
-            lds_barrier();
-            step2(n);
-            lds_barrier();
+            second(n);
         };
         uint32_t m0 = load_mask(0), m1 = load_mask(1);
         fetch(All{}, 0, fv0, m0);

@@ -91,3 +91,32 @@ def test_two_step_array_sizes(q, pad):
         fluid = slice(None) if mask is None else mask[1:-1] == 0
         assert np.array_equal(out[0][0][fluid], out[1][0][fluid])
         assert all(np.array_equal(a, b) for a, b in zip(out[0][1], out[1][1]))
+
+
+@pytest.mark.parametrize("q,variant", [(19, "f64"), (19, "f64a32"), (27, "f64"), (27, "f32s"), (27, "f32")])
+def test_two_step_held_values(orc, q, variant):
+    """Values held in registers from one plane to the next: one plane to a few,
+    z-chunks of one and two planes, rows of cells one more and one fewer than a
+    tile has, walls on z with both faces moving, solids and none."""
+    types = [PERIODIC] * 4 + [NOSLIP] * 2
+    vel = {P.UP: (0.02, 0.01, -0.01), P.DOWN: (-0.01, 0.0, 0.005)}
+    for Y, Z, zc, walls, solids in ((13, 1, 0, False, True), (14, 2, 1, False, False), (12, 3, 1, True, True),
+                                    (27, 4, 2, True, False), (7, 5, 0, True, True), (8, 6, 3, False, False)):
+        print(f"\n[case] held values q={q} {variant} 64x{Y}x{Z} chunk {zc} walls={walls} solids={solids}", flush=True)
+        ty, ve = (types, vel) if walls else ([PERIODIC] * 6, {})
+        ob, pb = Boundary(type=ty, vel=ve), P.boundary(ty, ve)
+        mask = (np.random.default_rng(4).random((Z, Y, 64)) < 0.2).astype(np.uint8) if solids else None
+        tau, F, init = 0.62, (2e-5, -1e-6, 1e-6), (P.INIT_PERTURBED, 5, 2e-3)
+        o = orc.cor_state(variant, q, 64, Y, Z)
+        orc.cor_init(o, 1.0, (0.01, 0.0, 0.0), init)
+        orc.cor_run(o, tau, F, ob, 7, mask)
+        fluid = orc.cor_flags(q, 64, Y, Z, ob, mask) == 0
+        with P.State(q, 64, Y, Z, variant, P.FUSED) as st:
+            st.set_tuning(capi.TUNE_TWO_STEP, 1)
+            st.set_tuning(capi.TUNE_TWO_ZCHUNK, zc)
+            assert st.scheme() == "pull2"
+            st.set_boundary(pb, mask)
+            st.initialize(1.0, (0.01, 0.0, 0.0), init, pb)
+            st.configure(tau, F, pb)
+            st.step(7)
+            assert np.array_equal(st.download_raw()[fluid], o["f"][fluid])
