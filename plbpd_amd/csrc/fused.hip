@@ -1039,9 +1039,10 @@ bool fused_two_eligible(const plb_state* s) {
         return grown <= 1.75 * s->two_any_bx * s->two_any_by * (double)s->Z;
     }
     // automatic: 4- and 8-byte storage, where two steps per pass measured
-    // 1.40x (D3Q19 256^3 FP32-shifted, 10% solids), 1.57x (walls only), 1.26x
-    // and 1.41x (FP64), 1.35x (D3Q27 FP32-shifted, walls) and 1.21x (D3Q27
-    // FP64, walls) faster on MI355X;
+    // faster on MI355X, one step per launch / two, us per step: D3Q19 256^3
+    // FP32-shifted 450 / 317 (10% solids) and 440 / 268 (walls only), FP64 915 /
+    // 594 and 922 / 515, D3Q27 256^3 walls only 641 / 442 (FP32-shifted) and
+    // 1,356 / 800 (FP64);
     // 2-byte storage ran 1.23x slower with solids (its one-step kernel is
     // closer to the arithmetic limit)
     if (s->tune_two < 0 && s->sbytes == 2) return false;

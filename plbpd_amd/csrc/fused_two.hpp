@@ -9,8 +9,8 @@
 // over a chunk of planes.  At each plane zi it computes step t + 1 on the
 // tile grown by one cell in x and y ((bx + 2) x (by + 2) cells, one per
 // thread), gathering step t from HBM, and keeps the result in an LDS ring
-// (ZRing: the directions with c_z = +1 for three planes, the others for
-// two).  It then computes step t + 2 on the tile at plane zi - 1, gathering
+// (ZRing: the directions with c_z = +1 for three planes, the others for two,
+// or, where two_hold() holds, two and one).  It then computes step t + 2 on the tile at plane zi - 1, gathering
 // from the ring (planes zi - 2, zi - 1, zi), and writes it to the other
 // population array.  The grown border is computed by both neighbouring tiles,
 // so workgroups never wait for each other: every workgroup reads only A and
