@@ -1075,6 +1075,8 @@ int fused_multi_steps(const plb_state* s) {
         return 1;
     const uint64_t cells = (uint64_t)s->X * (uint64_t)s->Y * (uint64_t)s->Z;
     if (cells > (1ull << 22)) return 1;
+    // one row of workgroups per 8 or 16 z-layers and per y-layer, at most 65,535 each
+    if ((uint64_t)s->Y > 65535u || (uint64_t)s->Z > 8u * 65535u) return 1;
     if ((uint64_t)s->q * s->pstride * s->sbytes > kMaxBuffer) return 1;
     return cells > (1ull << 18) && s->variant != kF64 ? 4 : kMultiSteps;
 }

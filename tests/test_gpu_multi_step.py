@@ -53,3 +53,21 @@ def test_multi_step_matches_oracle(orc, X, Y, Z, walls, solids, variant):
             a.step_graph(2 * spg + 3, spg)
             b.step(2 * spg + 3)
             assert np.array_equal(bits(a.download_raw())[fluid], bits(b.download_raw())[fluid]), spg
+
+
+@pytest.mark.parametrize("Y,Z", [(1, 8 * 65535 + 1), (65536, 3)])
+def test_layers_beyond_one_launch(orc, Y, Z):
+    """More layers than a launch has workgroup rows for: one step per launch."""
+    print(f"\n[case] multi-step f64 2x{Y}x{Z}", flush=True)
+    ob, pb = _bc((2,))
+    tau, F, init = 0.63, (2e-5, 0.0, 1e-6), (P.INIT_PERTURBED, 5, 2e-3)
+    fluid = orc.cor_flags(9, 2, Y, Z, ob, None) == 0
+    o = orc.cor_state("f64", 9, 2, Y, Z)
+    orc.cor_init(o, 1.0, (0.01, 0.0, 0.0), init)
+    orc.cor_run(o, tau, F, ob, 5, None)
+    with P.State(9, 2, Y, Z, "f64", P.FUSED) as st:
+        st.set_boundary(pb, None)
+        st.initialize(1.0, (0.01, 0.0, 0.0), init, pb)
+        st.configure(tau, F, pb)
+        st.step(5)
+        assert np.array_equal(st.download_raw()[fluid], o["f"][fluid])
