@@ -315,15 +315,16 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
         if constexpr (FLAGS) return mring[slot0 * NI + li];
         else return wall_cell(px, py, z);
     };
-    // The wall terms of a cell from coordinates that the compiler takes for new
-    // ones in every plane.  From the loop's own it computes each direction's wall
+    // The wall terms of a cell, for D3Q27 from coordinates that the compiler
+    // takes for new ones in every plane.  From the loop's own it computes each direction's wall
     // test and c_k . u_w before the loop and keeps them in registers through it:
-    // for D3Q27, next to the held values, 51 (FP64) and 45 (FP32) registers then
+    // next to the held values 51 (FP64) and 45 (FP32) registers then
     // went to scratch memory and back in every plane (128^3, lid on x / y, FP64 193 ->
     // 162 / 164 -> 138 us per step, FP32-shifted 134 -> 111 / 100 -> 86).
+    // D3Q19 has the registers (with FP16-shifted storage it ran 7% slower so).
     auto walls = [&](T (&f)[Q], T rho, uint32_t x, uint32_t y, uint32_t z) __attribute__((always_inline)) {
         if (MOV && a.bc.moving) {
-            asm volatile("" : "+v"(x), "+v"(y));
+            if constexpr (Q == 27) asm volatile("" : "+v"(x), "+v"(y));
             moving_wall_terms<Q, P>(f, rho, seams<I>(x, y, z, a), a);
         }
     };
