@@ -51,7 +51,7 @@ bool launch_batch2(const typename Prec<V>::S* A, typename Prec<V>::S* B, const B
     w.bc = bc;
     fill_wall_cub<Q, T>(bc, w.wcub);
     const dim3 grid(ntiles), block(two_threads(Q, (int)sizeof(typename Prec<V>::S)));
-    if (bc.moving)
+    if (two_walls(bc, false, (int)sizeof(typename Prec<V>::S)))
         hipLaunchKernelGGL((k_batch2<Q, V, true>), grid, block, 0, stream, A, B, doms, tiles, w);
     else
         hipLaunchKernelGGL((k_batch2<Q, V, false>), grid, block, 0, stream, A, B, doms, tiles, w);

@@ -875,7 +875,7 @@ int launch_kind(plb_state* s, KernelKind kind, int steps = 1) {
                 if constexpr (Q == 9) {
                     return fail(PLB_ERR_LOGIC, "no two-step kernel for D2Q9");
                 } else {
-                    if (!launch_pull2<Q, V>(a, two_geom(s), nb, a.bc.moving != 0, A, B, s->flags, s->nbmask,
+                    if (!launch_pull2<Q, V>(a, two_geom(s), nb, two_walls(a.bc, nb, (int)sizeof(S)), A, B, s->flags, s->nbmask,
                                             s->stream))
                         return fail(PLB_ERR_LOGIC, "no two-step kernel for this storage");
                 }

@@ -526,6 +526,19 @@ __host__ __device__ constexpr int two_rows(int q, int sbytes, int bx) {
         if (two_cells(bx, by) <= two_cap(q, sbytes)) best = by;
     return best >= 3 ? best : 0;
 }
+// Whether a boundary takes the two-step kernel's form with wall terms and zeros
+// at the cells of x walls: a moving wall, and walls on x without interior solids.
+// The zeros keep every line written whole (us per step without / with them:
+// D3Q19 FP64 128^3 91 / 77, 256^3 632 / 583, FP32-shifted 256^3 314 / 284, D3Q27
+// FP64 950 / 903, FP32-shifted 560 / 507; 512 domains of edges 16 to 96 1,188 /
+// 908).  2-byte storage, whose lines end inside a wavefront's store anyway, lost
+// 3-7% by the other form.  (The same stores in the form without walls made D3Q27
+// FP32-shifted 256^3 14% slower whatever its walls.)
+template <class T>
+bool two_walls(const FusedBC<T>& bc, bool nb, int sbytes) {
+    return bc.moving != 0 || (!nb && sbytes > 2 && bc.wall_lo[0]);
+}
+
 // The tile width a lattice and storage width prefer: 32 for 8-byte storage,
 // whose taller tile recomputes fewer grown-border cells (D3Q19 32 x 11
 // against 64 x 5: 6-13% faster from 128^3 to 384^3; D3Q27 fits 32-cell tiles

@@ -215,7 +215,8 @@ __device__ inline void lds_barrier() {
 // bx x by cells at (x0, y0), of any shape with at most two_cap() grown cells.
 // (With 64 x 8 and 32 x 11 tiles compiled in, D3Q19 256^3 ran 269 / 591 us per
 // step walls only, FP32-shifted / FP64, against 263 / 595 with the shape as an
-// argument.)  a: FusedArgs, or the like for one domain of a batch.
+// argument.)  a: FusedArgs, or the like for one domain of a batch.  MOV
+// (two_walls()): the form for moving walls and for walls on x.
 template <int Q, int V, int NB, bool MOV, int W, bool SPLIT, class Args>
 __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict__ A,
                                            typename Prec<V>::S* __restrict__ B, const uint8_t* __restrict__ flags,
@@ -331,11 +332,13 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
     auto finish = [&](uint32_t zo, bool zero, T (&f)[Q]) __attribute__((always_inline)) {
         const T rho = bgk<Q, P>(f, a, true);
         walls(f, rho, px, py, zo);
-        // Around interior solids a cell that is not fluid stores zeros, so
-        // that lines are written whole (but a wavefront of such cells
-        // nothing); wall cells alone store nothing.
-        const bool store = in_o && (NB || !zero);
-        store_own<Q, V, W>(f, rb, B, store ? (zo * XY + py * X + px) * sz : kNoStore, psz, NB && zero);
+        // Around interior solids and with walls on x, which begin and end
+        // every row, a cell that is not fluid stores zeros, so that lines are
+        // written whole (but a wavefront of such cells nothing); the wall
+        // rows of the other axes store nothing.
+        const bool whole = NB || (MOV && a.bc.wall_lo[0]);
+        const bool store = in_o && (whole || !zero);
+        store_own<Q, V, W>(f, rb, B, store ? (zo * XY + py * X + px) * sz : kNoStore, psz, whole && zero);
     };
     auto step2 = [&](uint32_t n) __attribute__((always_inline)) {
         const uint32_t zo = z0 + n - 2u;
