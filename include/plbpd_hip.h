@@ -275,8 +275,9 @@ int plb_bench_pattern(int device, int q, int x, int y, int z, int sbytes, int ve
                             /* the next wavefront); the row pull kernel's are    */
                             /* non-temporal without interior solids.            */
 #define PLB_TUNE_NT_STORE 2 /* non-temporal population stores (0/1; default 1); */
-                            /* the two-step kernel's and, on rows of no whole    */
-                            /* lines, the cell kernels' are ordinary             */
+                            /* the two-step kernel's and, on most lattices with  */
+                            /* rows of no whole lines, the cell pull kernel's    */
+                            /* are ordinary                                      */
 #define PLB_TUNE_SCHEME 3   /* streaming scheme of the fused step:              */
 #define PLB_SCHEME_AUTO 0   /*   pull (default; moving walls included)         */
 #define PLB_SCHEME_PUSH 1   /*   collide, then scatter to neighbours            */

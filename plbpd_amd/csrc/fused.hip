@@ -763,6 +763,26 @@ int multi_tile(const plb_state* s) {
     return tiles <= (uint64_t)s->num_cu ? 8 : 16;
 }
 
+// Whether the pull kernels' non-temporal stores pay.  A row that is no whole
+// number of lines ends inside a line that the next row's wavefronts go on
+// writing, and every wavefront's store begins and ends inside a line; ordinary
+// stores let the L2 put such lines together.  On MI355X, ordinary against
+// non-temporal, us per step: D3Q19 250 x 191 x 133 FP32-shifted 287 / 328,
+// FP16-shifted 172 / 196, 60^3 FP64 12.6 / 16.1, 100 x 50 x 50 FP32-shifted 10.4 /
+// 13.1.  Not where
+//   both arrays together are near the L2s' 32 MiB (50 x 72 x 73 FP16-shifted 9.1 /
+//     7.9, 60^3 7.6 / 6.7, 50^3 FP32-shifted 7.2 / 6.4, D3Q27 40^3 6.7 / 5.9);
+//   they are larger than the 256 MiB behind the L2s and few of a wavefront's lines
+//     are shared: 8-byte storage (D3Q27 300 x 200 x 100 664 / 622, 1000 x 1000 x 4
+//     389 / 340, D3Q19 24 x 200 x 200 73 / 68), and 4-byte storage on long rows (D3Q19
+//     1000 x 1000 x 4 160 / 152, D2Q9 2500 x 2500 125 / 111; 700-cell rows 207 / 230).
+bool nt_rows(const plb_state* s) {
+    const uint64_t row = (uint64_t)s->X * s->sbytes, both = 2 * (uint64_t)s->ncell * s->q * s->sbytes;
+    if (row % 128 == 0) return true;
+    if (both > (256ull << 20)) return s->sbytes == 8 || (s->sbytes == 4 && row >= 4000);
+    return both > (9ull << 20) && both <= (26ull << 20);
+}
+
 // Launch geometry and arguments shared by every fused-layout kernel.
 int launch_kind(plb_state* s, KernelKind kind, int steps = 1) {
     if (!s->bc_set) return fail(PLB_ERR_LOGIC, "fused step before the boundary was set");
@@ -838,12 +858,7 @@ int launch_kind(plb_state* s, KernelKind kind, int steps = 1) {
         a.xcd = (uint32_t)xm;
         a.dper = make_fastdiv(xm == 2 ? ntx * (nty / 8) : 1u);
         a.nt_load = s->tune_nt_load;
-        // A cell kernel's row that is no whole number of lines ends inside a
-        // line that the next row's wavefronts go on writing; ordinary stores
-        // let the L2 put such lines together (D3Q19 250 x 191 x 133 per step:
-        // FP32-shifted with solids 290 -> 239 us, FP16-shifted 160 -> 137,
-        // FP64 200 x 50 x 50 34 -> 31).
-        a.nt_store = s->tune_nt_store && (kind != kPull || (uint64_t)s->X * sizeof(S) % 128 == 0);
+        a.nt_store = s->tune_nt_store && (kind != kPull || nt_rows(s));
         a.tau = (T)s->tau;
         if (std::is_same<T, float>::value)  // CollisionSRT.cpp:19-20
             a.om = (T)(1. / (double)a.tau);
