@@ -325,8 +325,9 @@ int plb_bench_pattern(int device, int q, int x, int y, int z, int sbytes, int ve
                                 /* lattices from 2^18 cells that are not thin); 0 one */
                                 /* step per launch; -1 (default) automatic: on from   */
                                 /* 2^18 cells (2^19 for D3Q27 with x a multiple of    */
-                                /* 32), but for 2-byte storage only where x is no     */
-                                /* multiple of 32.  D2Q9 (reported as pull): 0 one    */
+                                /* 32); where x is no multiple of 32 if the tiles     */
+                                /* there fill the compute units; for 2-byte storage   */
+                                /* only on such lattices.  D2Q9 (reported as pull): 0 one    */
                                 /* step per launch, else up to 8 steps per launch of  */
                                 /* plb_step up to 2^22 cells.  The staged calls pair  */
                                 /* whole steps (plb_stream records one step and the   */

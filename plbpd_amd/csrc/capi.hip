@@ -314,6 +314,7 @@ int plb_state_create(const plb_state_desc* d, plb_state** out) {
     s->tune_two_zc = 0;
     s->tune_two_bx = 0;
     s->two_any_bx = s->two_any_by = 0;
+    s->two_any_pays = false;
     s->num_cu = 256;
     {
         int cu = 0;

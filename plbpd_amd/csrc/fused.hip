@@ -704,14 +704,16 @@ enum KernelKind { kPush, kPull, kGather, kStreamOnly, kCollideOnly, kAaEven, kAa
 // workgroup holds a compute unit's LDS, so the launch runs in rounds of the
 // workgroups resident at once (one per compute unit), and each chunk
 // of zc planes costs zc + 2 planes of work (the grown planes at its ends):
-// the chunk count minimises rounds x (zc + 2).  With the XCD mapping
+// the chunk count minimises rounds x (zc + 2), which *planes returns (narrow and
+// long lattices take as many chunks as there are compute units: D3Q19 30 x 30 x
+// 900 FP32-shifted, two tiles, 51 us per step with 30 chunks and 18 with 113).  With the XCD mapping
 // (PLB_TUNE_XCD not 0, compute units in multiples of 8) workgroup i runs on
 // XCD i mod 8, and XCD j takes the j-th of eight contiguous runs of the
 // (z-chunk, y-tile) pairs, ordered y-tile first, with every x-tile of each:
 // neighbouring tiles, whose grown borders overlap, then share that XCD's
 // L2.  The runs hold kx = ceil(pairs / 8) pairs (the last may be shorter),
 // so the rounds are counted per XCD.
-TwoGeom two_geom(const plb_state* s) {
+TwoGeom two_geom(const plb_state* s, uint64_t* planes = nullptr) {
     // rows of whole 64- or 32-cell tiles take those; other rows the shape that
     // two_shape found
     TwoGeom g;
@@ -733,17 +735,24 @@ TwoGeom two_geom(const plb_state* s) {
         const uint64_t kx = (nty * chunks + 7) / 8, per = ncu / 8;
         return (ntx * kx + per - 1) / per;
     };
-    uint64_t zc = Z;
+    uint64_t zc = Z, best = ~0ull;
     if (s->tune_two_zc > 0) {
         zc = std::min<uint64_t>((uint64_t)s->tune_two_zc, Z);
     } else {
-        uint64_t best = ~0ull;
-        for (uint64_t n = 1; n <= 32 && n <= Z; ++n) {
+        auto consider = [&](uint64_t n) {
+            if (n < 1 || n > Z) return;
             const uint64_t c = (Z + n - 1) / n, chunks = (Z + c - 1) / c;
             const uint64_t cost = rounds(chunks) * (c + 2);
             if (cost < best) best = cost, zc = c;
+        };
+        for (uint64_t n = 1; n <= 32; ++n) consider(n);
+        // the most chunks of one to four rounds
+        for (uint64_t r = 1; r <= 4; ++r) {
+            const uint64_t n = xcd ? ncu / 8 * r / ntx * 8 / nty : ncu * r / (ntx * nty);
+            if (n > 32) consider(n);
         }
     }
+    if (planes) *planes = best;
     g.zc = (uint32_t)zc;
     g.nzc = (uint32_t)((Z + zc - 1) / zc);
     // with fewer than eight pairs some XCDs would get none
@@ -1026,9 +1035,22 @@ int fused_two_tile_x(const plb_state* s) {
 }
 
 void fused_two_plan(plb_state* s) {
-    const TwoShape sh = s->q == 9 ? TwoShape{0, 0} : two_shape(s->q, (int)s->sbytes, s->X, s->Y);
+    s->two_any_bx = s->two_any_by = 0;
+    s->two_any_pays = false;
+    if (s->q == 9) return;
+    const TwoShape sh = two_shape(s->q, (int)s->sbytes, s->X, s->Y);
     s->two_any_bx = sh.bx;
     s->two_any_by = sh.by;
+    if (fused_two_tile_x(s) != 0) return;
+    uint64_t planes = 0;
+    (void)two_geom(s, &planes);
+    const TwoCost c = two_cost(s->q, (int)s->sbytes);
+    const double filled = (sh.bx + 2.0) * (sh.by + 2.0) / two_cap(s->q, (int)s->sbytes);
+    const double two = c.base + (double)planes * (c.plane + c.fill * filled);
+    const uint64_t XL = ((uint64_t)s->X + 63) / 64 * 64, YL = ((uint64_t)s->Y + 3) / 4 * 4, Z = (uint64_t)s->Z;
+    const double cells = std::max((double)s->ncell, 0.2 * (double)XL * (double)YL * (double)Z);
+    const double one = c.one_base + c.one_cell * 1e-6 * cells * 256 / s->num_cu;
+    s->two_any_pays = two <= one * (s->sbytes == 2 ? 1.22 : 1.0);
 }
 
 bool fused_two_eligible(const plb_state* s) {
@@ -1041,15 +1063,21 @@ bool fused_two_eligible(const plb_state* s) {
         // Rows that are no whole number of 32-cell tiles run in tiles of
         // their own shape (two_shape), with every storage type, from 2^18
         // cells on.  Their one-step kernel loads and stores rows at any
-        // alignment, and two steps per launch measured faster from there:
-        // D3Q19 250 x 191 x 133 290 -> 155-159 us per step (FP32-shifted,
-        // solids), 475 -> 272 (FP64), 160 -> 120 (FP16-shifted), 200 x 50 x 50
-        // FP64 34 -> 19; D3Q27 75 x 70 x 70 36 -> 23 (FP64), 28 -> 18; below,
-        // 50^3 (2^17 cells) ran 9.7 -> 8.8 (FP64) and 7.2 -> 7.8 (FP32-shifted),
-        // 40^3 5.1 -> 8.2.  Not where the grown borders (one layer each side in
+        // alignment, and two steps per launch measured faster on most lattices
+        // from there, one step per launch / two, us per step: D3Q19 250 x 191 x
+        // 133 284 / 136 (FP32-shifted), 510 / 216 (FP64), 171 / 95 (FP16-shifted),
+        // 200 x 50 x 50 FP64 32 / 19; D3Q27 75 x 70 x 70 37 / 22 (FP64), 22 / 15
+        // (FP32-shifted); below, 50^3 (2^17 cells) ran 9.7 / 8.8 (FP64) and 7.2 / 7.8
+        // (FP32-shifted), 40^3 5.1 / 8.2.  Automatic only where the costs of
+        // two_cost() say so, with two_any_pays set by fused_two_plan: cross-sections
+        // of a few cells fill no tile (D3Q19 9 x 9 x 4000 FP32-shifted 20 / 28).
+        // 2-byte storage, which has the least to gain, is allowed 1.22 times the
+        // one-step estimate, where two steps measured from 20% slower to 40% faster.  Never
+        // where the grown borders (one layer each side in
         // y and z as in x) make up for the saved pass: thin lattices.  A
         // forced tile width that does not divide the row has no such kernel.
         if (s->tune_two_bx > 0 || s->X % 32 == 0 || cells < (1ull << 18)) return false;
+        if (s->tune_two < 0 && !s->two_any_pays) return false;
         const double grown = (s->two_any_bx + 2.0) * (s->two_any_by + 2.0) * (s->Z + 2.0);
         return grown <= 1.75 * s->two_any_bx * s->two_any_by * (double)s->Z;
     }

@@ -574,6 +574,25 @@ inline TwoShape two_shape(int q, int sbytes, int X, int Y) {
     return best;
 }
 
+// What a step costs on 256 compute units, fitted to 130 lattices of 2^18 to 6.4
+// M cells on MI355X: with two steps per launch base + planes * (plane + fill *
+// filled) us, planes the planes that the compute units go through one after the
+// other and filled the part of two_cap() that a grown tile has (a plane takes
+// nearly as long in a tile of 200 cells as in one of 700); with one step per
+// launch of a cell kernel one_base + one_cell us per million cells, a wavefront's
+// row of up to 64 cells counted as 13 at least.  Lattices beyond the caches take
+// about 1.35 times either.
+struct TwoCost {
+    double base, plane, fill, one_base, one_cell;
+};
+inline TwoCost two_cost(int q, int sbytes) {
+    if (q == 19)
+        return sbytes == 8 ? TwoCost{3.3, 1.09, 0.69, 2.1, 56}
+                           : (sbytes == 4 ? TwoCost{1.5, 1.27, 0.41, 2.3, 30} : TwoCost{0.5, 1.77, 0.64, 4.6, 17.8});
+    return sbytes == 8 ? TwoCost{3.8, 1.47, 1.39, 0, 88}
+                       : (sbytes == 4 ? TwoCost{1.5, 1.44, 0.94, 1.8, 44} : TwoCost{0, 2.6, 0.85, 4.3, 25.5});
+}
+
 // Two pull steps in one pass (fused_two.hpp), tiles of g.bx x g.by cells.
 // Returns false where no kernel exists for (Q, V, g).
 template <int Q, int V>

@@ -115,10 +115,11 @@ struct plb_state {
     int tune_index64;     // 1: 64-bit index kernels even where 32-bit offsets fit
     int tune_vector;      // row pull kernel cells per lane (1, 2, 4) where X allows; 0 off; -1 auto
     int tune_lit_fuse;    // literal: 1 collision and push in one kernel when they follow each other
-    int tune_two;         // fused pull: two steps per launch where a kernel exists; 0 off, 1 on, -1 auto (4- and 8-byte storage)
+    int tune_two;         // fused pull: two steps per launch where a kernel exists; 0 off, 1 on, -1 auto (fused_two_eligible)
     int tune_two_zc;      // planes per z-chunk of the two-step launch; 0 = chosen from the grid
     int tune_two_bx;      // two-step tile width: 32 or 64 cells; 0 = automatic
     int two_any_bx, two_any_by;  // two-step tile shape for rows of no whole number of 32-cell tiles
+    bool two_any_pays;           // and whether such tiles are faster than one step per launch
     int num_cu;           // compute units of the state's device
     bool post_collision;  // fused: buf[cur] holds post-collision populations (pull step)
     // one-array state (PLB_MODE_FUSED_AA): buf[cur] only; aa_odd = after an
@@ -142,7 +143,7 @@ int timer_end(plb_state* s, TimerPair* tp);
 // state steps with the pull scheme and a kernel exists for its lattice,
 // storage and row length; the launch needs post-collision storage.
 bool fused_two_eligible(const plb_state* s);
-// Sets the two-step tile shape of a new state (fused.hip).
+// Sets the two-step tile shape of a new state and whether it pays (fused.hip).
 void fused_two_plan(plb_state* s);
 // Runs the step plb_stream deferred, if any (capi.hip).
 int fused_flush_deferred(plb_state* s);

@@ -120,3 +120,39 @@ def test_two_step_held_values(orc, q, variant):
             st.configure(tau, F, pb)
             st.step(7)
             assert np.array_equal(st.download_raw()[fluid], o["f"][fluid])
+
+
+def test_two_step_only_where_its_tiles_fill():
+    """Automatic only where a launch's tiles and chunks of planes use the chip:
+    not on cross-sections of a few cells, however long; asked for, still there."""
+    for q, X, Y, Z, variant, want in ((19, 9, 9, 4000, "f32s", "pull"), (19, 12, 12, 2000, "f16s", "pull"),
+                                      (27, 9, 9, 4000, "f32s", "pull"), (27, 300, 3, 300, "f16s", "pull"),
+                                      (19, 30, 30, 900, "f32s", "pull2"), (27, 24, 24, 500, "f64", "pull2"),
+                                      (19, 3, 300, 300, "f32s", "pull2"), (19, 250, 191, 133, "f16s", "pull2")):
+        with P.State(q, X, Y, Z, variant, P.FUSED) as st:
+            assert st.scheme() == want, (q, X, Y, Z, variant)
+            st.set_tuning(capi.TUNE_TWO_STEP, 1)
+            assert st.scheme() == "pull2"
+
+
+@pytest.mark.parametrize("q,X,Y,Z,variant", [(19, 24, 24, 500, "f32s"), (27, 30, 30, 300, "f64"), (19, 32, 9, 1200, "f64"),
+                                             (27, 64, 5, 1100, "f16s"), (19, 7, 7, 6000, "f32")])
+def test_more_chunks_than_planes_of_a_tile(q, X, Y, Z, variant):
+    """Long lattices of one or two tiles across, in as many z-chunks as there
+    are compute units: the values of one step per launch, bit for bit."""
+    types, vel = [PERIODIC] * 4 + [NOSLIP] * 2, {P.UP: (0.02, 0.01, -0.01), P.DOWN: (0.0, 0.0, 0.0)}
+    pb = P.boundary(types, vel)
+    print(f"\n[case] chunks {variant} q={q} {X}x{Y}x{Z}", flush=True)
+    mask = (np.random.default_rng(8).random((Z, Y, X)) < 0.1).astype(np.uint8)
+    out = []
+    for two in (1, 0):
+        with P.State(q, X, Y, Z, variant, P.FUSED) as st:
+            st.set_tuning(capi.TUNE_TWO_STEP, two)
+            assert st.scheme() == ("pull2" if two else "pull")
+            st.set_boundary(pb, mask)
+            st.initialize(1.0, (0.01, 0.0, 0.0), (P.INIT_PERTURBED, 5, 2e-3), pb)
+            st.configure(0.62, (2e-5, -1e-6, 1e-6), pb)
+            st.step(6)
+            raw = st.download_raw()[1:-1]
+            out.append((raw.view(np.uint16) if variant == "f16s" else raw)[mask[1:-1] == 0])
+    assert np.array_equal(out[0], out[1])
