@@ -344,6 +344,9 @@ int plb_set_tuning(plb_state* s, int key, int value);
  * PLB_SCHEME_PULL, PLB_SCHEME_PULL_TWO (pull, two steps per launch, for
  * pairs of steps) or PLB_SCHEME_AA. */
 int plb_step_scheme(const plb_state* s, int* scheme);
+/* The most steps that one launch of the next fused steps advances: 2 for
+ * PLB_SCHEME_PULL_TWO, up to 8 for D2Q9, else 1. */
+int plb_steps_per_launch(const plb_state* s, int* steps);
 
 /* ---- batched domains (no reference counterpart: one domain per PLBPD,
  * PLBPD.hpp:14-17) --------------------------------------------------------- */
@@ -374,8 +377,10 @@ int plb_batch_set_scheme(plb_batch* b, int scheme);
  * takes a contiguous run of tiles. */
 int plb_batch_set_mapping(plb_batch* b, int xcd_runs);
 int plb_batch_get_mapping(const plb_batch* b, int* xcd_runs);
-/* Times each candidate tiling and mapping over `steps` steps and keeps the
- * fastest.  results: up to max_results rows of {tile_cells, grid_blocks,
+/* Times each candidate tiling and mapping over `steps` steps, one step per
+ * launch (the launches the tiling and mapping are for: a batch that takes two
+ * steps per launch, plb_batch_steps_per_launch, uses them for odd steps only, and its
+ * plb_batch_step is faster than the times here), and keeps the fastest.  results: up to max_results rows of {tile_cells, grid_blocks,
  * mapping, ms_per_step}; *nresults = the rows written.  The candidates run
  * real steps on the batch: every candidate (60: 6 tile sizes x 5 grids x 2
  * mappings) advances all domains by 2 + (steps rounded up to even) steps, so
@@ -387,6 +392,8 @@ int plb_batch_autotune(plb_batch* b, int steps, double* results, int max_results
  * the same values bit for bit), graph-captured when steps_per_graph > 0.  The
  * tiling and mapping are those of the one-step launches. */
 int plb_batch_step(plb_batch* b, int nsteps, int steps_per_graph);
+/* The steps that a launch of plb_batch_step advances: 1 or 2. */
+int plb_batch_steps_per_launch(const plb_batch* b, int* steps);
 /* Baseline: the same steps with one launch per domain per step. */
 int plb_batch_step_per_domain(plb_batch* b, int nsteps);
 /* rho (x*y*z) and u (x*y*z*3) of domain d, compact AoS, double. */

@@ -154,6 +154,7 @@ def lib():
     L.plb_bench_pattern.argtypes = [i] * 9 + [C.POINTER(C.c_double), C.POINTER(C.c_double)]
     L.plb_set_tuning.argtypes = [vp, i, i]
     L.plb_step_scheme.argtypes = [vp, C.POINTER(C.c_int)]
+    L.plb_steps_per_launch.argtypes = [vp, C.POINTER(C.c_int)]
     if hasattr(L, "plb_batch_create"):
         L.plb_batch_create.argtypes = [i, i, i, C.POINTER(DomainDesc), C.POINTER(BoundaryC), i, C.POINTER(vp)]
         L.plb_batch_destroy.argtypes = [vp]
@@ -165,6 +166,7 @@ def lib():
         L.plb_batch_set_scheme.argtypes = [vp, i]
         L.plb_batch_get_mapping.argtypes = [vp, C.POINTER(C.c_int)]
         L.plb_batch_step.argtypes = [vp, i, i]
+        L.plb_batch_steps_per_launch.argtypes = [vp, C.POINTER(C.c_int)]
         L.plb_batch_step_per_domain.argtypes = [vp, i]
         L.plb_batch_download_moments.argtypes = [vp, i, vp, vp]
         L.plb_batch_cells.argtypes = [vp, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]
@@ -362,8 +364,11 @@ class State:
         return {SCHEME_PULL: "pull", SCHEME_AA: "aa", SCHEME_PULL_TWO: "pull2"}.get(v.value, "push")
 
     def steps_per_launch(self):
-        """Steps one launch of the fused kernel advances (2 for 'pull2')."""
-        return 2 if self.scheme() == "pull2" else 1
+        """The most steps one launch of the fused kernel advances (2 for
+        'pull2', up to 8 for D2Q9, else 1)."""
+        v = C.c_int()
+        check(lib().plb_steps_per_launch(self.h, C.byref(v)))
+        return v.value
 
     def global_moments(self):
         out = np.zeros(4, np.float64)
@@ -387,7 +392,8 @@ class State:
 
 
 class Batch:
-    """Many independent domains advanced together (one launch per step)."""
+    """Many independent domains advanced together (one launch for one or two
+    steps of all of them, steps_per_launch())."""
 
     def __init__(self, q, variant, domains, bc: BoundaryC, device=0):
         if isinstance(variant, str):
@@ -440,7 +446,8 @@ class Batch:
         return m.value
 
     def autotune(self, steps=10, max_results=128):
-        """Rows of (tile_cells, grid_blocks, mapping, ms_per_step)."""
+        """Rows of (tile_cells, grid_blocks, mapping, ms_per_step), timed with
+        one step per launch, which is what the tiling and mapping are for."""
         res = np.zeros((max_results, 4), np.float64)
         n = C.c_int(0)
         check(lib().plb_batch_autotune(self.h, int(steps), _p(res), max_results, C.byref(n)))
@@ -448,6 +455,12 @@ class Batch:
 
     def step(self, n, steps_per_graph=0):
         check(lib().plb_batch_step(self.h, int(n), int(steps_per_graph)))
+
+    def steps_per_launch(self):
+        """Steps one launch advances (1 or 2)."""
+        v = C.c_int()
+        check(lib().plb_batch_steps_per_launch(self.h, C.byref(v)))
+        return v.value
 
     def step_per_domain(self, n):
         check(lib().plb_batch_step_per_domain(self.h, int(n)))

@@ -907,6 +907,12 @@ int plb_batch_step(plb_batch* b, int nsteps, int steps_per_graph) {
     return batch_step_plain(b, nsteps - reps * steps_per_graph);
 }
 
+int plb_batch_steps_per_launch(const plb_batch* b, int* steps) {
+    if (!b || !steps) return fail(PLB_ERR_INVALID_ARGUMENT, "null argument");
+    *steps = batch_two(b) ? 2 : 1;
+    return PLB_OK;
+}
+
 int plb_batch_step_per_domain(plb_batch* b, int nsteps) {
     if (!b || nsteps < 0) return fail(PLB_ERR_INVALID_ARGUMENT, "bad arguments");
     PLB_HIP_TRY(hipSetDevice(b->device));

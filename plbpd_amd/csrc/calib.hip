@@ -222,6 +222,13 @@ int plb_step_scheme(const plb_state* s, int* scheme) {
     return PLB_OK;
 }
 
+int plb_steps_per_launch(const plb_state* s, int* steps) {
+    if (!s || !steps) return fail(PLB_ERR_INVALID_ARGUMENT, "null argument");
+    if (s->mode != PLB_MODE_FUSED) return fail(PLB_ERR_LOGIC, "literal mode has no fused scheme");
+    *steps = fused_two_eligible(s) ? 2 : fused_multi_steps(s);
+    return PLB_OK;
+}
+
 int plb_time_steps(plb_state* s, int nsteps, int steps_per_graph, double* ms) {
     if (!s || !ms) return fail(PLB_ERR_INVALID_ARGUMENT, "null argument");
     PLB_HIP_TRY(hipSetDevice(s->device));

@@ -71,3 +71,25 @@ def test_layers_beyond_one_launch(orc, Y, Z):
         st.configure(tau, F, pb)
         st.step(5)
         assert np.array_equal(st.download_raw()[fluid], o["f"][fluid])
+
+
+def test_steps_per_launch():
+    """What a launch advances, as the state reports it: D2Q9 with several steps
+    is reported as the pull scheme."""
+    with P.State(9, 256, 1, 64, "f64", P.FUSED) as st:
+        assert st.scheme() == "pull" and st.steps_per_launch() == 8
+        for key, value in ((capi.TUNE_TWO_STEP, 0), (capi.TUNE_INDEX64, 1), (capi.TUNE_SCHEME, capi.SCHEME_PUSH)):
+            st.set_tuning(key, value)
+            assert st.steps_per_launch() == 1
+            st.set_tuning(key, -1 if key == capi.TUNE_TWO_STEP else 0)
+            assert st.steps_per_launch() == 8
+    for Y, Z in ((1, 8 * 65535 + 1), (65536, 3)):
+        with P.State(9, 2, Y, Z, "f64", P.FUSED) as st:
+            assert st.steps_per_launch() == 1
+    with P.State(9, 256, 1, 64, "f64", P.FUSED_AA) as st:
+        assert st.steps_per_launch() == 1
+    with P.State(19, 64, 64, 64, "f64", P.FUSED) as st:
+        assert st.steps_per_launch() == 2
+    with P.State(9, 8, 1, 8, "f64", P.LITERAL) as st:
+        with pytest.raises(P.LogicError):
+            st.steps_per_launch()
