@@ -1107,21 +1107,38 @@ int fused_launch_two(plb_state* s) {
 
 // Steps per launch of a D2Q9 lattice.  Up to 2^22 cells a launch of several
 // steps measured faster than one launch per step (per step, one against
-// several): FP64 100 x 25 3.4 -> 1.3 us, 256 x 64 5.2 -> 1.4, 512 x 256 7.5 ->
-// 3.6, 1024 x 1024 31 -> 23, 2048 x 2048 113 -> 91; FP32-shifted 256 x 64 4.5 ->
-// 1.2, 1024 x 512 9.6 -> 7.7, 2048 x 2048 59 -> 58.  Above 2^18 cells, where
-// memory and not the launch is what a step waits for, FP32 arithmetic takes 4
-// steps, which recompute less (1024 x 512: 8.8 us with 8).
+// several): FP64 100 x 25 3.4 -> 1.1 us, 256 x 64 5.2 -> 1.3, 512 x 256 7.1 ->
+// 3.4, 1024 x 1024 32 -> 22, 2048 x 2048 112 -> 91; FP32-shifted 256 x 64 4.8 ->
+// 1.2, 1024 x 512 9.5 -> 7.3, 2048 x 1024 31 -> 26.  Above 2^18 cells, where
+// memory and not the launch is what a step waits for, 4-byte storage takes 4
+// steps, which recompute less (1024 x 512: 8.8 us with 8); 8-byte storage keeps 8
+// (FP64 with FP32 arithmetic 65,536 x 64: 129 us with 4, 93 with 8).
+//
+// Not where the tiles are mostly outside the lattice: a workgroup takes the time
+// of its whole tile, 256 of them about 11 us with 8-byte storage (one per
+// compute unit), 8.5 with 4-byte and 9 with 2-byte storage, and 3.9 with 4 steps, while a step per launch takes 2
+// us and 27, 14 or 9 us per million cells with 8-, 4- and 2-byte storage, or 1.7 per
+// million lanes of its 64 x 4 blocks.  One step per launch / several: FP64 65,536 x
+// 4 8.5 / 22 us, 1,048,576 x 1 32 / 342, 3 x 3 in 40,000 y-layers 65 / 209, 131,072 x 8
+// 31 / 43, 131,072 x 16 60 / 47; FP16-shifted 1024 x 1024 11.4 / 13.8; but 262,144
+// rows of 4 cells 139 / 86.
 int fused_multi_steps(const plb_state* s) {
     if (s->q != 9 || s->tune_two == 0 || s->tune_index64 || s->aa || !fused_uses_pull(s) ||
         s->mode != PLB_MODE_FUSED)
         return 1;
-    const uint64_t cells = (uint64_t)s->X * (uint64_t)s->Y * (uint64_t)s->Z;
+    const uint64_t X = (uint64_t)s->X, Y = (uint64_t)s->Y, Z = (uint64_t)s->Z, cells = X * Y * Z;
     if (cells > (1ull << 22)) return 1;
     // one row of workgroups per 8 or 16 z-layers and per y-layer, at most 65,535 each
-    if ((uint64_t)s->Y > 65535u || (uint64_t)s->Z > 8u * 65535u) return 1;
+    if (Y > 65535u || Z > 8u * 65535u) return 1;
     if ((uint64_t)s->q * s->pstride * s->sbytes > kMaxBuffer) return 1;
-    return cells > (1ull << 18) && s->variant != kF64 ? 4 : kMultiSteps;
+    const int steps = cells > (1ull << 18) && s->sbytes != 8 ? 4 : kMultiSteps;
+    const uint64_t t = (uint64_t)multi_tile(s), ncu = (uint64_t)s->num_cu;
+    const uint64_t tiles = (X + t - 1) / t * ((Z + t - 1) / t) * Y, rounds = (tiles + ncu - 1) / ncu;
+    const double several = (double)rounds * (s->sbytes == 8 ? 11.0 : (steps == 4 ? 3.9 : (s->sbytes == 4 ? 8.5 : 9.0))) / steps;
+    const double cell = s->sbytes == 8 ? 27e-6 : (s->sbytes == 4 ? 14.2e-6 : 9e-6);
+    const uint64_t lanes = (X + 63) / 64 * 64 * ((Y + 3) / 4 * 4) * Z;
+    const double one = 2.0 + std::max(cell * (double)cells, 1.7e-6 * (double)lanes) * 256 / (double)ncu;
+    return several <= one ? steps : 1;
 }
 
 int fused_launch_multi(plb_state* s, int steps) {

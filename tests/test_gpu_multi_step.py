@@ -93,3 +93,21 @@ def test_steps_per_launch():
     with P.State(9, 8, 1, 8, "f64", P.LITERAL) as st:
         with pytest.raises(P.LogicError):
             st.steps_per_launch()
+
+
+def test_multi_step_rule():
+    """Several steps per launch where the tiles lie in the lattice, so on every
+    lattice of test_multi_step_matches_oracle, and not on thin ones."""
+    several = [(1, 1, 1), (3, 1, 3), (5, 1, 7), (100, 1, 25), (64, 1, 40), (17, 3, 19), (201, 1, 131), (161, 1, 130),
+               (512, 1, 256), (4, 1, 262144)]
+    for X, Y, Z in several:
+        for variant in ("f64", "f32", "f64a32", "f32s", "f16s"):
+            with P.State(9, X, Y, Z, variant, P.FUSED) as st:
+                assert st.steps_per_launch() > 1, (X, Y, Z, variant)
+    for X, Y, Z in ((65536, 1, 4), (1048576, 1, 1), (3, 40000, 3), (131072, 1, 8)):
+        for variant in ("f64", "f32s", "f16s"):
+            with P.State(9, X, Y, Z, variant, P.FUSED) as st:
+                assert st.steps_per_launch() == 1, (X, Y, Z, variant)
+    for variant, steps in (("f64", 8), ("f64a32", 8), ("f32s", 4), ("f16s", 1)):
+        with P.State(9, 1024, 1, 1024, variant, P.FUSED) as st:
+            assert st.steps_per_launch() == steps, variant
