@@ -457,12 +457,14 @@ int batch_layout(plb_batch* b, int tile) {
 // domain and share their borders in that XCD's L2 (the runs in turn from the
 // largest and from the smallest, to spread the work evenly).
 // Two steps per launch from 2^18 cells on, unless the grown borders (domains a
-// few layers thin) cost more than the saved pass: the rule of
-// fused_two_eligible.  512 domains of edges 16 to 96 (44.8 M cells, D3Q19
-// FP32-shifted): one step per launch 1,162 us per step, two 881, and 830 since
-// the kernel's steps run straight through (FP64 2,570 and 1,628, FP16-shifted
-// 792 and 673 before that); 64 domains (6.1 M) 160 -> 140, 16 (1.1 M) 28.9 -> 28.6 (FP64 59
-// -> 48).
+// few layers thin) cost more than the saved pass, and where the cost of the
+// tiles (two_cost(), 1.25 times it beyond the caches for 4- and 8-byte storage) is
+// below that of the one-step kernel, 3 us and cell us per million cells: a tile of
+// a small domain takes nearly the time of a full one.  One step per launch / two, us per
+// step: 512 domains of edges 16 to 96 (44.2 M cells) D3Q19 FP32-shifted 1,168 / 825,
+// FP64 2,554 / 1,607, FP16-shifted 793 / 693; 64 of them (5.6 M) 147 / 128; 512
+// domains of 16^3 FP64 111 / 74, but FP32-shifted 53 / 62 and FP16-shifted 42 / 67; 3,000
+// of 10^3 FP64 166 / 215, FP32-shifted 87 / 210, FP16-shifted 59 / 260.
 int two_step_plan(plb_batch* b, int ncu) {
     b->ntwo = 0;
     if (b->q == 9 || b->total_cells < (1ull << 18)) return PLB_OK;
@@ -494,21 +496,29 @@ int two_step_plan(plb_batch* b, int ncu) {
         if (best == 0 || cost < best) best = cost, zbest = zc;
     }
     std::vector<std::pair<double, BTile>> list;
-    double grown = 0;
+    const TwoCost cost = two_cost(b->q, sb);
+    double grown = 0, two = 0, longest = 0;
     for (int d = 0; d < b->ndom; ++d) {
         const plb_domain_desc& D = b->desc[d];
         const TwoShape& t = shape[d];
         const int chunks = (D.z + zbest - 1) / zbest, c = (D.z + chunks - 1) / chunks;
+        const double plane = cost.plane + cost.fill * (t.bx + 2) * (t.by + 2) / cap;
+        longest = std::max(longest, plane * (c + 2));
         for (int z = 0; z < D.z; z += c)
             for (int y = 0; y < D.y; y += t.by)
                 for (int x = 0; x < D.x; x += t.bx) {
                     const int planes = std::min(c, D.z - z) + 2;
                     grown += (double)(t.bx + 2) * (t.by + 2) * planes;
+                    two += plane * planes;
                     list.push_back({weight(t) * planes, BTile{(uint32_t)d, (uint32_t)x, (uint32_t)y, (uint32_t)z,
                                                               (uint32_t)c, (uint32_t)t.bx, (uint32_t)t.by, 0}});
                 }
     }
     if (grown > 1.75 * (double)b->total_cells || list.size() >= (1ull << 31)) return PLB_OK;
+    two = std::max(two / ncu, longest) + 0.5 * longest;
+    if (sb > 2 && 2.0 * b->q * sb * (double)b->total_cells > 3e8) two *= 1.25;
+    const double cell = b->q == 19 ? (sb == 8 ? 50 : (sb == 4 ? 25 : 19.5)) : (sb == 8 ? 74 : (sb == 4 ? 37 : 27.5));
+    if (cost.base + two > 3 + cell * 1e-6 * (double)b->total_cells * 256 / ncu) return PLB_OK;
     std::stable_sort(list.begin(), list.end(), [](const auto& l, const auto& r) { return l.first > r.first; });
     std::vector<BTile> order(list.size());
     for (size_t g = 0; g < list.size(); g += 256) {
