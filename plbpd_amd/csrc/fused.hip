@@ -673,6 +673,7 @@ int fused_build_flags(plb_state* s, const plb_boundary* bc, const uint8_t* mask)
     s->has_solids = any_solid;
     s->bc = *bc;
     s->bc_set = true;
+    s->moments_valid = false;  // solid cells report rho_s and the wall's velocity
     return PLB_OK;
 }
 

@@ -69,3 +69,36 @@ def test_read_sizes(cells):
         for k in range(9):  # ascending, as the moments sum
             r += c[..., k]
         assert np.array_equal(st.download(P.FIELD_RHO, P.LAYOUT_COMPACT), r)
+
+
+@pytest.mark.parametrize("mode", [P.FUSED, P.FUSED_AA])
+@pytest.mark.parametrize("how", ["set_boundary", "configure", "reset"])
+@pytest.mark.parametrize("q,X,Y,Z", [(9, 40, 1, 9), (19, 33, 10, 9)])
+def test_read_after_the_boundary_changed(orc, q, X, Y, Z, how, mode):
+    """A read, another boundary and no step, a read: wall cells report the new
+    density and velocities, and new solids are solid."""
+    print(f"\n[case] read after {how} q={q} {X}x{Y}x{Z} mode={mode}", flush=True)
+    ob, pb = _bc()
+    types = [PERIODIC] * 4 + [NOSLIP] * 2
+    vel = {P.UP: (-0.03, 0.0, 0.0), P.DOWN: (0.01, 0.0, 0.0)}
+    ob2, pb2 = Boundary(type=types, vel=vel, rho_s=0.97), P.boundary(types, vel, 0.97)
+    mask2 = (np.random.default_rng(2).random((Z, Y, X)) < 0.2).astype(np.uint8) if how == "set_boundary" else None
+    tau, F, init = 0.64, (2e-5, 0.0, 1e-6), (P.INIT_PERTURBED, 6, 2e-3)
+    o = orc.cor_state("f64", q, X, Y, Z)
+    orc.cor_init(o, 1.0, (0.01, 0.0, 0.0), init)
+    orc.cor_run(o, tau, F, ob, 5)
+    with P.State(q, X, Y, Z, "f64", mode) as st:
+        st.set_boundary(pb)
+        st.initialize(1.0, (0.01, 0.0, 0.0), init, pb)
+        st.configure(tau, F, pb)
+        st.step(5)
+        for a, e in zip(st.moments(), orc.cor_moments(o, ob)):
+            assert np.array_equal(a, e)
+        if how == "set_boundary":
+            st.set_boundary(pb2, mask2)
+        elif how == "configure":
+            st.configure(tau, F, pb2)
+        else:
+            st.reset(pb2)
+        for a, e in zip(st.moments(), orc.cor_moments(o, ob2, mask2)):
+            assert np.array_equal(a, e)
