@@ -13,6 +13,7 @@
 #include <atomic>
 #include <cstring>
 #include <exception>
+#include <mutex>
 #include <string>
 #include <thread>
 
@@ -24,6 +25,8 @@ namespace plb {
 // The pinned pieces of one state or batch: allocated by its first read (for
 // that read and for the velocities of as many cells, and again for a larger
 // one: at most 12 MB), freed with it.  Two pieces per thread: one being written, one being read.
+// One read at a time holds them; reads of one state or batch from several
+// threads wait for each other.
 struct HostRing {
     static constexpr int kThreads = 3;
     static constexpr int kSlots = 2 * kThreads;
@@ -31,6 +34,7 @@ struct HostRing {
     char* buf = nullptr;
     size_t slot_bytes = 0;
     hipEvent_t ev[kSlots] = {};
+    std::mutex held;
 };
 
 inline void host_ring_free(HostRing* r) {
@@ -73,6 +77,7 @@ int host_read(HostRing* r, int device, hipStream_t stream, uint64_t items, size_
     const uint64_t most = HostRing::kSlotBytes / item_bytes, least = std::max<uint64_t>(1, std::min<uint64_t>(most, (128u << 10) / item_bytes));
     const uint64_t piece = std::max(least, std::min(most, (items + 7) / 8));
     const uint64_t pieces = (items + piece - 1) / piece;
+    std::lock_guard<std::mutex> hold(r->held);
     // not once for a density and again for the velocities (24 bytes a cell)
     // that are read after it: setting pinned memory up again costs 2 ms
     const size_t velocities = (size_t)std::min<uint64_t>((items + 7) / 8, HostRing::kSlotBytes / 24) * 24;

@@ -102,3 +102,30 @@ def test_read_after_the_boundary_changed(orc, q, X, Y, Z, how, mode):
             st.reset(pb2)
         for a, e in zip(st.moments(), orc.cor_moments(o, ob2, mask2)):
             assert np.array_equal(a, e)
+
+
+def test_reads_from_several_threads():
+    """One batch's domains, and one state's fields, read by several threads at
+    once: each gets what a read by itself gets."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    doms = [{"x": 40 + d, "y": 30, "z": 50 - d, "tau": 0.6 + 0.01 * d, "force": (1e-5, 0.0, 0.0)} for d in range(12)]
+    b = P.Batch(19, "f32s", doms, P.channel())
+    b.initialize(1.0, (0.01, 0.0, 0.0), (P.INIT_PERTURBED, 3, 2e-3))
+    b.step(6)
+    alone = [b.moments(d) for d in range(len(doms))]
+    with ThreadPoolExecutor(6) as pool:
+        for _ in range(3):
+            for (rho, u), (erho, eu) in zip(pool.map(b.moments, range(len(doms))), alone):
+                assert np.array_equal(rho, erho) and np.array_equal(u, eu)
+    b.close()
+    pb = _bc()[1]
+    for mode, fields in ((P.FUSED, (P.FIELD_RHO, P.FIELD_U)), (P.LITERAL, (P.FIELD_RHO, P.FIELD_U, P.FIELD_N))):
+        with P.State(19, 60, 50, 40, "f64", mode) as st:
+            st.initialize(1.0, (0.01, 0.0, 0.0), (P.INIT_PERTURBED, 3, 2e-3), pb)
+            st.configure(0.7, (1e-5, 0.0, 0.0), pb)
+            st.step(4)
+            alone = [st.download(f) for f in fields]
+            with ThreadPoolExecutor(6) as pool:
+                for f, got in zip(fields * 4, pool.map(st.download, fields * 4)):
+                    assert np.array_equal(got, alone[fields.index(f)])
