@@ -4,6 +4,8 @@
 //   f[k * pstride + c],  c = (z*Y + y)*X + x,  x fastest.
 #pragma once
 
+#include <algorithm>
+
 #include "bgk.hpp"
 #include "fastdiv.hpp"
 #include "state.hpp"
@@ -557,19 +559,18 @@ struct TwoShape {
     int bx, by;
 };
 inline TwoShape two_shape(int q, int sbytes, int X, int Y) {
-    const int cap = two_cap(q, sbytes);
+    const int64_t cap = two_cap(q, sbytes), x = X, y = Y;  // edges go up to 2^31 - 1
     TwoShape best{0, 0};
     double cost = 0;
-    const int widest = X < cap / 3 - 2 ? X : cap / 3 - 2;  // at least one row fits
-    for (int w = widest < 8 ? widest : 8; w <= widest; ++w) {
-        const int nx = (X + w - 1) / w, bx = (X + nx - 1) / nx;
-        int by = cap / (bx + 2) - 2;
-        by = by < Y ? by : Y;
-        const int ny = (Y + by - 1) / by;
-        by = (Y + ny - 1) / ny;
+    const int64_t widest = std::min(x, cap / 3 - 2);  // at least one row fits
+    for (int64_t w = std::min<int64_t>(widest, 8); w <= widest; ++w) {
+        const int64_t nx = (x + w - 1) / w, bx = (x + nx - 1) / nx;
+        int64_t by = std::min(cap / (bx + 2) - 2, y);
+        const int64_t ny = (y + by - 1) / by;
+        by = (y + ny - 1) / ny;
         const double lines = ((bx + 2.0) * sbytes / 128 + 1) / (bx * sbytes / 128.0);
-        const double c = (double)((bx + 2) * (by + 2)) * nx * ny * (1 + 0.25 * lines);
-        if (!best.bx || c < cost) best = TwoShape{bx, by}, cost = c;
+        const double c = (double)((bx + 2) * (by + 2)) * (double)nx * (double)ny * (1 + 0.25 * lines);
+        if (!best.bx || c < cost) best = TwoShape{(int)bx, (int)by}, cost = c;
     }
     return best;
 }
