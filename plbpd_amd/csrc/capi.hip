@@ -691,6 +691,10 @@ int plb_step(plb_state* s, int nsteps) {
     if (!s->configured) return fail(PLB_ERR_LOGIC, "plb_step before plb_configure");
     if (nsteps < 0) return fail(PLB_ERR_INVALID_ARGUMENT, "negative step count");
     const double* F = s->force;
+    // (plb_set_boundary takes a literal state's boundary as it is: a no-slip face
+    // without a velocity ends the first step there, with everything before it done)
+    bool whole = true;
+    for (int f = 0; f < 6; ++f) whole = whole && !(s->bc.type[f] == kNoslip && !s->bc.has_vel[f]);
     for (int i = 0; i < nsteps; ++i) {
         if (s->mode == PLB_MODE_LITERAL) {
             // PLBPD::march_in_time loop body (PLBPD.cpp:24-29).  With the
@@ -711,8 +715,8 @@ int plb_step(plb_state* s, int nsteps) {
                 if ((rc = timed(s, PLB_STAGE_COLLIDE, [&] { return lit_collide(s, s->tau, F); }))) return rc;
                 if ((rc = timed(s, PLB_STAGE_STREAM, [&] { return lit_push(s); }))) return rc;
             }
-            if ((rc = timed(s, PLB_STAGE_NOSLIP, [&] { return lit_noslip(s, bc, !fold || i + 1 == nsteps); })))
-                return rc;
+            const bool ntmp_read = !fold || i + 1 == nsteps || !whole;
+            if ((rc = timed(s, PLB_STAGE_NOSLIP, [&] { return lit_noslip(s, bc, ntmp_read); }))) return rc;
             if (fold && i + 1 < nsteps) continue;
             if ((rc = timed(s, PLB_STAGE_PERIODIC, [&] { return lit_periodic(s, bc); }))) return rc;
             if (fold) {

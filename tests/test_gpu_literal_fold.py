@@ -142,3 +142,33 @@ def test_noslip_passes_save_what_they_overwrite(orc, q, X, Y, Z, passes):
                 orc.lit_collide(o, tau, F), st.collide(tau, F)
                 st.synchronize()
             _same(st, o, end)
+
+
+@pytest.mark.parametrize("q,X,Y,Z", [(9, 20, 1, 6), (19, 6, 5, 4)])
+def test_step_that_ends_at_a_face_without_velocity(orc, q, X, Y, Z):
+    """A boundary set after plb_configure with a no-slip face that has no
+    velocity: the first step ends there, and every field is as the separate
+    calls leave it (the faces before it done, ntmp included)."""
+    print(f"\n[case] literal step ends early q={q} {X}x{Y}x{Z}", flush=True)
+    types = [NOSLIP, NOSLIP, UNSET, UNSET, NOSLIP, NOSLIP]
+    vel = {0: (0.01, 0.0, 0.02), 1: (0.0, 0.0, -0.01), 4: (0.05, 0.01, 0.0), 5: (0.0, -0.02, 0.0)}
+    ob, pb = _bc(types, vel)
+    first = [NOSLIP, NOSLIP, UNSET, UNSET, UNSET, UNSET]  # what is done before the face up
+    oe, _ = _bc(first, {f: vel[f] for f in (0, 1)})
+    _, bad = _bc(types, {f: vel[f] for f in (0, 1, 5)})
+    tau, F = 0.7, (1e-4, -2e-5, 3e-5)
+    o = orc.lit_state(q, X, Y, Z)
+    orc.lit_init(o, 1.0, (0.01, 0.0, 0.0), (P.INIT_PERTURBED, 31, 1e-2), ob)
+    orc.lit_run(o, tau, F, ob, 2)
+    orc.lit_collide(o, tau, F)
+    orc.lit_push(o)
+    orc.lit_noslip(o, oe)
+    for n in (1, 3):
+        with P.State(q, X, Y, Z, "f64", P.LITERAL) as st:
+            st.initialize(1.0, (0.01, 0.0, 0.0), (P.INIT_PERTURBED, 31, 1e-2), pb)
+            st.configure(tau, F, pb)
+            st.step(2)
+            st.set_boundary(bad)
+            with pytest.raises(P.OutOfRange):
+                st.step(n)
+            _same(st, o, n)
