@@ -104,7 +104,9 @@ typedef struct {
     int32_t variant;  /* PLB_F64 ... PLB_F16S */
     int32_t mode;     /* PLB_MODE_LITERAL or PLB_MODE_FUSED */
     int32_t device;   /* HIP device ordinal */
-    int32_t pop_pad;  /* fused layout: extra elements between population arrays; <0 = default */
+    int32_t pop_pad;  /* fused layout: extra elements between population arrays; literal */
+                      /* layout: 0 = as little memory as it takes (slower pushes);       */
+                      /* <0 = default                                                    */
 } plb_state_desc;
 
 /* Boundary(lbmodel, domain, solid_density, BoundaryType, BoundaryVelocity)

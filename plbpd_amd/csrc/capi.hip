@@ -368,7 +368,7 @@ int plb_state_create(const plb_state_desc* d, plb_state** out) {
         if (e == hipSuccess) e = hipMemset(s->u, 0, 3 * mom_bytes);
         return e;
     };
-    if (d->mode == PLB_MODE_LITERAL) lit_layout(s, false);
+    if (d->mode == PLB_MODE_LITERAL) lit_layout(s, d->pop_pad == 0);
     e = allocate();
     if (e == hipErrorOutOfMemory && d->mode == PLB_MODE_LITERAL) {
         // once more in the packed layout

@@ -684,23 +684,31 @@ int lit_ntmp_restore(plb_state* s) {
 }  // namespace
 
 // ------------------------------------------------------------ launchers ----
-// Device layout of a state (LitDims).  Rows of whole lines take up to an
-// eighth more memory for the pitch (where it would be more, only buffers below
-// 1 GiB get it), and two planes for the shift.  packed: the smallest form.
+// Device layout of a state (LitDims): rows of whole lines and the shift's two
+// planes, up to any size below 1 GiB per buffer and up to an eighth more memory
+// above; there rows of X + 2 cells and the two planes, or the packed form, if the
+// form before takes more.  packed: the smallest form.
 void lit_layout(plb_state* s, bool packed) {
     const uint64_t line = 128 / s->sbytes, X2 = (uint64_t)s->X + 2, ny = (uint64_t)s->Y + 2, nz = (uint64_t)s->Z + 2;
-    uint64_t nx = (X2 + line - 1) / line * line;
-    if (nx * 8 > X2 * 9 && nx * ny * nz * s->q * s->sbytes > (1ull << 30)) nx = X2;
-    if (packed) {
-        s->lit_nx = (int)X2;
-        s->lit_base = 0;
-        s->pstride = X2 * ny * nz;
+    const uint64_t least = X2 * ny * nz;
+    auto stride = [&](uint64_t nx, uint64_t* base) {
+        const uint64_t far = nx * ny + nx + 1;  // of a direction's shift
+        *base = (far + line - 1) / line * line + line - 1;
+        return (*base + nx * ny * nz + far + line - 1) / line * line;
+    };
+    auto fits = [&](uint64_t ps) { return ps * s->q * s->sbytes <= (1ull << 30) || ps * 8 <= least * 9; };
+    for (uint64_t nx : {(X2 + line - 1) / line * line, X2}) {
+        uint64_t base;
+        const uint64_t ps = stride(nx, &base);
+        if (packed || !fits(ps)) continue;
+        s->lit_nx = (int)nx;
+        s->lit_base = base;
+        s->pstride = ps;
         return;
     }
-    const uint64_t far = nx * ny + nx + 1;  // of a direction's shift
-    s->lit_nx = (int)nx;
-    s->lit_base = (far + line - 1) / line * line + line - 1;
-    s->pstride = (s->lit_base + nx * ny * nz + far + line - 1) / line * line;
+    s->lit_nx = (int)X2;
+    s->lit_base = 0;
+    s->pstride = least;
 }
 uint64_t lit_cells(const plb_state* s) { return (uint64_t)s->lit_nx * (s->Y + 2) * (s->Z + 2); }
 
