@@ -632,9 +632,8 @@ int batch_launch_two(plb_batch* b) {
         } else {
             FusedBC<T> bc;
             make_fused_bc<T>(b->bc, b->q, &bc);
-            if (!launch_batch2<Q, V>((const S*)b->buf[b->cur], (S*)b->buf[b->cur ^ 1], (const BDom<T>*)b->doms,
-                                     b->two_tiles, b->ntwo, bc, b->stream))
-                return fail(PLB_ERR_LOGIC, "no two-step kernel for this storage");
+            launch_batch2<Q, V>((const S*)b->buf[b->cur], (S*)b->buf[b->cur ^ 1], (const BDom<T>*)b->doms,
+                                b->two_tiles, b->ntwo, bc, b->stream);
             PLB_HIP_TRY(hipGetLastError());
             return PLB_OK;
         }

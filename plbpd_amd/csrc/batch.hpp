@@ -22,10 +22,9 @@ struct BTile {
     uint32_t dom, x0, y0, z0, zc, bx, by, pad;
 };
 
-// Two pull steps of every domain, A -> B (batch_two.hpp); false where no
-// kernel exists for (Q, V).
+// Two pull steps of every domain, A -> B (batch_two.hpp).
 template <int Q, int V>
-bool launch_batch2(const typename Prec<V>::S* A, typename Prec<V>::S* B, const BDom<typename Prec<V>::T>* doms,
+void launch_batch2(const typename Prec<V>::S* A, typename Prec<V>::S* B, const BDom<typename Prec<V>::T>* doms,
                    const BTile* tiles, uint32_t ntiles, const FusedBC<typename Prec<V>::T>& bc, hipStream_t stream);
 
 }  // namespace plb

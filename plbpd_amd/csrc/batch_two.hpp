@@ -29,7 +29,7 @@ struct BatchWalls {
 };
 
 template <int Q, int V, bool MOV>
-__global__ __launch_bounds__(two_threads(Q, (int)sizeof(typename Prec<V>::S)), 1) void k_batch2(
+__global__ __launch_bounds__(two_cap(Q, (int)sizeof(typename Prec<V>::S)), 1) void k_batch2(
     const typename Prec<V>::S* __restrict__ A, typename Prec<V>::S* __restrict__ B,
     const BDom<typename Prec<V>::T>* __restrict__ doms, const BTile* __restrict__ tiles,
     BatchWalls<typename Prec<V>::T> w) {
@@ -44,22 +44,21 @@ __global__ __launch_bounds__(two_threads(Q, (int)sizeof(typename Prec<V>::S)), 1
 }  // namespace
 
 template <int Q, int V>
-bool launch_batch2(const typename Prec<V>::S* A, typename Prec<V>::S* B, const BDom<typename Prec<V>::T>* doms,
+void launch_batch2(const typename Prec<V>::S* A, typename Prec<V>::S* B, const BDom<typename Prec<V>::T>* doms,
                    const BTile* tiles, uint32_t ntiles, const FusedBC<typename Prec<V>::T>& bc, hipStream_t stream) {
     using T = typename Prec<V>::T;
     BatchWalls<T> w;
     w.bc = bc;
     fill_wall_cub<Q, T>(bc, w.wcub);
-    const dim3 grid(ntiles), block(two_threads(Q, (int)sizeof(typename Prec<V>::S)));
+    const dim3 grid(ntiles), block(two_cap(Q, (int)sizeof(typename Prec<V>::S)));
     if (two_walls(bc, false, (int)sizeof(typename Prec<V>::S)))
         hipLaunchKernelGGL((k_batch2<Q, V, true>), grid, block, 0, stream, A, B, doms, tiles, w);
     else
         hipLaunchKernelGGL((k_batch2<Q, V, false>), grid, block, 0, stream, A, B, doms, tiles, w);
-    return true;
 }
 
 #define PLB_BATCH2_INST(Q, V)                                                                                  \
-    template bool launch_batch2<Q, V>(const typename Prec<V>::S*, typename Prec<V>::S*,                        \
+    template void launch_batch2<Q, V>(const typename Prec<V>::S*, typename Prec<V>::S*,                        \
                                       const BDom<typename Prec<V>::T>*, const BTile*, uint32_t,                \
                                       const FusedBC<typename Prec<V>::T>&, hipStream_t);
 #define PLB_BATCH2_INST_Q(Q)                                                                       \

@@ -1084,11 +1084,12 @@ bool fused_two_eligible(const plb_state* s) {
     }
     // automatic: 4- and 8-byte storage, where two steps per pass measured
     // faster on MI355X, one step per launch / two, us per step: D3Q19 256^3
-    // FP32-shifted 450 / 317 (10% solids) and 440 / 268 (walls only), FP64 915 /
-    // 594 and 922 / 515, D3Q27 256^3 walls only 641 / 442 (FP32-shifted) and
-    // 1,356 / 800 (FP64);
-    // 2-byte storage ran 1.23x slower with solids (its one-step kernel is
-    // closer to the arithmetic limit)
+    // FP32-shifted 464 / 317 (10% solids) and 446 / 267 (walls only), FP64 959 /
+    // 604 and 925 / 569, D3Q27 256^3 walls only 639 / 456 (FP32-shifted) and
+    // 1,336 / 857 (FP64).  2-byte storage, whose one-step kernel is closer to the
+    // arithmetic limit, ran slower on large lattices: D3Q19 256^3 248 / 286 (10%
+    // solids) and 220 / 235, 384^3 905 / 976 and 769 / 796, D3Q27 256^3 361 / 414 and
+    // 317 / 332 (128^3 37 / 35 and 35 / 32)
     if (s->tune_two < 0 && s->sbytes == 2) return false;
     // automatic: lattices of at least 2^18 cells (2^19 for D3Q27).  Below
     // that the launch has too few tiles and chunks of a few planes, and one

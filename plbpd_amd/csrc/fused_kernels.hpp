@@ -464,7 +464,8 @@ struct ZRing {
 };
 // Whether the two-step kernel holds (ZRing): for 8-byte storage, whose tiles
 // the LDS limits (D3Q19 32 x 11 -> 32 x 13 cells, D3Q27 32 x 7 -> 32 x 13), and
-// D3Q27 in 4-byte storage.  Per step, three planes kept / held: D3Q19 FP64 256^3
+// D3Q27 in 4-byte storage.  Per step, three planes kept / held, in one run (on
+// other cards the held forms took up to 10% longer): D3Q19 FP64 256^3
 // 636 / 594 us with solids, 553 / 515 walls only, 250 x 191 x 133 270 / 199;
 // D3Q27 FP64 256^3 1,007 / 800, 384^3 3,457 / 2,828; D3Q27 FP32-shifted 256^3
 // 467 / 442 (solids 579 / 518), 384^3 1,560 / 1,486.  D3Q19 in 4-byte storage,
@@ -475,8 +476,7 @@ __host__ __device__ constexpr bool two_hold(int q, int sbytes) { return sbytes =
 __host__ __device__ constexpr int two_lds(int q, int sbytes) {
     const bool h = two_hold(q, sbytes);
     const int planes = q == 19 ? (h ? ZRing<19, true>::planes() : ZRing<19, false>::planes())
-                               : (q == 27 ? (h ? ZRing<27, true>::planes() : ZRing<27, false>::planes())
-                                          : ZRing<9, false>::planes());
+                               : (h ? ZRing<27, true>::planes() : ZRing<27, false>::planes());
     return planes * sbytes + (h ? 4 : 8);
 }
 
@@ -485,44 +485,31 @@ __host__ __device__ constexpr int two_cells(int bx, int by) { return (bx + 2) * 
 // Whether the two-step kernel issues the step t gathers of the c_z = +1
 // directions an iteration earlier than the others (fused_two.hpp): D3Q19
 // with 4-byte storage, and with 8-byte storage around interior solids (nb).
-// The values held for the extra iteration fit there without spills (136
-// VGPRs with 4-byte storage, 256 with 8-byte); D3Q27 (9 such directions) and
-// 2-byte storage (13-row tiles at 128 VGPRs) spilled, and 8-byte storage
-// without interior solids measured 1% slower.
+// The values held for the extra iteration fit there without spills (123-139
+// VGPRs with 4-byte storage, 210 with 8-byte); D3Q27 (9 such directions)
+// and 2-byte storage (tiles of 1024 threads at 128 VGPRs) spilled, and 8-byte storage
+// without interior solids measured 1% slower (before its values were held).
 __host__ __device__ constexpr bool two_split(int q, int sbytes, bool nb) {
     return q == 19 && (sbytes == 4 || (sbytes == 8 && nb));
 }
 
-// Cells that a grown tile of any shape may have: the ring of that many cells
-// (two_lds(): its population planes and one or two 4-byte mask planes) fits the LDS
-// of a compute unit (160 KiB on gfx950; a workgroup takes all of it), within
-// 1024 threads, one per cell.  The split kernel with 4-byte storage takes at
-// most 704 cells: 64 x 9 tiles (768 threads) ran slower than 64 x 8, and so did
-// 64 x 11 (858 threads in 128 VGPRs: D3Q19 256^3 FP32-shifted 356 / 307 us
-// per step with solids / walls only, when 64 x 8 took 341 / 288).  8-byte storage
-// takes 512 (256 VGPRs a thread; with 768 threads it spilled: D3Q19 256^3 995
-// against 594 us per step with solids), D3Q27 in 4-byte storage 640 (768: 501
-// against 457 at 256^3 walls only).
+// Cells that a grown tile of any shape may have, and threads of a workgroup, one
+// per cell: whole wavefronts, and a ring (two_lds() bytes a cell) of 95 to 150 KB of a
+// compute unit's 160 KiB of LDS, so that a compute unit holds one workgroup.  With
+// 4-byte storage the registers set it: D3Q19 64 x 9 tiles (768 threads) ran slower than
+// 64 x 8 in 704, and so did 64 x 11 (858 threads in 128 VGPRs: 256^3 FP32-shifted
+// 356 / 307 us per step with solids / walls only, when 64 x 8 took 341 / 288); D3Q27
+// with 768 threads 501 us against 457 with 640 (256^3 walls only).  8-byte storage
+// takes 512 (256 VGPRs a thread; with 768 it spilled: D3Q19 256^3 995 against 594
+// us per step with solids), 2-byte storage as many threads as a workgroup may have.
 __host__ __device__ constexpr int two_cap(int q, int sbytes) {
-    const int lds = 160 * 1024 / two_lds(q, sbytes);
-    const int maxc = sbytes == 8 ? 512 : sbytes == 4 ? (q == 27 ? 640 : 704) : 1024;
-    if (lds >= maxc) return maxc;
-    // one slot more than cells where the last wavefront is cut short (two_slots)
-    return sbytes == 8 ? lds / 64 * 64 : lds - 1;
-}
-// Threads of a workgroup, and slots per plane of its ring: one per thread, so
-// that threads without a cell have a slot to write to as well, or as many as
-// fit the LDS, of which such threads share the last.
-__host__ __device__ constexpr int two_threads(int q, int sbytes) { return (two_cap(q, sbytes) + 63) / 64 * 64; }
-__host__ __device__ constexpr int two_slots(int q, int sbytes) {
-    const int lds = 160 * 1024 / two_lds(q, sbytes), t = two_threads(q, sbytes);
-    return t < lds ? t : lds;
+    return sbytes == 8 ? 512 : (sbytes == 4 ? (q == 27 ? 640 : 704) : 1024);
 }
 // Rows per tile for a lattice, a storage width and a tile width: the largest
 // BY whose grown tile, (bx + 2) x (BY + 2) cells, is within two_cap(); 0 where
 // no BY >= 3 is.
 __host__ __device__ constexpr int two_rows(int q, int sbytes, int bx) {
-    if (q == 27 && sbytes == 8 && bx > 32) return 0;  // 64 x 5 tiles: more grown cells than 32 x 13
+    if (q == 27 && sbytes == 8 && bx > 32) return 0;  // no kernel: 64 x 5 tiles have more grown cells than 32 x 13
     int best = 0;
     for (int by = 1; by <= 40; ++by)
         if (two_cells(bx, by) <= two_cap(q, sbytes)) best = by;
@@ -541,12 +528,11 @@ bool two_walls(const FusedBC<T>& bc, bool nb, int sbytes) {
     return bc.moving != 0 || (!nb && sbytes > 2 && bc.wall_lo[0]);
 }
 
-// The tile width a lattice and storage width prefer: 32 for 8-byte storage,
-// whose taller tile recomputes fewer grown-border cells (D3Q19 32 x 11
-// against 64 x 5: 6-13% faster from 128^3 to 384^3; D3Q27 fits 32-cell tiles
-// only), 64 otherwise (D3Q19 4-byte 32 x 18 against 64 x 8: 19-22% slower;
-// D3Q27 4-byte 32 x 16 against 64 x 7: 7-10% faster at 256^3 but 2.5%
-// slower at 384^3).
+// The tile width a storage width prefers: 32 for 8-byte storage, whose 32 x 13
+// tiles recompute fewer grown cells than 64 x 5 (D3Q19 128^3 and 256^3 9-15%
+// faster, 384^3 1%), 64 otherwise (D3Q19 4-byte 64 x 8 against 32 x 18 13-20%
+// faster from 128^3 to 384^3; D3Q27 4-byte 64 x 7 against 32 x 16 11% slower at
+// 128^3, 4-7% at 256^3, 2% faster to 4% slower at 384^3).
 __host__ __device__ constexpr int two_tile_pref(int q, int sbytes) { return (void)q, sbytes == 8 ? 32 : 64; }
 
 // The tile shape for rows of X cells and Y rows: nx x ny equal tiles (the last

@@ -213,9 +213,9 @@ __device__ inline void lds_barrier() {
 
 // The sweep of one workgroup over the planes [z0, z0 + zc) of the tile of
 // bx x by cells at (x0, y0), of any shape with at most two_cap() grown cells.
-// (With 64 x 8 and 32 x 11 tiles compiled in, D3Q19 256^3 ran 269 / 591 us per
-// step walls only, FP32-shifted / FP64, against 263 / 595 with the shape as an
-// argument.)  a: FusedArgs, or the like for one domain of a batch.  MOV
+// (With 64 x 8 and 32 x 11 tiles compiled in, before values were held, D3Q19
+// 256^3 ran 269 / 591 us per step walls only, FP32-shifted / FP64, against 263 /
+// 595 with the shape as an argument.)  a: FusedArgs, or the like for one domain of a batch.  MOV
 // (two_walls()): the form for moving walls and for walls on x.
 template <int Q, int V, int NB, bool MOV, int W, bool SPLIT, class Args>
 __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict__ A,
@@ -226,8 +226,8 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
     using S = typename P::S;
     using T = typename P::T;
     using I = uint32_t;
-    constexpr int NI = two_slots(Q, (int)sizeof(S)), NT = two_threads(Q, (int)sizeof(S));
-    static_assert(NI == NT || two_cap(Q, (int)sizeof(S)) < NI, "a slot for the threads without a cell");
+    constexpr int NI = two_cap(Q, (int)sizeof(S));  // threads, and cells per ring plane
+    static_assert(NI % 64 == 0 && NI * two_lds(Q, (int)sizeof(S)) <= 160 * 1024, "whole wavefronts, a ring that fits");
     const uint32_t RX = bx + 2u;  // grown row
     constexpr bool HOLD = two_hold(Q, (int)sizeof(S));
     __shared__ S ring[ZRing<Q, HOLD>::planes() * NI];
@@ -239,7 +239,6 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
     const uint32_t nplanes = std::min(zc, Z - z0) + 2u;
 
     // step t + 1: this thread's cell of the grown tile (wrapped coordinates)
-    const uint32_t slot = NI == NT ? tid : std::min(tid, (uint32_t)NI - 1u);  // in the ring
     const uint32_t ix = tid % RX, iy = tid / RX;
     const uint32_t gx = (x0 + ix + X - 1u) % X, gy = (y0 + iy + Y - 1u) % Y;
     // step t + 2: this thread's cell of the tile
@@ -307,8 +306,8 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
     // kernel is bound by neither alone (D3Q19 256^3 FP32-shifted around
     // solids: vector unit 65% busy, memory unit 67%), so what counts is
     // that both work at the same time: 341 -> 317 us per step with solids,
-    // 287 -> 268 walls only; FP64 647 -> 630 / 601 -> 589; D3Q27 384^3
-    // FP32-shifted 1,634 -> 1,560, FP64 3,638 -> 3,455.  (Stores in every
+    // 287 -> 268 walls only; before values were held FP64 647 -> 630 / 601 -> 589,
+    // D3Q27 384^3 FP32-shifted 1,634 -> 1,560, FP64 3,638 -> 3,455.  (Stores in every
     // wavefront and plane, dropped where there is nothing to store, so that
     // no wait for a load counts a path without them: no faster on large
     // lattices, 2-10% slower on small ones.)
@@ -377,9 +376,9 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
     };
     // The second half of an iteration: plane n is in the ring.  HOLD with
     // 4-byte storage collides after the barrier, next to the loads and the
-    // collision of the next plane (D3Q27 FP32-shifted 256^3 457 us per step
-    // against 477, 384^3 1,527 / 1,542; FP64, which waits on its stores there,
-    // 602 / 571 at D3Q19 256^3, 3,085 / 3,017 at D3Q27 384^3).
+    // collision of the next plane (after / before the barrier: D3Q27
+    // FP32-shifted 256^3 457 / 477 us per step, 384^3 1,527 / 1,542; FP64, which waits
+    // on its stores there, D3Q19 256^3 602 / 571, D3Q27 384^3 3,085 / 3,017).
     auto second = [&](uint32_t n) __attribute__((always_inline)) {
         lds_barrier();
         if constexpr (!HOLD) {
@@ -400,7 +399,7 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
         for (int k = 0; k < Q; ++k) f[k] = P::load_raw(fv[k]);
         const T rho = bgk<Q, P>(f, a, true);
         walls(f, rho, gx, gy, (z0 + n + Z - 1u) % Z);
-        ring_store<Q, 0, V, NI, HOLD>(f, ring, slot, HOLD ? n & 1u : n % 3u, HOLD ? 0u : n & 1u);
+        ring_store<Q, 0, V, NI, HOLD>(f, ring, tid, HOLD ? n & 1u : n % 3u, HOLD ? 0u : n & 1u);
     };
 
     if constexpr (!SPLIT) {
@@ -417,7 +416,7 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
             // last plane stay in bounds; their values are not used)
             mnext = load_mask(n + 1u);
             // the step t + 2 cells read this mask
-            if (FLAGS) mring[(HOLD ? 0u : n & 1u) * NI + slot] = mcur;
+            if (FLAGS) mring[(HOLD ? 0u : n & 1u) * NI + tid] = mcur;
             // (a wavefront of solid cells has nothing to compute)
             if (!__all(NB ? (mcur & 1u) != 0 : mcur != 0)) step1(n, fv);
             fetch(All{}, n + 1u, fv, mnext);
@@ -444,7 +443,7 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
         auto plane = [&](auto odd, uint32_t n, uint32_t& mc, uint32_t& mn) __attribute__((always_inline)) {
             S (&fc)[Q] = decltype(odd)::value ? fv1 : fv0;
             S (&fn)[Q] = decltype(odd)::value ? fv0 : fv1;
-            if (FLAGS) mring[(HOLD ? 0u : n & 1u) * NI + slot] = mc;
+            if (FLAGS) mring[(HOLD ? 0u : n & 1u) * NI + tid] = mc;
             mc = load_mask(n + 2u);
             fetch(Flat{}, n + 1u, fn, mn);
             step1(n, fc);
@@ -462,7 +461,7 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
 }
 
 template <int Q, int V, int NB, bool MOV, int W>
-__global__ __launch_bounds__(two_threads(Q, (int)sizeof(typename Prec<V>::S)), 1) void k_pull2(
+__global__ __launch_bounds__(two_cap(Q, (int)sizeof(typename Prec<V>::S)), 1) void k_pull2(
     const typename Prec<V>::S* __restrict__ A, typename Prec<V>::S* __restrict__ B,
     const uint8_t* __restrict__ flags, const uint32_t* __restrict__ nbmask, FusedArgs<typename Prec<V>::T> a,
     TwoGeom g) {
@@ -494,7 +493,7 @@ bool launch_pull2(const FusedArgs<typename Prec<V>::T>& a, const TwoGeom& g, boo
     constexpr int sb = (int)sizeof(typename Prec<V>::S);
     // the tile must fit the ring and the workgroup
     if (g.bx < 1 || g.by < 1 || (uint64_t)(g.bx + 2) * (g.by + 2) > (uint64_t)two_cap(Q, sb)) return false;
-    const dim3 grid(two_blocks(g)), block(two_threads(Q, sb));
+    const dim3 grid(two_blocks(g)), block(two_cap(Q, sb));
     auto go = [&](auto nbc, auto mvc, auto wc) {
         hipLaunchKernelGGL((k_pull2<Q, V, decltype(nbc)::value, decltype(mvc)::value, decltype(wc)::value>), grid,
                            block, 0, stream, A, B, flags, nbmask, a, g);

@@ -527,9 +527,9 @@ __device__ inline bool near_noslip(unsigned faces, const LitDims& g, int x, int 
 // no-slip pass only those of its face cells.  All of the outer layer's values
 // in place (38 one-lane stores per row of a lattice periodic in x, each into
 // lines of its own) and stores along c_k cost 191 us per step at 128^3 FP64;
-// the stores that remain, 157; whole lines (LitDims), 136 (FP32 77 -> 72,
-// 256^3 FP64 1,260 -> 1,107, D3Q27 64^3 27.6 -> 24.3): 4.7 TB/s of the 38 values
-// per cell at 128^3, 4.6 at 256^3, bound by memory.
+// the stores that remain, 157; whole lines (LitDims), 132, where the packed
+// form took 160 (256^3 FP64 990 and 1,209, D2Q9 4000 x 4000 465 and 523): 4.8 TB/s
+// of the 38 values per cell at 128^3, 5.2 at 256^3, bound by memory.
 template <int Q, class R>
 __global__ void k_moments_collide_push(LitDims g, R* __restrict__ n, R* __restrict__ rho, R* __restrict__ u,
                                        R* __restrict__ t, Periodic per, FaceResets<R> fr, MomentStores ms,
