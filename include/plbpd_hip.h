@@ -269,7 +269,8 @@ int plb_bench_pattern(int device, int q, int x, int y, int z, int sbytes, int ve
                       double* gbps, double* ms);
 /* Fused-kernel tuning knobs (no reference counterpart).  The defaults are
  * the settings measured fastest on MI355X for D3Q19 256^3; no knob changes
- * results; a change drops a captured step graph. */
+ * results; a change drops a captured step graph.  The knobs of the cell and row
+ * kernels act on launches of one step (plb_steps_per_launch). */
 #define PLB_TUNE_BLOCK_X 0  /* cells per block row: 64, 128, 256 (0 = from x)   */
 #define PLB_TUNE_NT_LOAD 1  /* non-temporal population loads of the push kernel */
                             /* (0/1; default 0).  The cell pull kernel's loads   */

@@ -111,3 +111,35 @@ def test_multi_step_rule():
     for variant, steps in (("f64", 8), ("f64a32", 8), ("f32s", 4), ("f16s", 1)):
         with P.State(9, 1024, 1, 1024, variant, P.FUSED) as st:
             assert st.steps_per_launch() == steps, variant
+
+
+@pytest.mark.parametrize("X,vec", [(100, 0), (256, 0), (64, 1), (128, 2), (256, 4), (384, 1), (512, 2)])
+@pytest.mark.parametrize("walls,solids", [((2,), False), ((0, 2), True), ((), False)])
+@pytest.mark.parametrize("variant", ["f64", "f32", "f64a32", "f32s", "f16s"])
+def test_single_steps_match_oracle(orc, X, vec, walls, solids, variant):
+    """One step per launch (staged calls, single steps, large lattices): the cell
+    pull kernel and the row pull kernel at each width, which runs of several
+    steps no longer reach on lattices of this size."""
+    print(f"\n[case] D2Q9 single steps {variant} X={X} vec={vec} walls={walls} solids={solids}", flush=True)
+    Z = 21
+    ob, pb = _bc(walls)
+    mask = (np.random.default_rng(3).random((Z, 1, X)) < 0.15).astype(np.uint8) if solids else None
+    tau, F, init = 0.63, (2e-5, 0.0, 1e-6), (P.INIT_PERTURBED, 5, 2e-3)
+    fluid = orc.cor_flags(9, X, 1, Z, ob, mask) == 0
+    bits = (lambda a: a.view(np.uint16)) if variant == "f16s" else (lambda a: a)
+    o = orc.cor_state(variant, 9, X, 1, Z)
+    orc.cor_init(o, 1.0, (0.01, 0.0, 0.0), init)
+    orc.cor_run(o, tau, F, ob, 9, mask)
+    with P.State(9, X, 1, Z, variant, P.FUSED) as a, P.State(9, X, 1, Z, variant, P.FUSED) as b:
+        for st in (a, b):
+            st.set_tuning(capi.TUNE_VECTOR, vec)
+            st.set_boundary(pb, mask)
+            st.initialize(1.0, (0.01, 0.0, 0.0), init, pb)
+            st.configure(tau, F, pb)
+        a.set_tuning(capi.TUNE_TWO_STEP, 0)
+        assert a.steps_per_launch() == 1 and b.steps_per_launch() == 8
+        a.step(9)
+        for _ in range(9):
+            b.step(1)
+        for st in (a, b):
+            assert np.array_equal(bits(st.download_raw())[fluid], bits(o["f"])[fluid])
