@@ -335,7 +335,7 @@ __device__ __forceinline__ void pull2_tile(const typename Prec<V>::S* __restrict
         // every row, a cell that is not fluid stores zeros, so that lines are
         // written whole (but a wavefront of such cells nothing); the wall
         // rows of the other axes store nothing.
-        const bool whole = NB || (MOV && a.bc.wall_lo[0]);
+        const bool whole = NB || (MOV && sizeof(S) > 2 && a.bc.wall_lo[0]);
         const bool store = in_o && (whole || !zero);
         store_own<Q, V, W>(f, rb, B, store ? (zo * XY + py * X + px) * sz : kNoStore, psz, whole && zero);
     };
