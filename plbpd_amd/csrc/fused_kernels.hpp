@@ -549,8 +549,11 @@ inline TwoShape two_shape(int q, int sbytes, int X, int Y) {
     TwoShape best{0, 0};
     double cost = 0;
     const int64_t widest = std::min(x, cap / 3 - 2);  // at least one row fits
+    int64_t last = 0;
     for (int64_t w = std::min<int64_t>(widest, 8); w <= widest; ++w) {
         const int64_t nx = (x + w - 1) / w, bx = (x + nx - 1) / nx;
+        if (nx == last) continue;  // the same tiles
+        last = nx;
         int64_t by = std::min(cap / (bx + 2) - 2, y);
         const int64_t ny = (y + by - 1) / by;
         by = (y + ny - 1) / ny;

@@ -24,7 +24,8 @@ namespace plb {
 
 // The pinned pieces of one state or batch: allocated by its first read (for
 // that read and for the velocities of as many cells, and again for a larger
-// one: at most 12 MB), freed with it.  Two pieces per thread: one being written, one being read.
+// one: at most 12 MB), freed with it.  Two pieces per thread that such a read
+// takes: one being written, one being read.
 // One read at a time holds them; reads of one state or batch from several
 // threads wait for each other.
 struct HostRing {
@@ -33,6 +34,7 @@ struct HostRing {
     static constexpr size_t kSlotBytes = (size_t)2 << 20;  // largest piece
     char* buf = nullptr;
     size_t slot_bytes = 0;
+    int slots = 0;
     hipEvent_t ev[kSlots] = {};
     std::mutex held;
 };
@@ -46,21 +48,26 @@ inline void host_ring_free(HostRing* r) {
     r->buf = nullptr;
 }
 
-inline int host_ring_ensure(HostRing* r, size_t slot_bytes) {
-    for (hipEvent_t& e : r->ev) {
-        if (e) continue;
-        PLB_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
-    if (r->buf && r->slot_bytes >= slot_bytes) return PLB_OK;
+inline int host_ring_ensure(HostRing* r, size_t slot_bytes, int slots) {
+    for (int i = 0; i < slots; ++i)
+        if (!r->ev[i]) PLB_HIP_TRY(hipEventCreateWithFlags(&r->ev[i], hipEventDisableTiming));
+    if (r->buf && r->slot_bytes >= slot_bytes && r->slots >= slots) return PLB_OK;
     if (r->buf) PLB_HIP_TRY(hipHostFree(r->buf));
     r->buf = nullptr;
-    size_t size = (size_t)64 << 10;
+    size_t size = std::max(r->slot_bytes, (size_t)64 << 10);
     while (size < slot_bytes) size *= 2;
+    slots = std::max(slots, r->slots);
     void* p = nullptr;
-    PLB_HIP_TRY(hipHostMalloc(&p, HostRing::kSlots * size, hipHostMallocDefault));
+    PLB_HIP_TRY(hipHostMalloc(&p, slots * size, hipHostMallocDefault));
     r->buf = (char*)p;
     r->slot_bytes = size;
+    r->slots = slots;
     return PLB_OK;
+}
+
+// Threads of a read: they pay for themselves from about 4 MB on.
+inline int host_read_threads(uint64_t bytes) {
+    return (int)std::min<uint64_t>(HostRing::kThreads, 1 + bytes / (4u << 20));
 }
 
 // Reads `items` items of item_bytes each: fill(first, count, slot) launches on
@@ -72,16 +79,20 @@ template <class Fill, class Put>
 int host_read(HostRing* r, int device, hipStream_t stream, uint64_t items, size_t item_bytes, const Fill& fill,
               const Put& put) {
     if (items == 0) return PLB_OK;
-    // pieces of an eighth of what is read, so that writing and taking overlap
-    // in a small read too
-    const uint64_t most = HostRing::kSlotBytes / item_bytes, least = std::max<uint64_t>(1, std::min<uint64_t>(most, (128u << 10) / item_bytes));
-    const uint64_t piece = std::max(least, std::min(most, (items + 7) / 8));
+    // pieces of an eighth of what is read, so that writing and taking overlap in
+    // a small read too, but no less than 512 KB: each costs a launch and a wait
+    // (1.1 MB in pieces of 128, 256 and 512 KB: 88, 64 and 58 us; 2.2 MB 115, 118 and 102)
+    const uint64_t most = HostRing::kSlotBytes / item_bytes,
+                   least = std::max<uint64_t>(1, std::min<uint64_t>(most, (512u << 10) / item_bytes));
+    const uint64_t piece = std::min(items, std::max(least, std::min(most, (items + 7) / 8)));
     const uint64_t pieces = (items + piece - 1) / piece;
     std::lock_guard<std::mutex> hold(r->held);
     // not once for a density and again for the velocities (24 bytes a cell)
     // that are read after it: setting pinned memory up again costs 2 ms
-    const size_t velocities = (size_t)std::min<uint64_t>((items + 7) / 8, HostRing::kSlotBytes / 24) * 24;
-    const int rc = host_ring_ensure(r, std::max<size_t>(piece * item_bytes, velocities));
+    const uint64_t cells = std::min(items, std::max<uint64_t>((512u << 10) / 24,
+                                                             std::min<uint64_t>(HostRing::kSlotBytes / 24, (items + 7) / 8)));
+    const uint64_t larger = std::max<uint64_t>(items * item_bytes, items * 24);
+    const int rc = host_ring_ensure(r, std::max<size_t>(piece * item_bytes, cells * 24), 2 * host_read_threads(larger));
     if (rc) return rc;
     const size_t slot_bytes = r->slot_bytes;
     std::atomic<uint64_t> next{0};
@@ -109,9 +120,7 @@ int host_read(HostRing* r, int device, hipStream_t stream, uint64_t items, size_
         }
         if (e != hipSuccess) failed.store((int)e);
     };
-    // threads pay for themselves from about 4 MB on
-    const uint64_t bytes = items * item_bytes;
-    const int threads = (int)std::min<uint64_t>(HostRing::kThreads, 1 + bytes / (4u << 20));
+    const int threads = host_read_threads(items * item_bytes);
     std::thread others[HostRing::kThreads];
     for (int w = 1; w < threads; ++w) {
         try {
